@@ -408,15 +408,15 @@ int moty_hip_matmul_i4_grouped_s_dev(float* y, const float* x, const uint8_t* q4
     if (rc) return rc;
     return launch_gemm_i4g(xq, sx, q4, scale, y, S, I, O, st);
   }
-  const bool per_token = S <= 4 || xf_gemv_per_token(S, I, O);
-  if (gs == 32 && per_token) {
-    // a few tokens: the one-token GEMV per token
+  if (gs == 32 && xf_gemv_per_token(S, I, O, false)) {
+    // a few tokens: the one-token GEMV per token (it refuses what it cannot
+    // take before launching anything)
     int rc = MOTY_OK;
     for (int s = 0; s < S && rc == MOTY_OK; s++)
       rc = launch_gemv_i4g_xf(x + (int64_t)s * I, q4, scale, nullptr, nullptr, y + (int64_t)s * O, I, O, st);
     if (rc != MOTY_EUNSUP) return rc;
   }
-  if (gs == 32 && S > 4) {
+  if (gs == 32 && S > 1) {
     const int rc = launch_gemm_i4g_xf(x, q4, scale, nullptr, nullptr, y, S, I, O, st);
     if (rc != MOTY_EUNSUP) return rc;
   }
@@ -632,18 +632,6 @@ int moty_hip_dense_ffn_i4g_dev(float* out, const float* x, int S, const uint8_t*
     if ((rc = launch_gemv_i4g(x, gate, gs, up, us, h, 1, D, I, st))) return rc;
     return launch_gemv_i4g(h, down, ds, nullptr, nullptr, out, 1, I, D, st);
   }
-  const bool xf_tok = S <= 4 || (xf_gemv_per_token(S, D, 2 * I) && xf_gemv_per_token(S, I, D));
-  if (!idot4 && xf_tok && D <= 16384 && I <= 16384 &&
-      !(((uintptr_t)x | (uintptr_t)gate | (uintptr_t)up | (uintptr_t)down | (uintptr_t)h) & 15)) {
-    // exact f32, per token: gate + up + SiLU in one pass, then down (the
-    // shapes fit, so no launch is refused after the first)
-    for (int s = 0; s < S; s++) {
-      if ((rc = launch_gemv_i4g_xf(x + (int64_t)s * D, gate, gs, up, us, h + (int64_t)s * I, D, I, st))) return rc;
-      if ((rc = launch_gemv_i4g_xf(h + (int64_t)s * I, down, ds, nullptr, nullptr, out + (int64_t)s * D, I, D, st)))
-        return rc;
-    }
-    return MOTY_OK;
-  }
   // one matmul_i4_grouped_s each, the path chosen per matrix as the
   // reference does (IDOT4 needs the row length a multiple of 64, <= 16384)
   auto mm = [&](const float* a, const uint8_t* w, const float* ws, float* o, int K, int N) -> int {
@@ -652,9 +640,7 @@ int moty_hip_dense_ffn_i4g_dev(float* out, const float* x, int S, const uint8_t*
       int r = launch_qrow_i8(a, (int8_t*)xq, sx, nullptr, S, K, K, K, st);
       return r ? r : launch_gemm_i4g((const int8_t*)xq, sx, w, ws, o, S, K, N, st);
     }
-    const bool tok = S <= 4 || xf_gemv_per_token(S, K, N);
-    if (!tok && launch_gemm_i4g_xf(a, w, ws, nullptr, nullptr, o, S, K, N, st) == MOTY_OK) return MOTY_OK;
-    if (tok) {
+    if (xf_gemv_per_token(S, K, N, false)) {
       // exact f32, a few tokens: the one-token GEMV per token (it refuses
       // what it cannot take before launching anything)
       int r = MOTY_OK;
@@ -662,13 +648,24 @@ int moty_hip_dense_ffn_i4g_dev(float* out, const float* x, int S, const uint8_t*
         r = launch_gemv_i4g_xf(a + (int64_t)s * K, w, ws, nullptr, nullptr, o + (int64_t)s * N, K, N, st);
       if (r != MOTY_EUNSUP) return r;
     }
+    if (S > 1) {
+      const int r = launch_gemm_i4g_xf(a, w, ws, nullptr, nullptr, o, S, K, N, st);
+      if (r != MOTY_EUNSUP) return r;
+    }
     return launch_i4g_f32(a, w, ws, o, S, K, N, st);
   };
-  if (!idot4 && !xf_tok && S > 4 && (D % 64) == 0 && !(((uintptr_t)x) & 15) &&
-      !(((uintptr_t)gate | (uintptr_t)up) & 7)) {
-    // exact f32, many tokens: gate + up + SiLU in one tiled pass, then down
-    if ((rc = launch_gemm_i4g_xf(x, gate, gs, up, us, h, S, D, I, st))) return rc;
-    return mm(h, down, ds, out, I, D);
+  if (!idot4) {
+    // exact f32: gate + up + SiLU in one pass, per token or tiled, where the
+    // kernels take the shape and its alignment; then down
+    rc = MOTY_EUNSUP;
+    if (xf_gemv_per_token(S, D, I, true)) {
+      rc = MOTY_OK;
+      for (int s = 0; s < S && rc == MOTY_OK; s++)
+        rc = launch_gemv_i4g_xf(x + (int64_t)s * D, gate, gs, up, us, h + (int64_t)s * I, D, I, st);
+    }
+    if (rc == MOTY_EUNSUP && S > 1) rc = launch_gemm_i4g_xf(x, gate, gs, up, us, h, S, D, I, st);
+    if (rc == MOTY_OK) return mm(h, down, ds, out, I, D);
+    if (rc != MOTY_EUNSUP) return rc;
   }
   if ((rc = mm(x, gate, gs, h, D, I))) return rc;
   if ((rc = mm(x, up, us, u, D, I))) return rc;

@@ -1117,150 +1117,300 @@ int launch_gemm_i4g(const int8_t* xq, const float* sx, const uint8_t* q4, const 
 }
 
 // ---------------------------------------------------------------------------
-// The exact-f32 path (IDOT4 unset) for many tokens, as a tiled GEMM on the
-// vector ALUs (the reference's float order admits no matrix-core form: each
-// product x*w is rounded on its own).  Workgroup tile: 64 tokens x 64 weight
-// rows (PAIR: 32 gate rows and the same 32 up rows), K steps of two groups.
-// Per step the workgroup stages x and the nibbles, expanded once to floats
-// (n - 8, exact), in LDS; thread (tx, ty) owns tokens ty + 16i and tile rows
-// tx + 16j (i, j < 4).  Each group's 32 elements sit in LDS in the order
-// 8*(e % 4) + e / 4, so for jj = 0..3 the eight elements
-// {jj, jj+4, jj+8, jj+12, jj+16, .., jj+28} that reduce to v[jj] of the
-// reference's tree are two 16-byte reads:
-//   t[j] = fma(x[j], w[j], x[16+j]*w[16+j])   (j < 16)
+// The exact-f32 path (IDOT4 unset) for several tokens, on f32 matrix
+// instructions.  v_mfma_f32_16x16x1_4b_f32 is four independent 16 x 16 outer
+// products with one fused multiply-add per output (k = 1), bit for bit
+// v_fma_f32 of the same operands (checked on random triples, wide exponents,
+// denormals and signed zeros), so block b of one instruction carries one j of
+// the reference's group step (nn/matmul.c:222-233 with FMA contraction):
+//   p    = fma(x[16+j], w[16+j], -0)          the rounded product, its sign of zero kept
+//   t[j] = fma(x[j], w[j], p)                 (j < 16)
 //   u[j] = t[j+8] + t[j];  v[j] = u[j+4] + u[j];  r = (v0 + v2) + (v1 + v3)
-//   a = fma(r, scale[g], a)                  (groups in ascending order)
-// -- nn/matmul.c:222-233 with FMA contraction, as the one-token kernels.
-constexpr int XF_BT = 64, XF_BO = 64, XF_KE = 64;  // tokens, weight rows, elements per K step
-constexpr int XF_LS = XF_KE + 4;                   // LDS row stride (floats): 16-byte reads conflict-free
+//   a    = fma(r, scale[g], a)                (groups in ascending order)
+// Instruction q takes j = q, q+4, q+8, q+12 in its four blocks, whose results
+// for one output land in one lane, so the tree is 15 adds per output and group
+// in registers, and a lane's operands are two float4s of its x row (elements
+// 4b.. and 16 + 4b.., b = lane / 16) and the four nibble bytes of the same
+// elements of its weight row.
+//
+// Wave (wm, wn, ks) owns TM x TN tiles of 16 tokens x 16 weight rows (PAIR:
+// TN = 2, the same 16 gate and up rows) and, of every K step's KG groups,
+// those with index ks mod KS.  With KS = 4 the waves of a tile hand the group
+// sums r over through LDS and wave ks continues the chains of the tile's
+// register ks: the r of different groups are independent, only the chain, one
+// FMA per group, is serial.  Steps are double-buffered in LDS, one barrier
+// per step.
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4_a8 __attribute__((ext_vector_type(4), aligned(8)));
 
-__device__ __forceinline__ int xf_pos(int e) { return ((e >> 5) << 5) + 8 * (e & 3) + ((e & 31) >> 2); }
+// signed byte K of w as a float
+template <int K>
+__device__ __forceinline__ float cvt_sb(uint32_t w) { return (float)(int)(int8_t)(w >> (8 * K)); }
 
-template <bool PAIR>
-__global__ __launch_bounds__(256, 2) void k_gemm_i4g_xf(const float* __restrict__ x, const uint8_t* __restrict__ q4,
-                                                        const float* __restrict__ scl,
-                                                        const uint8_t* __restrict__ q4b,
-                                                        const float* __restrict__ sclb, float* __restrict__ y,
-                                                        int M, int I, int O) {
-  __shared__ __align__(16) float xs[XF_BT * XF_LS];
-  __shared__ __align__(16) float ws[XF_BO * XF_LS];
-  __shared__ float ss[XF_BO][2];
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const int tb = blockIdx.y * XF_BT;
-  constexpr int OR = PAIR ? XF_BO / 2 : XF_BO;  // output rows per tile
-  const int ob = blockIdx.x * OR;
+template <int TM, int TN, int WM, int WN, int KS, int KG, bool PAIR>
+__global__ __launch_bounds__(64 * WM * WN * KS) void k_gemm_i4g_xf(const float* __restrict__ x,
+                                                                   const uint8_t* __restrict__ q4,
+                                                                   const float* __restrict__ scl,
+                                                                   const uint8_t* __restrict__ q4b,
+                                                                   const float* __restrict__ sclb,
+                                                                   float* __restrict__ y, int M, int I, int O) {
+  static_assert(!PAIR || TN == 2, "PAIR: one gate and one up tile per wave");
+  static_assert(KG % KS == 0 && (KS == 1 || KS == 4 || KS == 8), "groups of a step over the K waves");
+  constexpr int NT = 64 * WM * WN * KS;
+  constexpr int BM = 16 * TM * WM, BW = 16 * TN * WN;  // tokens, weight rows of the tile
+  constexpr int OC = PAIR ? BW / 2 : BW;               // output columns
+  constexpr int XS = KG * 128;      // LDS row stride of x: 16-byte chunks, XOR-swizzled by row
+  constexpr int WS = KG * 16 + 16;  // of the nibbles: padded, the 2-byte reads of 16 rows hit 16 banks
+  constexpr int XC = BM * KG * 8, WC = BW * KG;  // a step's 16-byte pieces of x and of the nibbles
+  constexpr int NX = (XC + NT - 1) / NT, NW = (WC + NT - 1) / NT;
+  constexpr int NR = KS == 1 ? 4 : 1;  // chains per tile and lane
+  __shared__ __align__(16) uint8_t xs[2][BM * XS];
+  __shared__ __align__(16) uint8_t ws[2][BW * WS];
+  __shared__ __align__(16) float ss[2][BW * KG];
+  __shared__ float rs[2][KS > 1 ? WM * WN * KG * TM * TN * 256 : 1];  // group sums of a step
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int ks = wv % KS, wt = wv / KS, wm = wt / WN, wn = wt % WN;
+  const int r16 = lane & 15, b = lane >> 4;
+  const int tb = blockIdx.y * BM, ob = blockIdx.x * OC;
   const int ng = I / 32, rb = I / 2;
-  // staging roles: x row tid/4, elements 16*(tid%4) .. +16 of the step;
-  // weight row tid/4, nibble bytes 8*(tid%4) .. +8 (elements 16*(tid%4) ..)
-  const int sr = tid >> 2, sq = tid & 3;
-  const int xt = tb + sr < M ? tb + sr : M - 1;
-  const float* xsrc = x + (int64_t)xt * I + 16 * sq;
-  const uint8_t* wsrc;
-  const float* ssrc;
-  {
-    int row = PAIR ? (sr & 31) : sr;
-    int o = ob + row < O ? ob + row : O - 1;
-    const bool up = PAIR && sr >= 32;
-    wsrc = (up ? q4b : q4) + (int64_t)o * rb + 8 * sq;
-    ssrc = (up ? sclb : scl) + (int64_t)o * ng;
-  }
-  float4 px[4];
-  uint2 pw;
-  float psc = 0.f;
-  auto gload = [&](int k0) {
+
+  // staging: piece c of x is chunk c % (8 KG) of row c / (8 KG), of the
+  // nibbles group c % KG of row c / KG.  Rows past the end re-read the last
+  // one; pieces past a row's end re-read its first (never used).
+  float4 px[NX];
+  u32x4_a8 pw[NW];
+  float ps[NW];
+  auto gload = [&](int g0) {
 #pragma unroll
-    for (int q = 0; q < 4; q++) px[q] = *(const float4*)(xsrc + k0 + 4 * q);
-    pw = *(const uint2*)(wsrc + k0 / 2);
-    if (sq < 2) psc = ssrc[k0 / 32 + sq];
+    for (int i = 0; i < NX; i++) {
+      const int c = tid + i * NT, row = c / (8 * KG), k = c % (8 * KG);
+      if (XC % NT == 0 || c < XC) {
+        const int t = tb + row < M ? tb + row : M - 1;
+        const int e = g0 * 32 + k * 4;
+        px[i] = *(const float4*)(x + (int64_t)t * I + (e < I ? e : 0));
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NW; i++) {
+      const int c = tid + i * NT, row = c / KG, k = c % KG;
+      if (WC % NT == 0 || c < WC) {
+        const bool up = PAIR && row >= OC;
+        const int on = ob + (up ? row - OC : row);
+        const int64_t o = on < O ? on : O - 1;
+        const int g = g0 + k < ng ? g0 + k : 0;
+        pw[i] = *(const u32x4_a8*)((up ? q4b : q4) + o * rb + g * 16);
+        ps[i] = (up ? sclb : scl)[o * ng + g];
+      }
+    }
   };
-  float a[4][4];
+  auto put = [&](int p) {
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+    for (int i = 0; i < NX; i++) {
+      const int c = tid + i * NT, row = c / (8 * KG), k = c % (8 * KG);
+      if (XC % NT == 0 || c < XC) *(float4*)(xs[p] + row * XS + ((k ^ (row & 15)) << 4)) = px[i];
+    }
 #pragma unroll
-    for (int j = 0; j < 4; j++) a[i][j] = 0.f;
+    for (int i = 0; i < NW; i++) {
+      const int c = tid + i * NT, row = c / KG, k = c % KG;
+      if (WC % NT == 0 || c < WC) {
+        *(u32x4_a8*)(ws[p] + row * WS + k * 16) = pw[i];
+        ss[p][row * KG + k] = ps[i];
+      }
+    }
+  };
+
+  v16f neg0;
+#pragma unroll
+  for (int i = 0; i < 16; i++) neg0[i] = -0.f;
+  asm("" : "+v"(neg0));  // keeps it in registers: else rebuilt every step
+  float a[TM][TN][NR];
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+#pragma unroll
+      for (int r = 0; r < NR; r++) a[i][j][r] = 0.f;
+  float sc[TN][KG];  // this lane's weight rows' scales of the step
+  const int nstep = (ng + KG - 1) / KG;
+
+  // KS > 1: this wave's share of the chains over step st's group sums
+  auto chain = [&](int st) {
+    if (ks >= 4) return;
+    const int n = ng - st * KG < KG ? ng - st * KG : KG;
+    const float* rp = rs[st & 1] + wt * (KG * TM * TN * 256) + ks * 64 + lane;
+#pragma unroll
+    for (int k = 0; k < KG; k++)
+      if (k < n)
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+          for (int j = 0; j < TN; j++)
+            a[i][j][0] = __fmaf_rn(rp[((k * TM + i) * TN + j) * 256], sc[j][k], a[i][j][0]);
+  };
+
   gload(0);
-  for (int k0 = 0; k0 < I; k0 += XF_KE) {
-    __syncthreads();  // the previous step's reads are done
-    {
-      const float* pv = (const float*)px;
-#pragma unroll
-      for (int e = 0; e < 16; e++) xs[sr * XF_LS + xf_pos(16 * sq + e)] = pv[e];
-      const uint32_t wd[2] = {pw.x, pw.y};
-#pragma unroll
-      for (int b = 0; b < 8; b++) {
-        const uint32_t byte = (wd[b >> 2] >> (8 * (b & 3))) & 0xffu;
-        ws[sr * XF_LS + xf_pos(16 * sq + 2 * b)] = (float)(byte & 15u) - 8.f;
-        ws[sr * XF_LS + xf_pos(16 * sq + 2 * b + 1)] = (float)(byte >> 4) - 8.f;
-      }
-      if (sq < 2) ss[sr][sq] = psc;
-    }
+  put(0);
+  if (nstep > 1) gload(KG);
+  for (int st = 0; st < nstep; st++) {
+    // step st is staged, the group sums of step st - 1 are handed over, and
+    // every wave is done with the buffers of step st - 1
     __syncthreads();
-    if (k0 + XF_KE < I) gload(k0 + XF_KE);
+    if (KS > 1 && st > 0) chain(st - 1);
+    const int p = st & 1;
+    if (st + 1 < nstep) {
+      put(p ^ 1);
+      if (st + 2 < nstep) gload((st + 2) * KG);
+    }
 #pragma unroll
-    for (int g = 0; g < 2; g++) {
-      float w02[4][4], v[4][4];
+    for (int j = 0; j < TN; j++) {
+      const int row = PAIR ? j * OC + wn * 16 + r16 : (wn * TN + j) * 16 + r16;
 #pragma unroll
-      for (int h = 0; h < 4; h++) {
-        const int jj = h == 0 ? 0 : (h == 1 ? 2 : (h == 2 ? 1 : 3));  // v0, v2, then v1, v3
-        float X[4][8], W[4][8];
+      for (int k = 0; k < KG; k++) sc[j][k] = ss[p][row * KG + k];
+    }
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          *(float4*)&X[i][0] = *(const float4*)(xs + (ty + 16 * i) * XF_LS + 32 * g + 8 * jj);
-          *(float4*)&X[i][4] = *(const float4*)(xs + (ty + 16 * i) * XF_LS + 32 * g + 8 * jj + 4);
-        }
+    for (int gi = 0; gi < KG / KS; gi++) {
+      const int g = gi * KS + ks;
+      if (st * KG + g >= ng) break;  // wave-uniform
+      float4 xl[TM], xh[TM];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-          *(float4*)&W[j][0] = *(const float4*)(ws + (tx + 16 * j) * XF_LS + 32 * g + 8 * jj);
-          *(float4*)&W[j][4] = *(const float4*)(ws + (tx + 16 * j) * XF_LS + 32 * g + 8 * jj + 4);
-        }
+      for (int i = 0; i < TM; i++) {
+        const uint8_t* base = xs[p] + ((wm * TM + i) * 16 + r16) * XS;
+        xl[i] = *(const float4*)(base + (((g * 8 + b) ^ r16) << 4));
+        xh[i] = *(const float4*)(base + (((g * 8 + 4 + b) ^ r16) << 4));
+      }
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+      for (int j = 0; j < TN; j++) {
+        const int row = PAIR ? j * OC + wn * 16 + r16 : (wn * TN + j) * 16 + r16;
+        const uint8_t* base = ws[p] + row * WS + g * 16 + 2 * b;
+        const uint32_t n = (uint32_t)*(const uint16_t*)base | ((uint32_t)*(const uint16_t*)(base + 8) << 16);
+        // bytes: elements 4b, 4b+2, 16+4b, 16+4b+2 (even) and their odd neighbours, as n - 8
+        const uint32_t ev = nib_minus8(n & 0x0f0f0f0fu), od = nib_minus8((n >> 4) & 0x0f0f0f0fu);
+        const float wl[4] = {cvt_sb<0>(ev), cvt_sb<0>(od), cvt_sb<1>(ev), cvt_sb<1>(od)};
+        const float wh[4] = {cvt_sb<2>(ev), cvt_sb<2>(od), cvt_sb<3>(ev), cvt_sb<3>(od)};
 #pragma unroll
-          for (int j = 0; j < 4; j++) {
-            // t at j = jj, jj+4, jj+8, jj+12: slots 0..3, partners in slots 4..7
-            float t[4];
+        for (int i = 0; i < TM; i++) {
+          const float xlo[4] = {xl[i].x, xl[i].y, xl[i].z, xl[i].w}, xhi[4] = {xh[i].x, xh[i].y, xh[i].z, xh[i].w};
+          // the eight matrix instructions together, then the adds: left to
+          // itself the compiler chains each pair and waits for it (M = 250,
+          // I = 4096, O = 12288 gate/up 937 -> 860 us); memory and scalar
+          // instructions may cross
+          v16f t[4];
+          __builtin_amdgcn_sched_barrier(0x4 | 0x10 | 0x80);
 #pragma unroll
-            for (int k = 0; k < 4; k++) t[k] = __fmaf_rn(X[i][k], W[j][k], X[i][k + 4] * W[j][k + 4]);
-            const float vv = (t[3] + t[1]) + (t[2] + t[0]);  // u[jj+4] + u[jj]
-            if (h == 0 || h == 2) v[i][j] = vv;
-            else if (h == 1) w02[i][j] = v[i][j] + vv;  // v0 + v2
-            else a[i][j] = __fmaf_rn(w02[i][j] + (v[i][j] + vv), ss[tx + 16 * j][g], a[i][j]);
+          for (int q = 0; q < 4; q++) t[q] = __builtin_amdgcn_mfma_f32_16x16x1f32(xhi[q], wh[q], neg0, 0, 0, 0);
+#pragma unroll
+          for (int q = 0; q < 4; q++) t[q] = __builtin_amdgcn_mfma_f32_16x16x1f32(xlo[q], wl[q], t[q], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0x4 | 0x10 | 0x80);
+          float v[4][4];
+#pragma unroll
+          for (int q = 0; q < 4; q++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[q][r] = (t[q][12 + r] + t[q][4 + r]) + (t[q][8 + r] + t[q][r]);
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            const float s = (v[0][r] + v[2][r]) + (v[1][r] + v[3][r]);
+            if constexpr (KS == 1)
+              a[i][j][r] = __fmaf_rn(s, sc[j][g], a[i][j][r]);
+            else
+              rs[p][((wt * KG + g) * TM * TN + i * TN + j) * 256 + r * 64 + lane] = s;
           }
+        }
       }
     }
   }
+  if constexpr (KS > 1) {
+    __syncthreads();
+    chain(nstep - 1);
+  }
+  if (KS > 4 && ks >= 4) return;
+  // lane l, register r of a tile: token 4 (l / 16) + r, weight row l % 16
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int t = tb + ty + 16 * i;
-    if (t >= M) continue;
-    if (PAIR) {
+  for (int i = 0; i < TM; i++)
 #pragma unroll
-      for (int j = 0; j < 2; j++) {
-        const int o = ob + tx + 16 * j;
-        if (o < O) y[(int64_t)t * O + o] = ref_silu_mul(a[i][j], a[i][j + 2]);
-      }
-    } else {
+    for (int r = 0; r < NR; r++) {
+      const int t = tb + (wm * TM + i) * 16 + 4 * b + (KS == 1 ? r : ks);
+      if (t >= M) continue;
+      if constexpr (PAIR) {
+        const int o = ob + wn * 16 + r16;
+        if (o < O) y[(int64_t)t * O + o] = ref_silu_mul(a[i][0][r], a[i][1][r]);
+      } else {
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const int o = ob + tx + 16 * j;
-        if (o < O) y[(int64_t)t * O + o] = a[i][j];
+        for (int j = 0; j < TN; j++) {
+          const int o = ob + (wn * TN + j) * 16 + r16;
+          if (o < O) y[(int64_t)t * O + o] = a[i][j][r];
+        }
       }
     }
-  }
 }
 
-// many tokens, exact f32: I % 64 == 0, 16-byte aligned x and 8-byte aligned
-// nibbles; PAIR (q4b): y = silu(gate) * up
+// The tile shapes, by the time one workgroup takes alone on a CU per 4096
+// elements of I (measured on MI355X over M = 1..500 and six (I, O) pairs;
+// workgroups on one CU share its SIMDs, so a launch takes about
+// ceil(workgroups / 256) of these).  Small tiles with the K steps split over
+// waves fill the chip when there are few, large ones cost less per output:
+//   gate + up, tokens x columns: 16 x 32 47 us, 16 x 64 78, 64 x 64 250
+//   one matrix:  16 x 32 25 us, 16 x 64 43, 32 x 64 71, 64 x 64 128
+// (the 64 x 64 ones run at 0.7 of the rate of their matrix and vector
+// instructions alone: 446 clocks per 16 x 16 tile and group, since the two
+// kinds do not overlap on a SIMD here).
+struct XfTile {
+  int bm, oc;
+  double us;
+};
+static constexpr XfTile XF_PAIR[] = {{16, 32, 47}, {16, 64, 78}, {64, 64, 250}};
+static constexpr XfTile XF_ONE[] = {{16, 32, 25}, {16, 64, 43}, {32, 64, 71}, {64, 64, 128}};
+
+static int xf_pick(int M, int I, int O, bool pair, double* us) {
+  const XfTile* t = pair ? XF_PAIR : XF_ONE;
+  const int n = pair ? 3 : 4;
+  int best = 0;
+  double bt = 0;
+  for (int k = 0; k < n; k++) {
+    const int64_t wgs = (int64_t)((M + t[k].bm - 1) / t[k].bm) * ((O + t[k].oc - 1) / t[k].oc);
+    const double us_k = (double)((wgs + 255) / 256) * t[k].us * I / 4096;
+    if (k == 0 || us_k < bt) best = k, bt = us_k;
+  }
+  *us = bt;
+  return best;
+}
+
+// S tokens: the one-token GEMV once per token (about 4 us plus the matrix
+// bytes at 5 TB/s each: 5.0 us at 1024 x 3072 gate + up, 14.2 at 4096 x
+// 12288), or the GEMM above?  The GEMM wins from 3 tokens at the smaller
+// shapes and from 6 at the larger one (82 us for up to 16 tokens).
+bool xf_gemv_per_token(int S, int I, int O, bool pair) {
+  if (S <= 1) return true;
+  if (S > 64) return false;
+  double gemm_us;
+  xf_pick(S, I, O, pair, &gemm_us);
+  const double gemv_us = 4.0 + ((double)O * I * (pair ? 1.25 : 0.625)) / 5.0e6;
+  return S * gemv_us < gemm_us + 3.0;
+}
+
+// I % 32 == 0, 16-byte aligned x and 8-byte aligned nibbles; PAIR (q4b):
+// y = silu(gate) * up
 int launch_gemm_i4g_xf(const float* x, const uint8_t* q4, const float* scl, const uint8_t* q4b, const float* sclb,
                        float* y, int M, int I, int O, hipStream_t st) {
-  if ((I % XF_KE) || (((uintptr_t)x) & 15) || ((((uintptr_t)q4) | ((uintptr_t)q4b)) & 7)) return MOTY_EUNSUP;
+  if ((I % 32) || (((uintptr_t)x) & 15) || ((((uintptr_t)q4) | ((uintptr_t)q4b)) & 7)) return MOTY_EUNSUP;
   if (M <= 0 || O <= 0) return MOTY_OK;
-  const int orow = q4b ? XF_BO / 2 : XF_BO;
-  dim3 grid((O + orow - 1) / orow, (M + XF_BT - 1) / XF_BT);
-  if (q4b)
-    hipLaunchKernelGGL(k_gemm_i4g_xf<true>, grid, dim3(256), 0, st, x, q4, scl, q4b, sclb, y, M, I, O);
-  else
-    hipLaunchKernelGGL(k_gemm_i4g_xf<false>, grid, dim3(256), 0, st, x, q4, scl, q4b, sclb, y, M, I, O);
+  double us;
+  const int k = xf_pick(M, I, O, q4b != nullptr, &us);
+  const XfTile t = q4b ? XF_PAIR[k] : XF_ONE[k];
+  const dim3 grid((O + t.oc - 1) / t.oc, (M + t.bm - 1) / t.bm);
+#define XF(TM, TN, WM, WN, KS, KG, P)                                                                          \
+  hipLaunchKernelGGL((k_gemm_i4g_xf<TM, TN, WM, WN, KS, KG, P>), grid, dim3(64 * WM * WN * KS), 0, st, x, q4, \
+                     scl, q4b, sclb, y, M, I, O)
+  if (q4b) {
+    if (k == 0) XF(1, 2, 1, 2, 4, 4, true);
+    else if (k == 1) XF(1, 2, 1, 4, 4, 4, true);
+    else XF(1, 2, 4, 4, 1, 2, true);
+  } else {
+    if (k == 0) XF(1, 1, 1, 2, 8, 8, false);
+    else if (k == 1) XF(1, 1, 1, 4, 4, 4, false);
+    else if (k == 2) XF(2, 1, 1, 4, 4, 4, false);
+    else XF(1, 1, 4, 4, 1, 2, false);
+  }
+#undef XF
   LAUNCH_TRY("k_gemm_i4g_xf");
   return MOTY_OK;
 }

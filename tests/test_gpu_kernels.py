@@ -231,6 +231,44 @@ def test_i4g_f32(ops, S, I, O):
     assert same_bits(y, y2), mismatch(y, y2)
 
 
+@pytest.mark.parametrize("S,I,O", [
+    # every tile shape of the several-token GEMM (16 x 32, 16 x 64, 32 x 64,
+    # 64 x 64 by the grid's size), ragged in tokens and rows; 1, 3 and 9
+    # groups: less than a K step, one that is not full, several and a part
+    (6, 32, 30), (17, 288, 70), (40, 96, 2760), (64, 96, 4198), (150, 96, 4200), (129, 288, 4170)])
+def test_i4g_f32_gemm_tiles(ops, S, I, O):
+    say("i4g f32 gemm tiles", S, I, O)
+    q4, s = o_pack_int4_grouped(randn(O + I, (O, I), 0.02))
+    x = randn(S + 2 * I, (S, I))
+    # zeros of both signs, denormals, values past the f32 range when summed
+    x[0, :8] = [0.0, -0.0, 1e-40, -1e-40, 3e38, -3e38, 1e-30, 0.0]
+    x[1, :32] = -0.0
+    x[2, 5], x[3, 5], x[4, 5] = np.inf, -np.inf, np.nan
+    y = to_np(ops.matmul_i4_grouped_s(to_dev(x), to_dev(q4), to_dev(s), 32, False))
+    y2 = o_matmul_i4g(x, q4, s, False)
+    assert (np.isnan(y) == np.isnan(y2)).all()
+    fine = ~np.isnan(y2)
+    assert same_bits(y[fine], y2[fine]), mismatch(y[fine], y2[fine])
+
+
+@pytest.mark.parametrize("S,D,I", [(5, 96, 64), (33, 96, 2752), (190, 32, 4320), (3, 1056, 3008)])
+def test_dense_ffn_i4g_f32_tiles(ops, S, D, I):
+    """The gate + up form of the same tiles (16 x 32, 16 x 64, 64 x 64), and
+    a few tokens where gate/up and down may take different kernels."""
+    say("dense_ffn_i4g f32 tiles", S, D, I)
+    gq, gs = o_pack_int4_grouped(randn(S + D, (I, D), 0.02))
+    uq, us = o_pack_int4_grouped(randn(S + D + 1, (I, D), 0.02))
+    dq, ds = o_pack_int4_grouped(randn(S + I, (D, I), 0.02))
+    x = randn(S + 3, (S, D))
+    y = to_np(ops.dense_ffn_i4g(to_dev(x), to_dev(gq), to_dev(gs), to_dev(uq), to_dev(us), to_dev(dq), to_dev(ds),
+                                False))
+    g = o_matmul_i4g(x, gq, gs, False)
+    u = o_matmul_i4g(x, uq, us, False)
+    oracle().o_silu_mul(ptr(g), ptr(u), g.size)
+    y2 = o_matmul_i4g(g, dq, ds, False)
+    assert same_bits(y, y2), mismatch(y, y2)
+
+
 @pytest.mark.parametrize("S,I,O", [(8, 2048, 64), (3, 33, 5), (2, 16, 3), (1, 100, 7), (5, 2049, 128)])
 def test_matmul_f32(ops, S, I, O):
     say("matmul_f32", S, I, O)
