@@ -533,18 +533,25 @@ int moty_hip_dense_ffn_q8_dev(float* out, const float* x, int S, const int8_t* g
     if (rc) return rc;
     return launch_gemv_q8(h, down, ds, nullptr, nullptr, out, S, I, D, st);
   }
+  // gate and up in one pass with the SiLU epilogue where the tiled kernel
+  // takes the rows (D % 128 == 0), else one GEMM each and silu_mul
+  const bool pair = (D % 128) == 0;
   const size_t b_xq = al256((size_t)S * (D > I ? D : I)), b_sx = al256((size_t)S * 4);
   const size_t b_g = al256((size_t)S * I * 4);
-  int rc = scratch_get(d, b_xq + b_sx + 2 * b_g, st, &sp);
+  int rc = scratch_get(d, b_xq + b_sx + (pair ? 1 : 2) * b_g, st, &sp);
   if (rc) return rc;
   int8_t* xq = (int8_t*)sp;
   float* sx = (float*)((char*)sp + b_xq);
   float* g = (float*)((char*)sp + b_xq + b_sx);
-  float* u = (float*)((char*)sp + b_xq + b_sx + b_g);
   if ((rc = launch_qrow_i8(x, xq, sx, nullptr, S, D, D, D, st))) return rc;
-  if ((rc = launch_gemm_q8(xq, sx, gate, gs, g, S, D, I, st))) return rc;
-  if ((rc = launch_gemm_q8(xq, sx, up, us, u, S, D, I, st))) return rc;
-  if ((rc = launch_silu_mul(g, u, (int64_t)S * I, st))) return rc;
+  if (pair) {
+    if ((rc = launch_gemm_q8_pair(xq, sx, gate, gs, up, us, g, S, D, I, st))) return rc;
+  } else {
+    float* u = (float*)((char*)sp + b_xq + b_sx + b_g);
+    if ((rc = launch_gemm_q8(xq, sx, gate, gs, g, S, D, I, st))) return rc;
+    if ((rc = launch_gemm_q8(xq, sx, up, us, u, S, D, I, st))) return rc;
+    if ((rc = launch_silu_mul(g, u, (int64_t)S * I, st))) return rc;
+  }
   if ((rc = launch_qrow_i8(g, xq, sx, nullptr, S, I, I, I, st))) return rc;
   return launch_gemm_q8(xq, sx, down, ds, out, S, I, D, st);
 }

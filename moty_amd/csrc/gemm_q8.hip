@@ -153,42 +153,59 @@ __global__ __launch_bounds__(GM_NT, 2) void k_gemm_q8(const int8_t* __restrict__
 // 16-byte bank groups.  A DMA instruction fills 8 rows (1 KiB): lane l loads
 // row l/8's chunk (l%8) ^ ((row >> 1) & 7) into slot l%8.
 // WGM x WGN waves over the block tile (each wave TM x TN outputs).  KS = 2
-// runs two such groups of waves on alternate K blocks (the int32 partial
-// sums are added at the end: exact), doubling the loads and MFMAs in flight
-// per workgroup where the grid has few tiles.
-template <int BM, int BN, int S, int WGM = 2, int WGN = 2, int KS = 1>
+// or 4 runs that many groups of waves on alternate K blocks (the int32 partial
+// sums are added at the end: exact), multiplying the loads and MFMAs in flight
+// per workgroup where the grid has few tiles.  PAIR: the tile's weight rows
+// are BN / 2 gate rows and the same up rows, a wave's TN half and half, and
+// y = silu(gate) * up (the reference's gate_up + silu_rows, nn/ffn.c:28-37)
+// without the two [M][O] f32 matrices between.
+template <int BM, int BN, int S, int WGM = 2, int WGN = 2, int KS = 1, bool PAIR = false, int GM = 4>
 __global__ __launch_bounds__(64 * WGM * WGN * KS) void k_gemm_q8_dma(const int8_t* __restrict__ xq,
                                                                      const float* __restrict__ sx,
                                                                      const int8_t* __restrict__ W,
                                                                      const float* __restrict__ scale,
+                                                                     const int8_t* __restrict__ W2,
+                                                                     const float* __restrict__ scale2,
                                                                      float* __restrict__ y, int M, int K, int O) {
   constexpr int NW = WGM * WGN;              // waves per K group
   constexpr int STAGE = (BM + BN) * GM_KB;   // one K group's share of a stage
   constexpr int NI = (BM + BN) / (8 * NW);   // DMA instructions per wave per stage
   constexpr int TM = BM / WGM, TN = BN / WGN, FM = TM / 32, FN = TN / 32;
-  static_assert((BM + BN) % (8 * NW) == 0 && FM >= 1 && FN >= 1, "tile shape");
+  constexpr int OC = PAIR ? BN / 2 : BN, TC = PAIR ? TN / 2 : TN;  // output columns of the tile, of a wave
+  static_assert((BM + BN) % (8 * NW) == 0 && FM >= 1 && FN >= 1 && (!PAIR || FN % 2 == 0), "tile shape");
   static_assert(KS == 1 || KS * STAGE * S >= (KS - 1) * NW * 64 * FM * FN * 64, "room for the partial sums");
   __shared__ __align__(1024) int8_t lds[S * KS * STAGE];
   __shared__ float s_sx[BM];
+  __shared__ uint64_t s_exp[PAIR ? 32 : 1];
   const int tid = threadIdx.x, lane = tid % MOTY_WAVE, wv = tid / MOTY_WAVE;
   const int kg = wv / NW, w = wv % NW;
   const int wm = w / WGN, wn = w % WGN;
   const int r32 = lane & 31, h = lane >> 5;
   int bx = blockIdx.x, by = blockIdx.y;
   {
-    // workgroups go round-robin over the 8 XCDs by linear id: give XCD x a
-    // (gy/2) x (gx/4) block of tiles, so its L2 pulls in half the
-    // activation rows and a quarter of the weight rows (row-major order
-    // gave each XCD every activation row and an eighth of the weights)
-    const int gx = gridDim.x, gy = gridDim.y;
-    if (gx % 4 == 0 && gy % 2 == 0) {
-      const int lin = by * gx + bx, x = lin & 7, j = lin >> 3;
+    // workgroups go round-robin over the 8 XCDs by linear id.  GM > 0: each
+    // XCD takes a contiguous run of tiles, walked column by column in groups
+    // of GM tile rows, so the 32 tiles its CUs hold at a time share 4 blocks
+    // of activation rows and 8 of weight rows in its L2 (256 x 256 tiles, M =
+    // 2000, 24576 x 4096: 273 -> 265 us).  GM = 0, for grids of short K loops:
+    // XCD x takes a (gy/2) x (gx/4) block, half the activation rows and a
+    // quarter of the weight rows (64 x 128 tiles, M = 512, 10240 x 1024: 13.5
+    // us against 17.6 in runs, 15.0 in plain order)
+    const int gx = gridDim.x, gy = gridDim.y, lin = by * gx + bx, xcd = lin & 7, j = lin >> 3;
+    if constexpr (GM > 0) {
+      const int n = gx * gy, q = n / 8, r = n % 8;
+      const int id = xcd * q + (xcd < r ? xcd : r) + j;
+      const int m0 = id / (GM * gx) * GM, in = id % (GM * gx);
+      const int gs = gy - m0 < GM ? gy - m0 : GM;
+      by = m0 + in % gs;
+      bx = in / gs;
+    } else if (gx % 4 == 0 && gy % 2 == 0) {
       const int bw = gx / 4;
-      bx = (x & 3) * bw + j % bw;
-      by = (x >> 2) * (gy / 2) + j / bw;
+      bx = (xcd & 3) * bw + j % bw;
+      by = (xcd >> 2) * (gy / 2) + j / bw;
     }
   }
-  const int mb = by * BM, nb = bx * BN;
+  const int mb = by * BM, nb = bx * OC;
   const int8_t* src[NI];
 #pragma unroll
   for (int i = 0; i < NI; i++) {
@@ -198,8 +215,12 @@ __global__ __launch_bounds__(64 * WGM * WGN * KS) void k_gemm_q8_dma(const int8_
       const int m = mb + row < M ? mb + row : M - 1;  // rows past the end: loaded, never stored
       src[i] = xq + (int64_t)m * K + c * 16;
     } else {
-      const int n = nb + row - BM < O ? nb + row - BM : O - 1;
-      src[i] = W + (int64_t)n * K + c * 16;
+      // PAIR: a wave's TN weight rows are the TC gate rows of its columns,
+      // then the same up rows
+      const int r = row - BM, q = PAIR ? r % TN % TC : 0;
+      int n = nb + (PAIR ? r / TN * TC + q : r);
+      n = n < O ? n : O - 1;
+      src[i] = (PAIR && r % TN >= TC ? W2 : W) + (int64_t)n * K + c * 16;
     }
   }
   const int nk = K / GM_KB;
@@ -224,8 +245,9 @@ __global__ __launch_bounds__(64 * WGM * WGN * KS) void k_gemm_q8_dma(const int8_
   float scn[FN];
 #pragma unroll
   for (int j = 0; j < FN; j++) {
-    const int n = nb + wn * TN + j * 32 + r32;
-    scn[j] = scale[n < O ? n : O - 1];
+    const bool up = PAIR && j >= FN / 2;
+    const int n = nb + wn * TC + (up ? j - FN / 2 : j) * 32 + r32;
+    scn[j] = (up ? scale2 : scale)[n < O ? n : O - 1];
   }
 #pragma unroll
   for (int s = 0; s < S - 1; s++) issue(s);
@@ -287,21 +309,81 @@ __global__ __launch_bounds__(64 * WGM * WGN * KS) void k_gemm_q8_dma(const int8_
       }
     }
   }
-  if (tid < BM) s_sx[tid] = sxr;
+  if (PAIR) exp_tab_lds(s_exp);
+  for (int i = tid; i < BM; i += 64 * WGM * WGN * KS) s_sx[i] = i == tid ? sxr : sx[mb + i < M ? mb + i : M - 1];
   __syncthreads();
   if (kg) return;
 #pragma unroll
-  for (int j = 0; j < FN; j++) {
-    const int n = nb + wn * TN + j * 32 + r32;
+  for (int j = 0; j < (PAIR ? FN / 2 : FN); j++) {
+    const int n = nb + wn * TC + j * 32 + r32;
     if (n >= O) continue;
 #pragma unroll
     for (int i = 0; i < FM; i++)
 #pragma unroll
       for (int r = 0; r < 16; r++) {
         const int ml = wm * TM + i * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-        if (mb + ml < M) __builtin_nontemporal_store((scn[j] * s_sx[ml]) * (float)acc[i][j][r], y + (int64_t)(mb + ml) * O + n);
+        float v = (scn[j] * s_sx[ml]) * (float)acc[i][j][r];
+        if constexpr (PAIR) v = ref_silu_mul(v, (scn[j + FN / 2] * s_sx[ml]) * (float)acc[i][j + FN / 2][r], s_exp);
+        if (mb + ml < M) __builtin_nontemporal_store(v, y + (int64_t)(mb + ml) * O + n);
       }
   }
+}
+
+// Tile shapes of k_gemm_q8_dma: rows of y, columns of y, and the time of a
+// launch as max(l0 + l1 * nk, u * (e + f * nk)) us for nk K blocks of 128 and
+// u = ceil(tiles / 256) tiles on the busiest CU: the first term is a lone
+// tile's K loop, the second the CU's share of L2 -> LDS bytes and MFMAs.
+// Fitted on MI355X to M = 5..4000 over (I, O) = (1024, 10240), (3072, 1024),
+// (4096, 4096), (5632, 2048), (12288, 4096) and, gate + up, (1024, 3072),
+// (2048, 5632), (4096, 12288), weights rotating past the Infinity Cache.
+// Where each wins: few tokens are bound by the weight stream and take narrow
+// tiles with the K blocks split over wave groups (M = 24: 22 us for 2 x
+// 12288 x 4096, 17 us for 4096 x 12288; 64-row tiles took 38 and 22); many
+// tokens by the bytes every CU pulls from L2 (about 20 a clock), which fall
+// with the tile's width (M = 2000: 24576 x 4096 with SiLU 258 us in 256 x
+// 256 tiles against 484 + 82 for two GEMMs in 64 x 64 and silu_mul; 4096 x
+// 12288 120 us in 128 x 128 against 205).
+struct Q8Tile {
+  int bm, oc;
+  double l0, l1, e, f;
+};
+static constexpr Q8Tile Q8_ONE[] = {{32, 32, 2.5, 0.145, 2.5, 0.155}, {32, 64, 2.5, 0.19, 3.1, 0.20},
+                                    {64, 64, 2.0, 0.35, 0.5, 0.225},  {64, 128, 2.0, 0.66, 0.4, 0.40},
+                                    {128, 128, 2.5, 0.76, 1.6, 0.61}, {256, 256, 13.0, 1.5, 13.0, 2.05}};
+static constexpr Q8Tile Q8_PAIR[] = {{32, 32, 4.5, 0.20, 2.9, 0.25},
+                                     {64, 32, 5.0, 0.30, 4.8, 0.33},
+                                     {128, 64, 2.5, 1.0, 2.6, 0.64},
+                                     {256, 128, 16.0, 2.0, 16.0, 2.0}};
+
+template <int N>
+static int q8_pick(const Q8Tile (&t)[N], int M, int K, int O) {
+  int best = 0;
+  double bt = 0;
+  for (int k = 0; k < N; k++) {
+    const int64_t tiles = (int64_t)((M + t[k].bm - 1) / t[k].bm) * ((O + t[k].oc - 1) / t[k].oc);
+    const double nk = K / GM_KB, u = (double)((tiles + 255) / 256);
+    const double lone = t[k].l0 + t[k].l1 * nk, full = u * (t[k].e + t[k].f * nk), us = lone > full ? lone : full;
+    if (k == 0 || us < bt) best = k, bt = us;
+  }
+  return best;
+}
+
+int launch_gemm_q8_pair(const int8_t* xq, const float* sx, const int8_t* W, const float* scale, const int8_t* W2,
+                        const float* scale2, float* y, int M, int K, int O, hipStream_t st) {
+  if (K % GM_KB) return MOTY_EUNSUP;
+  if (M <= 0 || O <= 0) return MOTY_OK;
+  const int k = q8_pick(Q8_PAIR, M, K, O);
+  const dim3 grid((O + Q8_PAIR[k].oc - 1) / Q8_PAIR[k].oc, (M + Q8_PAIR[k].bm - 1) / Q8_PAIR[k].bm);
+#define QP(BM, BN, S, WM, WN, KS)                                                                             \
+  hipLaunchKernelGGL((k_gemm_q8_dma<BM, BN, S, WM, WN, KS, true>), grid, dim3(64 * WM * WN * KS), 0, st, xq,  \
+                     sx, W, scale, W2, scale2, y, M, K, O)
+  if (k == 0) QP(32, 64, 3, 1, 1, 2);
+  else if (k == 1) QP(64, 64, 3, 2, 1, 2);
+  else if (k == 2) QP(128, 128, 2, 4, 2, 1);
+  else QP(256, 256, 2, 2, 4, 1);
+#undef QP
+  LAUNCH_TRY("k_gemm_q8_dma pair");
+  return MOTY_OK;
 }
 
 int launch_gemm_q8(const int8_t* xq, const float* sx, const int8_t* W, const float* scale, float* y, int M,
@@ -309,34 +391,20 @@ int launch_gemm_q8(const int8_t* xq, const float* sx, const int8_t* W, const flo
   if (K % 16) return MOTY_EUNSUP;
   if (M <= 0 || O <= 0) return MOTY_OK;
   if (K % GM_KB == 0) {
-    // 64 x 64 tiles (several workgroups per CU hide the DMA latency); three
-    // stages for K <= 1024, four for longer rows.  Measured on MI355X, M =
-    // 512: N=10240, K=1024: 17.3 us vs 18.8 register-staged; K=2048, N=1024:
-    // 7.7 vs 9.6; K=3072: 10.0 vs 12.5.
-    // Tiles from a sweep on MI355X at M = 512 (the C2 projections): 64 x 64
-    // tiles of 4 waves while the grid holds at least 256 of them (N = 10240,
-    // K = 1024: 15.2 us); below that 64 x 32 tiles with two groups of 2 waves
-    // on alternate K blocks (N = 1024, K = 2048: 7.1 us vs 7.4; K = 3072: 8.7
-    // vs 9.3) -- these GEMMs are bound by each workgroup's K-loop latency,
-    // not by the grid's width.  Four groups of 2 waves (three stages) where
-    // K holds at least 4 blocks: 6.3 / 7.3 us against 6.9 / 8.5 with two,
-    // timed back to back on rotating weights (inside the C2 layer step, after
-    // the wide GEMM, both forms average 8.0 us).  Grids of at least 512
-    // tiles of 64 x 128 with K <= 1024 (C2's fused N = 10240): those tiles,
-    // 8 waves, two stages, 13.3 us against 15.0 (median 14.2 against 16.8)
-    // for 64 x 64 in three; 128 x 64 13.5, 128 x 128 13.8-14.1, three stages
-    // of 64 x 128 16.2.  Both GEMMs write y with nontemporal stores: the
-    // output (21 MB for C2's fused GEMM) then does not sit dirty in L2 to be
-    // evicted under the next kernels' reads (C2 step 42.7 -> 40.8 us).
-#define QD(BM, BN, S, WM, WN, KS)                                                                             \
-  hipLaunchKernelGGL((k_gemm_q8_dma<BM, BN, S, WM, WN, KS>), dim3((O + BN - 1) / BN, (M + BM - 1) / BM),       \
-                     dim3(64 * WM * WN * KS), 0, st, xq, sx, W, scale, y, M, K, O)
-    const bool narrow = (int64_t)((M + 63) / 64) * ((O + 63) / 64) < 256;
-    if (narrow && K >= 4 * GM_KB) QD(64, 32, 3, 2, 1, 4);
-    else if (narrow && K >= 2 * GM_KB) QD(64, 32, 4, 2, 1, 2);
-    else if (K <= 1024 && (int64_t)((M + 63) / 64) * ((O + 127) / 128) >= 512) QD(64, 128, 2, 2, 4, 1);
-    else if (K <= 1024) QD(64, 64, 3, 2, 2, 1);
-    else QD(64, 64, 4, 2, 2, 1);
+    // Every form writes y with nontemporal stores: the output then does not
+    // sit dirty in L2 to be evicted under the next kernels' reads (at M =
+    // 512 a layer's seven projections 42.7 -> 40.8 us).
+    const int k = q8_pick(Q8_ONE, M, K, O);
+    const dim3 grid((O + Q8_ONE[k].oc - 1) / Q8_ONE[k].oc, (M + Q8_ONE[k].bm - 1) / Q8_ONE[k].bm);
+#define QD(BM, BN, S, WM, WN, KS, GM)                                                                         \
+  hipLaunchKernelGGL((k_gemm_q8_dma<BM, BN, S, WM, WN, KS, false, GM>), grid, dim3(64 * WM * WN * KS), 0, st, \
+                     xq, sx, W, scale, nullptr, nullptr, y, M, K, O)
+    if (k == 0) QD(32, 32, 4, 1, 1, 4, 4);
+    else if (k == 1) QD(32, 64, 3, 1, 2, 4, 4);
+    else if (k == 2) QD(64, 64, 3, 2, 2, 1, 4);
+    else if (k == 3) QD(64, 128, 2, 2, 4, 1, 0);
+    else if (k == 4) QD(128, 128, 2, 4, 2, 1, 4);
+    else QD(256, 256, 2, 2, 4, 1, 4);
 #undef QD
     LAUNCH_TRY("k_gemm_q8_dma");
     return MOTY_OK;

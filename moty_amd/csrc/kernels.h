@@ -52,6 +52,11 @@ int launch_ffn1h_q8(const float* x, const int8_t* G, const float* gs, const int8
 int launch_gemm_q8(const int8_t* xq, const float* sx, const int8_t* W, const float* scale, float* y, int M, int K,
                    int O, hipStream_t st);
 
+// gate and up in one pass, y [M][O] = silu(x.W^T) * (x.W2^T): K % 128 == 0,
+// else MOTY_EUNSUP
+int launch_gemm_q8_pair(const int8_t* xq, const float* sx, const int8_t* W, const float* scale, const int8_t* W2,
+                        const float* scale2, float* y, int M, int K, int O, hipStream_t st);
+
 // q4b/sclb non-null: PAIR mode (S = 1), y = silu(x.q4^T) * (x.q4b^T)
 int launch_gemv_i4g(const float* x, const uint8_t* q4, const float* scl, const uint8_t* q4b, const float* sclb,
                     float* y, int S, int I, int O, hipStream_t st);

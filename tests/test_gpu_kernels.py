@@ -169,6 +169,44 @@ def test_matmul_q_s(ops, S, I, O):
     assert same_bits(y, y2), mismatch(y, y2)
 
 
+@pytest.mark.parametrize("S,I,O", [
+    # each tile shape of the int8 GEMM (32 x 32 and 32 x 64 with K split four
+    # ways, 64 x 64, 64 x 128, 128 x 128, 256 x 256), ragged in tokens and
+    # rows, with one K block, fewer than the wave groups, and many
+    (600, 4096, 100), (3, 128, 31), (100, 3072, 2081), (300, 256, 3001), (70, 128, 33), (250, 128, 20001),
+    (1001, 1024, 10239), (2001, 1024, 10241), (4095, 12288, 4095)])
+def test_gemm_q8_tiles(ops, S, I, O):
+    say("gemm_q8 tiles", S, I, O)
+    g = torch.Generator(device="cuda").manual_seed(S + I + O)
+    xq = torch.randint(-127, 128, (S, I), generator=g, device="cuda", dtype=torch.int8)
+    q = torch.randint(-128, 128, (O, I), generator=g, device="cuda", dtype=torch.int8)
+    sx, s = (torch.rand(n, generator=g, device="cuda") * 0.01 + 1e-3 for n in (S, O))
+    y = ops.matmul_q8_preq(xq, sx, q, s)
+    # every sum is below 2^31 and every product exact in float64
+    acc = xq.double() @ q.double().t().contiguous()
+    ref = (s[None, :] * sx[:, None]) * acc.float()
+    assert torch.equal(y, ref)
+
+
+@pytest.mark.parametrize("S,D,I", [
+    # each gate + up tile (32 x 32, 64 x 32, 128 x 64, 256 x 128 columns),
+    # ragged; D % 128 != 0 runs the two GEMMs and silu_mul
+    (5, 128, 48), (24, 1024, 3088), (70, 1024, 3072), (130, 256, 2000), (2001, 4096, 12304), (37, 1088, 3008)])
+def test_dense_ffn_q8_prefill_tiles(ops, S, D, I):
+    """The fused gate + up GEMM against one GEMM each and silu_mul."""
+    say("dense_ffn_q8 tiles", S, D, I)
+    g = torch.Generator(device="cuda").manual_seed(S + D + I)
+
+    def q8(O, K):
+        return (torch.randint(-128, 128, (O, K), generator=g, device="cuda", dtype=torch.int8),
+                torch.rand(O, generator=g, device="cuda") * 1e-4 + 1e-5)
+    (wg, sg), (wu, su), (wd, sd) = q8(I, D), q8(I, D), q8(D, I)
+    x = torch.randn((S, D), generator=g, device="cuda")
+    y = ops.dense_ffn_q8(x, wg, sg, wu, su, wd, sd)
+    h = ops.silu_mul(ops.matmul_q_s(x, wg, sg), ops.matmul_q_s(x, wu, su))
+    assert torch.equal(y, ops.matmul_q_s(h, wd, sd))
+
+
 def test_matmul_q8_extremes(ops):
     # w = -128 everywhere and activations at +-127 (simd_tests.c rep 0)
     S, I, O = 9, 4096, 40
