@@ -24,6 +24,8 @@
 #include "common.h"
 #include "kernels.h"
 
+#include <type_traits>
+
 namespace moty {
 
 // ---------------------------------------------------------------------------
@@ -386,284 +388,341 @@ static int launch_r4_gemv(const float* x, const uint8_t* W, const uint16_t* d16,
 }
 
 // ---------------------------------------------------------------------------
-// Prefill GEMM on v_mfma_i32_32x32x32_i8: one MFMA per group (K = 32 = the
-// group), so each group's integer sum comes out separately and is folded
-// into the float chain per output in group order.  Block tile 64 tokens x 64
-// weight rows, 4 waves as 2 x 2 (32 x 32 each).  Per K block of 4 groups the
-// workgroup stages in LDS, by whole-line loads: the tokens' int8 codes, the
-// weight codes (Q4R4: 16 packed bytes per row and group, unpacked to low /
-// high nibbles for the two MFMA halves; Q8R4: 32 codes), the decoded f16
-// scales per (row, group), and per (group, token) the activation scale xs,
-// the integer offset m8 = -8*xsum for per-token-kernel tokens (else 0) and
-// the tile kernel's offset term xct = (8*xsum)*xs (0 for per-token tokens):
+// Prefill GEMM on int8 MFMA, one per group (K = 32 = the group), so each
+// group's integer sum comes out separately and is folded into the float chain
+// per output in group order:
 //   acc = fma(float(s + m8), dd*xs, acc);  acc = fma(-dd, xct, acc)
+// with m8 = -8*xsum for per-token-kernel tokens (t >= 4*floor(S/4); else 0)
+// and xct the tile kernel's offset term (8*xsum)*xs (0 for per-token tokens)
 // reproduces both reference forms (the second FMA adds -dd*0 to a nonzero-
 // signed or +0 accumulator: exactly nothing).  Q8R4 runs the first FMA only.
-// WV = 8 / 16: eight waves of 16 tokens x 32 rows each (two
-// v_mfma_i32_16x16x32_i8 per group) or sixteen of 16 x 16, over the same block tile and staging (done by the first four
-// waves), for grids that give one workgroup per CU: two waves per SIMD
-// instead of one.  Lane l's fragments: A = codes [8(l/16), +8) of token row
-// l % 16; B = the same k of weight row l % 16 -- for Q4R4 the low (k < 16)
-// or high nibbles of bytes [8(l/16 % 2), +8) of the row's 16 group bytes,
-// byte j holding codes j and j + 16.
-constexpr int R4M_NT = 256;
-constexpr int R4M_KG = 4;                 // groups per K block
-constexpr int R4M_AS = R4M_KG * 32 + 16;  // A row stride (bytes)
+//
+// The weight rows are the MFMA's rows and the tokens its columns: a lane then
+// holds one token (of each token tile), whose xs and xct it reads once per
+// group, and reads the scales dd of its 16 rows as four float4s, shared by
+// all its token tiles.  With the operands the other way round the per-token
+// xs, xct and m8 were 8-12 ds_read_b128 per group and 32 x 32 outputs, and
+// the CU's LDS pipe, 14 reads x 4 waves x 8 clocks = 448, was the whole time
+// (424 clocks measured for 275 of MFMA and vector work).  What is left is
+// that work: 34 clocks of MFMA and 64 vector operations (convert, dd*xs, two
+// FMAs) of 2.6 per 16 registers, which do not overlap on a SIMD.
+//
+// Tiles of MT x MT outputs (32: v_mfma_i32_32x32x32_i8; 16: 16x16x32, for
+// grids that leave SIMDs idle), RT row tiles x TT token tiles per wave, WR x
+// WT waves.  PAIR: W is a row-fused [gate; up] matrix of 2*O rows, RT = 2,
+// tile 0 gate rows and tile 1 the same up rows, y [S][O] = silu(gate) * up
+// (the gate_up + silu_rows of nn/ffn.c:28-37).  Steps of 4 groups are
+// double-buffered in LDS, one barrier each, with the next two on their way to
+// registers (with one, the load latency of a step was its time on small grids).
+constexpr int R4M_KG = 4;                 // groups per K step
+constexpr int R4M_AS = R4M_KG * 32 + 16;  // LDS row stride of the token codes (bytes)
 
-// PAIR (WV = 4): W is a row-fused [gate; up] matrix of 2*O rows; the tile's
-// first 32 weight rows are gate rows 32*bx + [0, 32), the last 32 the up rows
-// O + 32*bx + [0, 32), and the epilogue writes y [S][O] = silu(gate) * up
-// (the gate_up + silu_rows of nn/ffn.c:28-37; the up waves hand their sums
-// over through LDS).
-template <bool Q8, bool TILE = false, int WV = 4, bool PAIR = false>
-__global__ __launch_bounds__(64 * WV, WV <= 8 ? 8 / WV : 1) void k_r4_gemm(const int8_t* __restrict__ xq, const float* __restrict__ xs,
-                                                       const int32_t* __restrict__ xm,
-                                                       const uint8_t* __restrict__ W,
-                                                       const uint16_t* __restrict__ d16, float* __restrict__ y,
-                                                       int S, int I, int O) {
-  constexpr int GB = Q8 ? 128 : 64;
-  constexpr int RB = Q8 ? 32 : 16;          // bytes per (row, group)
-  constexpr int BS = R4M_KG * RB + 16;      // B row stride (bytes)
-  constexpr int NBC = Q8 ? 2 : 1;           // B chunks per thread
-  constexpr int NWN = WV / 4, JN = 4 / NWN;  // WV >= 8: waves along the rows, 16-row tiles per wave
-  static_assert(WV == 4 || WV == 8 || WV == 16, "waves");
-  static_assert(!PAIR || WV == 4, "PAIR runs the 32 x 32 waves");
-  __shared__ __align__(16) int8_t sA[64 * R4M_AS];
-  __shared__ __align__(16) uint8_t sB[64 * BS];
-  __shared__ float sD[64 * R4M_KG];         // [row][group]
-  __shared__ __align__(16) float sX[R4M_KG * 64], sC[R4M_KG * 64];  // [group][token]
-  __shared__ __align__(16) int sM[R4M_KG * 64];
-  const int tid = threadIdx.x, lane = tid % MOTY_WAVE, wv = tid / MOTY_WAVE;
-  const int wm = wv >> 1, wn = wv & 1;
-  const int r32 = lane & 31, hk = lane >> 5;
-  const int mb = blockIdx.y * 64, nb0 = blockIdx.x * (PAIR ? 32 : 64);
-  const int nb = I / 32, S4 = S / 4 * 4;
+typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+
+template <bool Q8, bool PAIR, int MT, int RT, int TT, int WR, int WT>
+__global__ __launch_bounds__(64 * WR * WT, 2) void k_r4_gemm(const int8_t* __restrict__ xq, const float* __restrict__ xs,
+                                                          const int32_t* __restrict__ xm,
+                                                          const uint8_t* __restrict__ W,
+                                                          const uint16_t* __restrict__ d16, float* __restrict__ y,
+                                                          int S, int I, int O) {
+  static_assert(!PAIR || RT == 2, "PAIR: a gate and an up tile");
+  constexpr int NT = 64 * WR * WT;
+  constexpr int GB = Q8 ? 128 : 64, RB = Q8 ? 32 : 16;  // bytes of a block and group, of a row and group
+  constexpr int BT = MT * TT * WT, BR = MT * RT * WR;   // tokens, weight rows of the tile
+  constexpr int OC = PAIR ? BR / 2 : BR;                // output columns
+  constexpr int BS = R4M_KG * RB + 16;                  // LDS row stride of the weight codes (bytes)
+  constexpr int NQ = MT / 8;                            // float4s of rows per lane: 4 (MT 32) or 2
+  constexpr int ND = MT == 32 ? 16 : 4;                 // registers of a tile
+  constexpr int AC = BT * R4M_KG * 2, BC = BR * R4M_KG * (RB / 16), DC = BR / 4 * R4M_KG, TC = BT * R4M_KG;
+  constexpr int NA = (AC + NT - 1) / NT, NB = (BC + NT - 1) / NT, NDC = (DC + NT - 1) / NT, NTC = (TC + NT - 1) / NT;
+  __shared__ __align__(16) int8_t sA[2][BT * R4M_AS];
+  __shared__ __align__(16) uint8_t sB[2][BR * BS];
+  __shared__ __align__(16) float sD[2][R4M_KG * BR];  // [group][row]
+  __shared__ __align__(16) float sX[2][R4M_KG * BT], sC[2][Q8 ? 4 : R4M_KG * BT];  // [group][token]
+  __shared__ int sM[2][Q8 ? 4 : R4M_KG * BT];
+  __shared__ uint64_t s_exp[PAIR ? 32 : 1];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int wr = wv % WR, wt = wv / WR;
+  const int rl = lane % MT, hk = lane / MT;  // this lane's row / token of a tile, its K part
+  const int mb = blockIdx.y * BT, ob = blockIdx.x * OC;
+  const int nb = I / 32, S4 = S / 4 * 4, nstep = (nb + R4M_KG - 1) / R4M_KG;
   const int O4 = ((PAIR ? 2 * O : O) + 3) / 4;
+  const bool tile = Q8 || mb + BT <= S4 || S == S4;  // no per-token tokens here: m8 is 0 throughout
+  if (PAIR) exp_tab_lds(s_exp);
 
-  // copy assignments
-  const int8_t* srcA[2];
-#pragma unroll
-  for (int i = 0; i < 2; i++) {
-    const int q = tid + i * R4M_NT;
-    int m = mb + (q >> 3);
-    m = m < S ? m : S - 1;
-    srcA[i] = xq + (int64_t)m * I + (q & 7) * 16;
-  }
-  // B: thread -> (row tid/4, group tid%4), Q8R4 two 16-byte halves
-  const int trow = tid >> 2;
-  int orow = !PAIR ? nb0 + trow : trow < 32 ? nb0 + trow : O + nb0 + trow - 32;
-  int ob = orow / 4;
-  ob = ob < O4 ? ob : O4 - 1;
-  const uint8_t* srcB = W + (size_t)ob * nb * GB + (size_t)(orow & 3) * RB;
-  const uint16_t* srcD = d16 + (size_t)ob * nb * 4 + (orow & 3);
-  // token scales: thread -> (group tid/64, token tid%64)
-  const int st_t = mb + (tid & 63), st_g = tid >> 6;
-  const int st_tc = st_t < S ? st_t : S - 1;
-  const bool st_tile = st_t < S4;
-
+  // staging.  Rows past the end re-read the last block or token; groups past
+  // the end group 0 (their scales and codes are zeroed when staged).
+  auto blk = [&](int r4) {  // global 4-row block of tile row 4 * r4
+    const int row = 4 * r4, o = PAIR && row >= OC ? O + ob + row - OC : ob + row;
+    return o / 4 < O4 ? o / 4 : O4 - 1;
+  };
+  // Every load is unconditional, from clamped piece numbers and addresses
+  // (the last piece is then stored more than once, the same bytes): with no
+  // branch around a load the compiler waits for the set it needs alone.
   struct Set {
-    int4 a[2];
-    int4 b[NBC];
-    uint32_t d;
-    float x;
-    int m;
+    v4i a[NA], b[NB];
+    u32x2_a2 d[NDC];
+    float x[NTC];
+    int m[NTC];
   };
   Set s0, s1;
-  const bool stager = WV == 4 || tid < R4M_NT;  // wave-uniform
-  const int glast = (nb - 1) / R4M_KG * R4M_KG;
-  auto gload = [&](int g0, Set& sv) {
-    if (!stager) return;
-    const int gc = g0 < nb ? g0 : glast;
-    const int kb = gc * 32;
+  auto piece = [&](int i, int n) { return n % NT == 0 || tid + i * NT < n ? tid + i * NT : n - 1; };
+  // The pieces' addresses are set up once and move by the same bytes every
+  // step; only a last step that is not full looks at each piece's group.
+  const int8_t* pa[NA];
+  const uint8_t* pb[NB];
+  const uint16_t* pd[NDC];
+  uint32_t px[NTC];
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-      const int q = tid + i * R4M_NT;
-      sv.a[i] = *(const int4*)(srcA[i] + (kb + (q & 7) * 16 < I ? kb : -(q & 7) * 16));
+  for (int i = 0; i < NA; i++) {
+    const int c = piece(i, AC), t = c / (2 * R4M_KG), m = mb + t < S ? mb + t : S - 1;
+    pa[i] = xq + (int64_t)m * I + c % (2 * R4M_KG) * 16;
+  }
+  constexpr int PB = R4M_KG * GB / 16;  // a block's 16-byte pieces of a step: consecutive threads take consecutive ones
+#pragma unroll
+  for (int i = 0; i < NB; i++) {
+    const int c = piece(i, BC);
+    pb[i] = W + (size_t)blk(c / PB) * nb * GB + c % PB * 16;
+  }
+#pragma unroll
+  for (int i = 0; i < NDC; i++) {
+    const int c = piece(i, DC);
+    pd[i] = d16 + ((size_t)blk(c / R4M_KG) * nb + c % R4M_KG) * 4;
+  }
+#pragma unroll
+  for (int i = 0; i < NTC; i++) {
+    const int c = piece(i, TC), t = c / R4M_KG, m = mb + t < S ? mb + t : S - 1;
+    px[i] = (uint32_t)m * nb + c % R4M_KG;
+  }
+  auto gload = [&](int st, Set& v) {
+    const int s = st < nstep ? st : nstep - 1, left = nb - s * R4M_KG;  // uniform
+    // a piece of a group past the row's end takes the row's first piece
+#pragma unroll
+    for (int i = 0; i < NA; i++) {
+      const int k = piece(i, AC) % (2 * R4M_KG);
+      v.a[i] = *(const v4i*)(pa[i] + (k / 2 < left ? s * (R4M_KG * 32) : -k * 16));
     }
-    const int g = gc + (tid & 3) < nb ? gc + (tid & 3) : 0;
 #pragma unroll
-    for (int i = 0; i < NBC; i++) sv.b[i] = *(const int4*)(srcB + (size_t)g * GB + 16 * i);
-    sv.d = srcD[(size_t)g * 4];
-    const int gt = gc + st_g < nb ? gc + st_g : 0;
-    sv.x = xs[(size_t)st_tc * nb + gt];
-    sv.m = xm[(size_t)st_tc * nb + gt];
+    for (int i = 0; i < NB; i++) {
+      const int q = piece(i, BC) % PB;
+      v.b[i] = *(const v4i*)(pb[i] + (q / (GB / 16) < left ? s * (R4M_KG * GB) : -q * 16));
+    }
+#pragma unroll
+    for (int i = 0; i < NDC; i++) {
+      const int k = piece(i, DC) % R4M_KG;
+      v.d[i] = *(const u32x2_a2*)(pd[i] + (k < left ? s * (R4M_KG * 4) : -k * 4));
+    }
+#pragma unroll
+    for (int i = 0; i < NTC; i++) {
+      const int k = piece(i, TC) % R4M_KG;
+      const uint32_t at = px[i] + (k < left ? s * R4M_KG : -k);
+      v.x[i] = xs[at];
+      if (!Q8) v.m[i] = xm[at];
+    }
     __builtin_amdgcn_sched_barrier(0);
   };
-  float accf[16];
+  auto put = [&](int p, const Set& v) {
 #pragma unroll
-  for (int r = 0; r < 16; r++) accf[r] = 0.f;
-  auto stage = [&](int g0, Set& sv) {
-    const int kb = g0 * 32;
-    if (stager) {
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-      const int q = tid + i * R4M_NT;
-      *(int4*)(sA + (q >> 3) * R4M_AS + (q & 7) * 16) = sel4(kb + (q & 7) * 16 < I, sv.a[i]);
+    for (int i = 0; i < NA; i++) {
+      const int c = piece(i, AC), t = c / (2 * R4M_KG), k = c % (2 * R4M_KG);
+      *(v4i*)(sA[p] + t * R4M_AS + k * 16) = v.a[i];
     }
-    const bool gok = g0 + (tid & 3) < nb;
 #pragma unroll
-    for (int i = 0; i < NBC; i++) *(int4*)(sB + (tid >> 2) * BS + (tid & 3) * RB + 16 * i) = sel4(gok, sv.b[i]);
-    sD[(tid >> 2) * R4M_KG + (tid & 3)] = gok ? f16_to_f32(sv.d) : 0.f;
-    {
-      const bool ok = g0 + st_g < nb;
-      const float xv = ok ? sv.x : 0.f;
-      sX[st_g * 64 + (tid & 63)] = xv;
-      sM[st_g * 64 + (tid & 63)] = (ok && !st_tile) ? -8 * sv.m : 0;
-      sC[st_g * 64 + (tid & 63)] = (ok && st_tile) ? (8.f * (float)sv.m) * xv : 0.f;
+    for (int i = 0; i < NB; i++) {
+      constexpr int PR = RB / 16;
+      const int c = piece(i, BC), r4 = c / PB, q = c % PB, k = q / (GB / 16), h = q % (GB / 16);
+      *(v4i*)(sB[p] + (r4 * 4 + h / PR) * BS + k * RB + h % PR * 16) = v.b[i];
     }
+#pragma unroll
+    for (int i = 0; i < NDC; i++) {
+      const int c = piece(i, DC), r4 = c / R4M_KG, k = c % R4M_KG;
+      const auto h = [](uint32_t u) { return (float)__builtin_bit_cast(_Float16, (uint16_t)u); };  // exact
+      *(float4*)(sD[p] + k * BR + r4 * 4) = float4{h(v.d[i].x & 0xffffu), h(v.d[i].x >> 16),
+                                                   h(v.d[i].y & 0xffffu), h(v.d[i].y >> 16)};
     }
-    __syncthreads();
-    gload(g0 + 2 * R4M_KG, sv);
-    if constexpr (WV >= 8) {
-      // wave: tokens wm16 * 16 + [0, 16) x rows wn16 * 16 * JN + [0, 16 * JN)
-      const int wm16 = wv / NWN, wn16 = wv % NWN, r16 = lane & 15, q4 = lane >> 4;
-      const int ngk = (nb - g0) < R4M_KG ? (nb - g0) : R4M_KG;
-      const int tb = wm16 * 16 + 4 * q4;  // this lane's 4 tokens (D rows)
 #pragma unroll
-      for (int gg = 0; gg < R4M_KG; gg++) {
-        if (gg >= ngk) break;  // wave-uniform
-        const long a = *(const long*)(sA + (wm16 * 16 + r16) * R4M_AS + gg * 32 + q4 * 8);
-        const float4 xv = *(const float4*)(sX + gg * 64 + tb);
-        const int4 mv = (Q8 || TILE) ? int4{0, 0, 0, 0} : *(const int4*)(sM + gg * 64 + tb);
-        const float4 cv = Q8 ? float4{0.f, 0.f, 0.f, 0.f} : *(const float4*)(sC + gg * 64 + tb);
+    for (int i = 0; i < NTC; i++) {
+      const int c = piece(i, TC), t = c / R4M_KG, k = c % R4M_KG;
+      sX[p][k * BT + t] = v.x[i];
+      if (!Q8) {
+        const bool per_token = mb + t >= S4;
+        sC[p][k * BT + t] = per_token ? 0.f : (8.f * (float)v.m[i]) * v.x[i];
+        sM[p][k * BT + t] = per_token ? -8 * v.m[i] : 0;
+      }
+    }
+  };
+
+  float acc[RT][TT][ND];
 #pragma unroll
-        for (int jn = 0; jn < JN; jn++) {
-          const int row = wn16 * 16 * JN + jn * 16 + r16;
-          long b;
+  for (int j = 0; j < RT; j++)
+#pragma unroll
+    for (int i = 0; i < TT; i++)
+#pragma unroll
+      for (int r = 0; r < ND; r++) acc[j][i][r] = 0.f;
+  auto row0 = [&](int j) { return PAIR ? j * OC + wr * MT : (wr * RT + j) * MT; };  // first tile row of row tile j
+
+  // NG groups from gg on: every fragment and MFMA first, then the chains in
+  // group order, so the reads and MFMAs of one group hide behind another's
+  typedef typename std::conditional<MT == 32, v16i, v4i>::type vd;
+  auto groups = [&](int p, int gg, auto ngs, auto tl) {
+    constexpr int NG = decltype(ngs)::value;
+    constexpr bool TILE = decltype(tl)::value;
+    vd d[NG][RT][TT];
+    float xv[NG][TT], cv[NG][TT];
+    int mv[NG][TT];
+#pragma unroll
+    for (int g = 0; g < NG; g++) {
+      if constexpr (MT == 32) {
+        v4i fb[TT];
+#pragma unroll
+        for (int i = 0; i < TT; i++)
+          fb[i] = *(const v4i*)(sA[p] + ((wt * TT + i) * 32 + rl) * R4M_AS + (gg + g) * 32 + hk * 16);
+#pragma unroll
+        for (int j = 0; j < RT; j++) {
+          v4i fa;
           if (Q8) {
-            b = *(const long*)(sB + row * BS + gg * RB + q4 * 8);
-          } else {
-            const uint2 w = *(const uint2*)(sB + row * BS + gg * RB + (q4 & 1) * 8);
-            const int sh = (q4 >> 1) * 4;
-            b = (long)(((w.x >> sh) & 0x0f0f0f0fu) | ((uint64_t)((w.y >> sh) & 0x0f0f0f0fu) << 32));
+            fa = *(const v4i*)(sB[p] + (row0(j) + rl) * BS + (gg + g) * RB + hk * 16);
+          } else {  // low nibbles for hk = 0 (codes 0..15), high for hk = 1
+            const v4i w = *(const v4i*)(sB[p] + (row0(j) + rl) * BS + (gg + g) * RB);
+#pragma unroll
+            for (int q = 0; q < 4; q++) fa[q] = (w[q] >> (4 * hk)) & 0x0f0f0f0f;
           }
-          const v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, v4i{0, 0, 0, 0}, 0, 0, 0);
-          const float dd = sD[row * R4M_KG + gg];
-          float* ac = accf + 4 * jn;
+#pragma unroll
+          for (int i = 0; i < TT; i++) d[g][j][i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa, fb[i], vd{}, 0, 0, 0);
+        }
+      } else {
+        long fb[TT];
+#pragma unroll
+        for (int i = 0; i < TT; i++)
+          fb[i] = *(const long*)(sA[p] + ((wt * TT + i) * 16 + rl) * R4M_AS + (gg + g) * 32 + hk * 8);
+#pragma unroll
+        for (int j = 0; j < RT; j++) {
+          long fa;
           if (Q8) {
-            ac[0] = __fmaf_rn((float)d[0], dd * xv.x, ac[0]);
-            ac[1] = __fmaf_rn((float)d[1], dd * xv.y, ac[1]);
-            ac[2] = __fmaf_rn((float)d[2], dd * xv.z, ac[2]);
-            ac[3] = __fmaf_rn((float)d[3], dd * xv.w, ac[3]);
-          } else {
-            ac[0] = __fmaf_rn(-dd, cv.x, __fmaf_rn((float)(d[0] + mv.x), dd * xv.x, ac[0]));
-            ac[1] = __fmaf_rn(-dd, cv.y, __fmaf_rn((float)(d[1] + mv.y), dd * xv.y, ac[1]));
-            ac[2] = __fmaf_rn(-dd, cv.z, __fmaf_rn((float)(d[2] + mv.z), dd * xv.z, ac[2]));
-            ac[3] = __fmaf_rn(-dd, cv.w, __fmaf_rn((float)(d[3] + mv.w), dd * xv.w, ac[3]));
+            fa = *(const long*)(sB[p] + (row0(j) + rl) * BS + (gg + g) * RB + hk * 8);
+          } else {  // K part hk: codes 8 hk .. + 8, nibbles hk / 2 of bytes 8 (hk % 2) ..
+            const uint2 w = *(const uint2*)(sB[p] + (row0(j) + rl) * BS + (gg + g) * RB + (hk & 1) * 8);
+            const int sh = (hk >> 1) * 4;
+            fa = (long)(((w.x >> sh) & 0x0f0f0f0fu) | ((uint64_t)((w.y >> sh) & 0x0f0f0f0fu) << 32));
           }
+#pragma unroll
+          for (int i = 0; i < TT; i++) d[g][j][i] = __builtin_amdgcn_mfma_i32_16x16x32_i8(fa, fb[i], vd{}, 0, 0, 0);
         }
       }
-    } else if constexpr (Q8) {
-      // Straight-line over the block's groups -- fragments, the MFMAs, then
-      // the epilogues in group order -- so the MFMAs overlap.  Groups past
-      // the row end hold zero codes and scales: their steps add exactly
-      // nothing (fma(0, 0, acc) = acc; acc is never -0).
-      if (g0 < nb) {
-        v4i af[R4M_KG], bf[R4M_KG];
 #pragma unroll
-        for (int gg = 0; gg < R4M_KG; gg++) {
-          af[gg] = *(const v4i*)(sA + (wm * 32 + r32) * R4M_AS + gg * 32 + hk * 16);
-          bf[gg] = *(const v4i*)(sB + (wn * 32 + r32) * BS + gg * RB + hk * 16);
-        }
-        v16i dsum[R4M_KG];
-#pragma unroll
-        for (int gg = 0; gg < R4M_KG; gg++)
-          dsum[gg] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[gg], bf[gg], v16i{}, 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);  // all MFMAs issue before the epilogues
-#pragma unroll
-        for (int gg = 0; gg < R4M_KG; gg++) {
-          const float dd = sD[(wn * 32 + r32) * R4M_KG + gg];
-          // D layout: lane l, register r -> token 8*(r/4) + 4*(l/32) + r%4, row l%32
-#pragma unroll
-          for (int q = 0; q < 4; q++) {
-            const float4 xv = *(const float4*)(sX + gg * 64 + wm * 32 + 8 * q + 4 * hk);
-            accf[4 * q + 0] = __fmaf_rn((float)dsum[gg][4 * q + 0], dd * xv.x, accf[4 * q + 0]);
-            accf[4 * q + 1] = __fmaf_rn((float)dsum[gg][4 * q + 1], dd * xv.y, accf[4 * q + 1]);
-            accf[4 * q + 2] = __fmaf_rn((float)dsum[gg][4 * q + 2], dd * xv.z, accf[4 * q + 2]);
-            accf[4 * q + 3] = __fmaf_rn((float)dsum[gg][4 * q + 3], dd * xv.w, accf[4 * q + 3]);
-          }
-        }
+      for (int i = 0; i < TT; i++) {
+        const int t = (gg + g) * BT + (wt * TT + i) * MT + rl;
+        xv[g][i] = sX[p][t];
+        cv[g][i] = Q8 ? 0.f : sC[p][t];
+        mv[g][i] = TILE ? 0 : sM[p][t];
       }
+    }
+    // register r of a tile: row 8 (r / 4) + 4 hk + r % 4 (MT 32), 4 hk + r (MT 16)
+#pragma unroll
+    for (int g = 0; g < NG; g++)
+#pragma unroll
+      for (int j = 0; j < RT; j++)
+#pragma unroll
+        for (int q = 0; q < ND / 4; q++) {
+          const float4 dv = *(const float4*)(sD[p] + (gg + g) * BR + row0(j) + 8 * q + 4 * hk);
+          const float dd[4] = {dv.x, dv.y, dv.z, dv.w};
+#pragma unroll
+          for (int i = 0; i < TT; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+              float& a = acc[j][i][4 * q + r];
+              a = __fmaf_rn((float)(d[g][j][i][4 * q + r] + mv[g][i]), dd[r] * xv[g][i], a);
+              if (!Q8) a = __fmaf_rn(-dd[r], cv[g][i], a);
+            }
+        }
+  };
+  // as many groups at once as 64 registers of sums allow
+  constexpr int NGB = RT * TT * ND * 4 <= 64 ? 4 : (RT * TT * ND * 2 <= 64 ? 2 : 1);
+  auto compute = [&](int p, int n, auto tl) {
+    if (n == R4M_KG) {  // uniform; straight-line: a branch per group would wait for each on its own
+#pragma unroll
+      for (int gg = 0; gg < R4M_KG; gg += NGB) groups(p, gg, std::integral_constant<int, NGB>{}, tl);
     } else {
-      // Q4R4 (a heavier epilogue): group by group, within the register budget
-      const int ngk = (nb - g0) < R4M_KG ? (nb - g0) : R4M_KG;
-#pragma unroll
-      for (int gg = 0; gg < R4M_KG; gg++) {
-        if (gg >= ngk) break;  // wave-uniform
-        const v4i a = *(const v4i*)(sA + (wm * 32 + r32) * R4M_AS + gg * 32 + hk * 16);
-        const int4 w = *(const int4*)(sB + (wn * 32 + r32) * BS + gg * RB);
-        // this half's nibbles (low for hk = 0, high for hk = 1): one shift
-        // and one mask per word in every lane, no divergent branch
-        const int sh = 4 * hk;
-        const int4 u = int4{(w.x >> sh) & 0x0f0f0f0f, (w.y >> sh) & 0x0f0f0f0f, (w.z >> sh) & 0x0f0f0f0f,
-                            (w.w >> sh) & 0x0f0f0f0f};
-        v16i dsum = {};
-        dsum = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, v4i{u.x, u.y, u.z, u.w}, dsum, 0, 0, 0);
-        const float dd = sD[(wn * 32 + r32) * R4M_KG + gg];
-        // D layout: lane l, register r -> token 8*(r/4) + 4*(l/32) + r%4, row l%32
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          const int tb = wm * 32 + 8 * q + 4 * hk;
-          const float4 xv = *(const float4*)(sX + gg * 64 + tb);
-          // every token in the tile kernel's form (S % 4 == 0): m8 is 0 throughout
-          const int4 mv = TILE ? int4{0, 0, 0, 0} : *(const int4*)(sM + gg * 64 + tb);
-          const float4 cv = *(const float4*)(sC + gg * 64 + tb);
-          accf[4 * q + 0] = __fmaf_rn(-dd, cv.x, __fmaf_rn((float)(dsum[4 * q + 0] + mv.x), dd * xv.x, accf[4 * q + 0]));
-          accf[4 * q + 1] = __fmaf_rn(-dd, cv.y, __fmaf_rn((float)(dsum[4 * q + 1] + mv.y), dd * xv.y, accf[4 * q + 1]));
-          accf[4 * q + 2] = __fmaf_rn(-dd, cv.z, __fmaf_rn((float)(dsum[4 * q + 2] + mv.z), dd * xv.z, accf[4 * q + 2]));
-          accf[4 * q + 3] = __fmaf_rn(-dd, cv.w, __fmaf_rn((float)(dsum[4 * q + 3] + mv.w), dd * xv.w, accf[4 * q + 3]));
-        }
-      }
+#pragma unroll 1
+      for (int gg = 0; gg < n; gg++) groups(p, gg, std::integral_constant<int, 1>{}, tl);
     }
-    __syncthreads();
+  };
+
+  auto step = [&](int st, Set& v) {  // v: step st + 1's pieces; step st + 3's next
+    __syncthreads();  // step st is staged; every wave is done with step st - 1
+    const int p = st & 1;
+    put(p ^ 1, v);
+    gload(st + 3, v);
+    const int n = nb - st * R4M_KG < R4M_KG ? nb - st * R4M_KG : R4M_KG;
+    if (tile) compute(p, n, std::true_type{});  // workgroup-uniform
+    else compute(p, n, std::false_type{});
   };
   gload(0, s0);
-  gload(R4M_KG, s1);
-  for (int g0 = 0; g0 < nb; g0 += 2 * R4M_KG) {
-    stage(g0, s0);
-    stage(g0 + R4M_KG, s1);
+  gload(1, s1);
+  put(0, s0);
+  gload(2, s0);
+  for (int st = 0; st < nstep; st += 2) {
+    step(st, s1);
+    if (st + 1 < nstep) step(st + 1, s0);
   }
   // retire the clamped prefetches once before the conditional stores
   __builtin_amdgcn_s_waitcnt(0);
-  if constexpr (WV >= 8) {
-    const int wm16 = wv / NWN, wn16 = wv % NWN, r16 = lane & 15, q4 = lane >> 4;
+  // a lane's registers 4q..4q+3 are four consecutive columns of its token
+  const bool vec = (O & 3) == 0 && (((uintptr_t)y) & 15) == 0;
 #pragma unroll
-    for (int jn = 0; jn < JN; jn++) {
-      const int col = nb0 + wn16 * 16 * JN + jn * 16 + r16;
-      if (col >= O) continue;
+  for (int i = 0; i < TT; i++) {
+    const int t = mb + (wt * TT + i) * MT + rl;
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int t = mb + wm16 * 16 + 4 * q4 + r;
-        if (t < S) y[(int64_t)t * O + col] = accf[4 * jn + r];
+    for (int j = 0; j < (PAIR ? 1 : RT); j++)
+#pragma unroll
+      for (int q = 0; q < ND / 4; q++) {
+        const int o = ob + row0(j) + 8 * q + 4 * hk;
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          v[r] = acc[j][i][4 * q + r];
+          if constexpr (PAIR) v[r] = ref_silu_mul(v[r], acc[1][i][4 * q + r], s_exp);
+        }
+        if (t >= S || o >= O) continue;
+        float* yp = y + (int64_t)t * O + o;
+        if (vec) {
+          *(float4*)yp = float4{v[0], v[1], v[2], v[3]};
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            if (o + r < O) yp[r] = v[r];
+        }
       }
-    }
-    return;
   }
-  if constexpr (PAIR) {
-    // up sums (wn = 1) to the gate waves through LDS, [r][wm][lane]
-    float* xch = (float*)sA;
-    __syncthreads();
-    if (wn == 1) {
-#pragma unroll
-      for (int r = 0; r < 16; r++) xch[r * 128 + wm * 64 + lane] = accf[r];
-    }
-    __syncthreads();
-    const int col = nb0 + r32;
-    if (wn == 1 || col >= O) return;
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const int t = mb + wm * 32 + 8 * (r >> 2) + 4 * hk + (r & 3);
-      if (t < S) y[(int64_t)t * O + col] = ref_silu_mul(accf[r], xch[r * 128 + wm * 64 + lane]);
-    }
-    return;
+}
+
+// Tile shapes of k_r4_gemm: tokens, output columns, and the time of a launch
+// as max(l0 + l1 * n, u * (e + f * n)) us for n steps of 4 groups and u =
+// ceil(tiles / 256) tiles on the busiest CU: a lone tile's step latency, and
+// the SIMDs' work.  Fitted on MI355X to M = 4..500 over (I, O) = (3072, 1024),
+// (9728, 2560), (12288, 4096) and, gate + up, (1024, 3072), (2560, 9728),
+// (4096, 12288).  Small tiles (16 x 16 MFMA) for few tokens: M = 4, 24576 x
+// 4096 36 us and 4096 x 12288 60 us; 64-token ones in 32 x 32 for many: M =
+// 301, 190 and 152 us against 246 and 195 in the former 64 x 64 tiles.
+struct R4Tile {
+  int bt, oc;
+  double l0, l1, e, f;
+};
+static constexpr R4Tile R4_PAIR[2][3] = {{{16, 32, 3.0, 0.85, 1.2, 0.25}, {32, 64, 4.0, 2.0, 2.0, 0.69}, {64, 64, 4.0, 1.95, 4.0, 1.31}},
+                                         {{16, 32, 3.0, 0.75, 1.2, 0.25}, {32, 64, 4.0, 2.0, 2.0, 0.95}, {64, 64, 4.0, 1.75, 4.0, 1.10}}};
+static constexpr R4Tile R4_ONE[2][4] = {{{16, 32, 2.5, 0.60, 1.0, 0.16}, {32, 64, 4.0, 0.87, 2.0, 0.50}, {64, 64, 4.0, 1.22, 4.0, 0.80}, {64, 128, 4.0, 1.52, 6.0, 1.50}},
+                                        {{16, 32, 2.5, 0.52, 1.0, 0.16}, {32, 64, 4.0, 0.72, 2.0, 0.46}, {64, 64, 4.0, 0.90, 4.0, 0.64}, {64, 128, 4.0, 1.15, 6.0, 1.28}}};
+template <int N>
+static int r4_pick(const R4Tile (&t)[N], int S, int I, int O) {
+  int best = 0;
+  double bt = 0;
+  for (int k = 0; k < N; k++) {
+    const int64_t tiles = (int64_t)((S + t[k].bt - 1) / t[k].bt) * ((O + t[k].oc - 1) / t[k].oc);
+    const double n = (I + 32 * R4M_KG - 1) / (32 * R4M_KG), u = (double)((tiles + 255) / 256);
+    const double lone = t[k].l0 + t[k].l1 * n, full = u * (t[k].e + t[k].f * n), us = lone > full ? lone : full;
+    if (k == 0 || us < bt) best = k, bt = us;
   }
-  const int col = nb0 + wn * 32 + r32;
-  if (col >= O) return;
-#pragma unroll
-  for (int r = 0; r < 16; r++) {
-    const int t = mb + wm * 32 + 8 * (r >> 2) + 4 * hk + (r & 3);
-    if (t < S) y[(int64_t)t * O + col] = accf[r];
-  }
+  return best;
 }
 
 // y [S][O] = R4 matmul of x [S][I]; xq/xs/xm: scratch for the activation
@@ -679,25 +738,20 @@ int launch_r4_matmul(bool q8, const float* x, const uint8_t* W, const uint16_t* 
   if (!xq || !xs || !xm) return MOTY_EINVAL;  // the GEMM path needs the activation scratch
   int rc = launch_quant_g32(x, xq, xs, xm, S, I, st);
   if (rc) return rc;
-  dim3 grid((O + 63) / 64, (S + 63) / 64);
-  // at most one workgroup per CU: sixteen waves of 16 x 16 (four per SIMD
-  // instead of one); measured on MI355X at S = 256, 4096 x 12288: Q4R4 92.7
-  // us against 132 with four waves (eight: 112), Q8R4 95.9 against 104.  The
-  // wider grids keep four waves of 32 x 32 (24576 x 4096: 147 us; eight or
-  // sixteen waves 179 / 191).
-  const bool few = (int64_t)grid.x * grid.y <= 256;
-#define R4G(Q, T, WV) \
-  hipLaunchKernelGGL((k_r4_gemm<Q, T, WV>), grid, dim3(64 * WV), 0, st, xq, xs, xm, W, d16, y, S, I, O)
-  if (q8) {
-    if (few) R4G(true, false, 16);
-    else R4G(true, false, 4);
-  } else if (S % 4 == 0) {  // every token in the tile kernel's form
-    if (few) R4G(false, true, 16);
-    else R4G(false, true, 4);
-  } else {
-    if (few) R4G(false, false, 16);
-    else R4G(false, false, 4);
-  }
+  const int k = r4_pick(R4_ONE[q8], S, I, O);
+  const R4Tile& t = R4_ONE[q8][k];
+  const dim3 grid((O + t.oc - 1) / t.oc, (S + t.bt - 1) / t.bt);
+#define R4G(MT, TT, WR, WT)                                                                                      \
+  if (q8)                                                                                                        \
+    hipLaunchKernelGGL((k_r4_gemm<true, false, MT, 1, TT, WR, WT>), grid, dim3(64 * WR * WT), 0, st, xq, xs, xm, \
+                       W, d16, y, S, I, O);                                                                      \
+  else                                                                                                           \
+    hipLaunchKernelGGL((k_r4_gemm<false, false, MT, 1, TT, WR, WT>), grid, dim3(64 * WR * WT), 0, st, xq, xs, xm, \
+                       W, d16, y, S, I, O)
+  if (k == 0) { R4G(16, 1, 2, 1); }
+  else if (k == 1) { R4G(16, 2, 4, 1); }
+  else if (k == 2) { R4G(32, 1, 2, 2); }
+  else { R4G(32, 1, 4, 2); }
 #undef R4G
   LAUNCH_TRY("k_r4_gemm");
   return MOTY_OK;
@@ -711,11 +765,19 @@ int launch_r4_gate_up_gemm(bool q8, const float* x, const uint8_t* W, const uint
   if (S <= 0) return MOTY_OK;
   int rc = launch_quant_g32(x, xq, xs, xm, S, D, st);
   if (rc) return rc;
-  dim3 grid((I + 31) / 32, (S + 63) / 64);
-#define R4P(Q, T) hipLaunchKernelGGL((k_r4_gemm<Q, T, 4, true>), grid, dim3(R4M_NT), 0, st, xq, xs, xm, W, d16, h, S, D, I)
-  if (q8) R4P(true, false);
-  else if (S % 4 == 0) R4P(false, true);
-  else R4P(false, false);
+  const int k = r4_pick(R4_PAIR[q8], S, D, I);
+  const R4Tile& t = R4_PAIR[q8][k];
+  const dim3 grid((I + t.oc - 1) / t.oc, (S + t.bt - 1) / t.bt);
+#define R4P(MT, WR, WT)                                                                                          \
+  if (q8)                                                                                                        \
+    hipLaunchKernelGGL((k_r4_gemm<true, true, MT, 2, 1, WR, WT>), grid, dim3(64 * WR * WT), 0, st, xq, xs, xm,   \
+                       W, d16, h, S, D, I);                                                                      \
+  else                                                                                                           \
+    hipLaunchKernelGGL((k_r4_gemm<false, true, MT, 2, 1, WR, WT>), grid, dim3(64 * WR * WT), 0, st, xq, xs, xm,  \
+                       W, d16, h, S, D, I)
+  if (k == 0) { R4P(16, 2, 1); }
+  else if (k == 1) { R4P(32, 2, 1); }
+  else { R4P(32, 2, 2); }
 #undef R4P
   LAUNCH_TRY("k_r4_gemm<pair>");
   return MOTY_OK;

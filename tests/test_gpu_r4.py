@@ -170,3 +170,34 @@ def test_dense_ffn_r4(ops, q8, S, D, I):
     h = o_silu(y[:, :I], y[:, I:])
     ref = o_matmul_r4(h, q2, d2, D, q8)
     assert same_bits(out, ref), mismatch(out, ref)
+
+
+@pytest.mark.parametrize("q8", [False, True])
+@pytest.mark.parametrize("O,I,S", [
+    # every tile of the several-token GEMM (16 x 32, 32 x 64, 64 x 64, 64 x
+    # 128), ragged in rows and tokens (S % 4 != 0: both of the reference's
+    # token forms, in one tile and in different ones), 1, 5 and 33 groups
+    (31, 32, 5), (4099, 32, 130), (8201, 32, 70), (8201, 32, 301), (2050, 32, 503), (8201, 32, 701), (101, 1056, 70),
+    (4100, 160, 131), (36, 160, 64)])
+def test_matmul_r4_tiles(ops, q8, O, I, S):
+    say("matmul r4 tiles", q8, O, I, S)
+    q, d = o_pack_r4(randn(O + I, (O, I), 0.02), q8)
+    x = randn(S + 3, (S, I))
+    y = to_np(ops.matmul_r4(to_dev(x), to_dev(q), to_dev(d.view(np.int16)), O, q8))
+    y2 = o_matmul_r4(x, q, d, O, q8)
+    assert same_bits(y, y2), mismatch(y, y2)
+
+
+@pytest.mark.parametrize("q8", [False, True])
+@pytest.mark.parametrize("S,D,I", [(5, 32, 96), (70, 32, 8224), (130, 32, 4128), (35, 32, 8224), (67, 288, 160)])
+def test_dense_ffn_r4_tiles(ops, q8, S, D, I):
+    """The gate + up form of the same tiles against the plain matmul, SiLU
+    and the plain matmul again."""
+    say("dense_ffn r4 tiles", q8, S, D, I)
+    gu = ops.pack_r4(to_dev(randn(S + D, (2 * I, D), 0.02)), q8)
+    dn = ops.pack_r4(to_dev(randn(S + I, (D, I), 0.02)), q8)
+    x = to_dev(randn(S + 5, (S, D)))
+    y = ops.dense_ffn_r4(x, *gu, *dn, I, q8)
+    gu_y = ops.matmul_r4(x, *gu, 2 * I, q8)
+    h = ops.silu_mul(gu_y[:, :I].contiguous(), gu_y[:, I:].contiguous())
+    assert torch.equal(y, ops.matmul_r4(h, *dn, D, q8))
