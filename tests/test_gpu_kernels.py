@@ -95,6 +95,20 @@ def test_qrow_i8_rows(ops, S, I):
     assert same_bits(to_np(sx), sx2) and same_bits(to_np(q), q2)
 
 
+@pytest.mark.parametrize("S,I", [(1, 4100), (3, 8192), (2, 12288), (5, 16380), (2, 16384), (3, 2052), (2, 16400)])
+def test_qrow_i8_wide_rows(ops, S, I):
+    """Rows past the wave form's: held in the registers of one workgroup up
+    to 16384 (2, 4, 6 or 8 float4s a thread, the last ones partial)."""
+    say("qrow wide", S, I)
+    x = randn(S * I + 9, (S, I)) * 3
+    x[0, I - 1] = 77.0  # the maximum in the last element
+    if S > 1:
+        x[1] = 0.0
+    q, sx, _ = ops.qrow_i8(to_dev(x), group_sums=False)
+    q2, sx2 = o_qrow(x)
+    assert same_bits(to_np(sx), sx2) and same_bits(to_np(q), q2)
+
+
 def test_qrow_zero_row(ops):
     q, sx, _ = ops.qrow_i8(torch.zeros((2, 64), device="cuda:0"))
     assert (to_np(sx) == np.float32(1e-12)).all() and not to_np(q).any()
