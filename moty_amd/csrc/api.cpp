@@ -125,9 +125,29 @@ static bool capturing(hipStream_t st) {
   return hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
 }
 
+// The first time a second stream uses the arena: everything queued so far is
+// waited for once, and from then on each use records an event (scratch_mark).
+// In the relaxed capture mode, so that a capture the caller has open on some
+// other stream neither forbids the wait nor is broken by it.
+static int scratch_second_stream(Dev* d, hipStream_t st) {
+  d->scr_multi = true;
+  if (capturing(st) || d->scr_cap) return MOTY_OK;  // captured work is ordered by the caller
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  const hipError_t e = hipDeviceSynchronize();
+  if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  return e == hipSuccess ? MOTY_OK : check_hip(e, "scratch hand-over between streams");
+}
+
 int scratch_get(Dev* d, size_t bytes, hipStream_t st, void** p) {
-  if (d->scr_used && d->scr_stream != st && d->scr_ev_ok && !capturing(st))
-    HIP_TRY(hipStreamWaitEvent(st, d->scr_ev, 0));
+  if (d->scr_used && d->scr_stream != st) {
+    if (!d->scr_multi) {
+      const int rc = scratch_second_stream(d, st);
+      if (rc) return rc;
+    } else if (d->scr_ev_ok && !capturing(st)) {
+      HIP_TRY(hipStreamWaitEvent(st, d->scr_ev, 0));
+    }
+  }
   int rc = arena_get(d->scratch, bytes, p);
   if (rc) return rc;
   d->scr_stream = st;
@@ -139,7 +159,11 @@ int scratch_get(Dev* d, size_t bytes, hipStream_t st, void** p) {
 void scratch_mark(Dev* d) {
   d->scr_pend = false;
   d->scr_ev_ok = false;
-  if (capturing(d->scr_stream)) return;
+  // One stream so far: no event.  A program that keeps to one stream then
+  // pays neither the record (about 3 us of a 14 us decode call) nor its
+  // barrier between the kernels of successive calls.
+  d->scr_cap = capturing(d->scr_stream);
+  if (d->scr_cap || !d->scr_multi) return;
   if (!d->scr_ev && hipEventCreateWithFlags(&d->scr_ev, hipEventDisableTiming) != hipSuccess) {
     d->scr_ev = nullptr;
     return;
@@ -253,7 +277,7 @@ int moty_hip_shutdown(void) {
     d.stream = nullptr;
     if (d.scr_ev) hipEventDestroy(d.scr_ev);
     d.scr_ev = nullptr;
-    d.scr_used = d.scr_pend = d.scr_ev_ok = false;
+    d.scr_used = d.scr_pend = d.scr_ev_ok = d.scr_multi = d.scr_cap = false;
     if (d.fx_ev) hipEventDestroy(d.fx_ev);
     d.fx_ev = nullptr;
     d.fx_used = d.fx_ev_ok = false;

@@ -25,13 +25,14 @@ struct Dev {
   int cus = 0;  // compute units
   hipStream_t stream = nullptr;
   Arena scratch, io;
-  // the stream whose queued work last used `scratch`, and an event recorded
-  // on it when that call returned (after its work was queued) that orders a
-  // later call on another stream behind that work; scr_pend: a call took the
-  // arena and has not returned yet; scr_ev_ok: scr_ev marks the last use
-  // (false when that use was under graph capture)
+  // the stream whose queued work last used `scratch`; scr_multi: more than
+  // one stream has used it, and from then on an event recorded on the stream
+  // when a call returns (after its work was queued) orders a later call on
+  // another stream behind that work; scr_pend: a call took the arena and has
+  // not returned yet; scr_ev_ok: scr_ev marks the last use; scr_cap: the last
+  // use was under graph capture (and left no event)
   hipStream_t scr_stream = nullptr;
-  bool scr_used = false, scr_pend = false, scr_ev_ok = false;
+  bool scr_used = false, scr_pend = false, scr_ev_ok = false, scr_multi = false, scr_cap = false;
   hipEvent_t scr_ev = nullptr;
   // device address of this device's copy of the fixed no-allocation
   // scratch array (api.cpp), taken once at set-up, and the same ordering
@@ -60,7 +61,8 @@ int arena_get(Arena& a, size_t bytes, void** p);
 // it).  Streams under graph capture are left unordered.
 int scratch_get(Dev* d, size_t bytes, hipStream_t st, void** p);
 // Called as an entry point returns (ScrGuard): when it took the scratch
-// arena, record scr_ev on its stream, behind the work it queued.
+// arena and several streams use it, record scr_ev on its stream, behind the
+// work it queued.
 void scratch_mark(Dev* d);
 struct ScrGuard {
   Dev* d;

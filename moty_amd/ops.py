@@ -11,11 +11,13 @@ from . import MotyHipMoe, ORDER_EXPERT, check, lib
 
 
 def _p(t):
-    return None if t is None else C.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The raw handle of torch's current stream (current_stream() builds a
+    Stream object around it: 2.7 us of a 14 us decode call)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _dev(*ts):

@@ -227,3 +227,43 @@ def test_moe_olmoe_full_routing_and_sampled_rows(ops):
     # determinism across calls (slot order inside experts is atomic-order)
     y3 = L(to_dev(x))
     assert same_bits(to_np(y), to_np(y3))
+
+
+_TWO_STREAMS = r"""
+import sys
+sys.path.insert(0, {root!r})
+import torch
+from moty_amd import ops
+def q8(O, K, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return (torch.randint(-128, 128, (O, K), generator=g, device="cuda", dtype=torch.int8),
+            torch.rand(O, generator=g, device="cuda") * 1e-4 + 1e-5)
+w = q8(3072, 1024, 1) + q8(3072, 1024, 2) + q8(1024, 3072, 3)
+xs = [torch.randn(S, 1024, device="cuda", generator=torch.Generator(device="cuda").manual_seed(S)) for S in (1500, 7, 900, 3)]
+ss = [torch.cuda.Stream() for _ in range(3)]
+torch.cuda.synchronize()
+# the first use of the arena is queued on one stream and the next, at once, on
+# others (no call has run before: the hand-over the library does once), then
+# on and on between them
+outs = []
+for r in range(6):
+    for k, x in enumerate(xs):
+        with torch.cuda.stream(ss[(r + k) % 3]):
+            outs.append((x, ops.dense_ffn_q8(x, *w)))
+torch.cuda.synchronize()
+for x, y in outs:
+    assert torch.equal(y, ops.dense_ffn_q8(x, *w)), x.shape
+print("two streams ok")
+"""
+
+
+def test_scratch_handed_between_streams_from_the_first_call(dev):
+    """A fresh process: before any call the library keeps no event for its
+    scratch, and the first call on a second stream has to wait all the same."""
+    import os
+    import subprocess
+    import sys
+    say("scratch over streams, fresh process")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", _TWO_STREAMS.format(root=root)], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "two streams ok" in r.stdout, r.stdout[-1000:] + r.stderr[-2000:]
