@@ -78,6 +78,13 @@ static int dev_init(int d) {
       g_dev[d].f1_on = e && e[0] == '1';
     }
     HIP_TRY(hipStreamCreateWithFlags(&g_dev[d].stream, hipStreamNonBlocking));
+    {
+      // a first megabyte of scratch: calls of a few tokens (grouped int4 takes
+      // S * I bytes of codes) can then be captured without ever having run
+      void* p = nullptr;
+      const int rc = arena_get(g_dev[d].scratch, (size_t)1 << 20, &p);
+      if (rc) return rc;
+    }
     g_dev[d].ready = true;
   }
   t_dev = d;
@@ -411,9 +418,9 @@ int moty_hip_matmul_i4_grouped_s_dev(float* y, const float* x, const uint8_t* q4
   hipStream_t st = STREAM(stream);
   if (idot4 && gs == 32 && (I % 64) == 0 && I <= 16384) {
     if (need_al16("matmul_i4_grouped_s", x, q4)) return MOTY_EUNSUP;
-    if (S <= 4) return launch_gemv_i4g(x, q4, scale, nullptr, nullptr, y, S, I, O, st);
+    if (S == 1) return launch_gemv_i4g(x, q4, scale, nullptr, nullptr, y, I, O, st);
     void* sp;
-    if (gemm_i4g_h_fits(S, I, O) && !(((uintptr_t)x | (uintptr_t)q4 | (uintptr_t)scale) & 15)) {
+    if (S > I4G_FEW_MAX && gemm_i4g_h_fits(S, I, O) && !(((uintptr_t)x | (uintptr_t)q4 | (uintptr_t)scale) & 15)) {
       // f16 codes + f16 MFMA: one FMA per output and group in the epilogue
       const size_t hb = al256((size_t)S * I * 2);
       int rc = scratch_get(d, hb + al256((size_t)S * 4), st, &sp);
@@ -430,6 +437,7 @@ int moty_hip_matmul_i4_grouped_s_dev(float* y, const float* x, const uint8_t* q4
     float* sx = (float*)((char*)sp + xb);
     rc = launch_qrow_i8(x, xq, sx, nullptr, S, I, I, I, st);
     if (rc) return rc;
+    if (S <= I4G_FEW_MAX) return launch_gemm_i4g_few(xq, sx, q4, scale, nullptr, nullptr, y, S, I, O, st);
     return launch_gemm_i4g(xq, sx, q4, scale, y, S, I, O, st);
   }
   if (gs == 32 && xf_gemv_per_token(S, I, O, false)) {
@@ -524,7 +532,7 @@ int moty_hip_gate_up_silu_i4g_dev(float* h, const float* x, const uint8_t* gate,
   if (D <= 0 || I <= 0 || !h || !x || !gate || !gs || !up || !us)
     return set_error("gate_up_silu_i4g: bad arguments"), MOTY_EINVAL;
   if (need_al16("gate_up_silu_i4g", x, gate, up)) return MOTY_EUNSUP;
-  int rc = launch_gemv_i4g(x, gate, gs, up, us, h, 1, D, I, STREAM(stream));
+  int rc = launch_gemv_i4g(x, gate, gs, up, us, h, D, I, STREAM(stream));
   if (rc == MOTY_EUNSUP) set_error("gate_up_silu_i4g: D=%d unsupported (D %% 64 == 0, D <= 16384)", D);
   return rc;
 }
@@ -639,7 +647,7 @@ int moty_hip_dense_ffn_i4g_dev(float* out, const float* x, int S, const uint8_t*
   if (idot4 && need_al16("dense_ffn_i4g", x, gate, up, down)) return MOTY_EUNSUP;
   hipStream_t st = STREAM(stream);
   const bool vec = idot4 && (D % 64) == 0 && (I % 64) == 0 && D <= 16384 && I <= 16384;  // both matrices
-  const bool h16 = vec && S > 4 && gemm_i4g_h_fits(S, D, I) && gemm_i4g_h_fits(S, I, D) &&
+  const bool h16 = vec && S > I4G_FEW_MAX && gemm_i4g_h_fits(S, D, I) && gemm_i4g_h_fits(S, I, D) &&
                    !(((uintptr_t)x | (uintptr_t)gate | (uintptr_t)gs | (uintptr_t)up | (uintptr_t)us |
                       (uintptr_t)down | (uintptr_t)ds) & 15);
   const int W = D > I ? D : I;
@@ -660,16 +668,25 @@ int moty_hip_dense_ffn_i4g_dev(float* out, const float* x, int S, const uint8_t*
     return launch_gemm_i4g_h((const uint16_t*)xq, sx, down, ds, nullptr, nullptr, out, S, I, D, st);
   }
   if (vec && S == 1) {
-    if ((rc = launch_gemv_i4g(x, gate, gs, up, us, h, 1, D, I, st))) return rc;
-    return launch_gemv_i4g(h, down, ds, nullptr, nullptr, out, 1, I, D, st);
+    if ((rc = launch_gemv_i4g(x, gate, gs, up, us, h, D, I, st))) return rc;
+    return launch_gemv_i4g(h, down, ds, nullptr, nullptr, out, I, D, st);
+  }
+  if (vec && S <= I4G_FEW_MAX) {
+    int8_t* q = (int8_t*)xq;
+    if ((rc = launch_qrow_i8(x, q, sx, nullptr, S, D, D, D, st))) return rc;
+    if ((rc = launch_gemm_i4g_few(q, sx, gate, gs, up, us, h, S, D, I, st))) return rc;
+    if ((rc = launch_qrow_i8(h, q, sx, nullptr, S, I, I, I, st))) return rc;
+    return launch_gemm_i4g_few(q, sx, down, ds, nullptr, nullptr, out, S, I, D, st);
   }
   // one matmul_i4_grouped_s each, the path chosen per matrix as the
   // reference does (IDOT4 needs the row length a multiple of 64, <= 16384)
   auto mm = [&](const float* a, const uint8_t* w, const float* ws, float* o, int K, int N) -> int {
     if (idot4 && (K % 64) == 0 && K <= 16384) {
-      if (S <= 4) return launch_gemv_i4g(a, w, ws, nullptr, nullptr, o, S, K, N, st);
+      if (S == 1) return launch_gemv_i4g(a, w, ws, nullptr, nullptr, o, K, N, st);
       int r = launch_qrow_i8(a, (int8_t*)xq, sx, nullptr, S, K, K, K, st);
-      return r ? r : launch_gemm_i4g((const int8_t*)xq, sx, w, ws, o, S, K, N, st);
+      if (r) return r;
+      if (S <= I4G_FEW_MAX) return launch_gemm_i4g_few((const int8_t*)xq, sx, w, ws, nullptr, nullptr, o, S, K, N, st);
+      return launch_gemm_i4g((const int8_t*)xq, sx, w, ws, o, S, K, N, st);
     }
     if (xf_gemv_per_token(S, K, N, false)) {
       // exact f32, a few tokens: the one-token GEMV per token (it refuses

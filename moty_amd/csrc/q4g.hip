@@ -19,93 +19,6 @@
 
 namespace moty {
 
-// ---------------------------------------------------------------------------
-// IDOT4 GEMV, S <= 4.  Workgroup: 4 waves, RB rows.  Per 64-group chunk:
-// phase 1 -- every lane computes one group's integer dot for each token
-// (16 B of nibbles, coalesced) and parks it with the group scale in LDS;
-// phase 2 -- one lane per (row, token) extends its FMA chain over the chunk's
-// 64 groups in order.  Activations are quantized into LDS at the start.
-constexpr int Q4V_NT = 256;
-constexpr int Q4V_ROWS = 16;  // rows per workgroup
-
-template <int S_>
-__global__ __launch_bounds__(Q4V_NT) void k_gemv_i4g(const float* __restrict__ x, const uint8_t* __restrict__ q4,
-                                                     const float* __restrict__ scl, float* __restrict__ y, int I,
-                                                     int O) {
-  extern __shared__ __align__(16) int8_t xq_s[];  // [S_][I]
-  __shared__ int dv[Q4V_ROWS][S_][65];
-  __shared__ float sv[Q4V_ROWS][65];
-  __shared__ float red[Q4V_NT / MOTY_WAVE][S_];
-  __shared__ float sx_s[S_];
-  const int lane = threadIdx.x % MOTY_WAVE, wv = threadIdx.x / MOTY_WAVE;
-  const int ng = I / 32, rb = I / 2;
-  const int ob = blockIdx.x * Q4V_ROWS;
-  // activation quantization (qrow_i8) into LDS
-#pragma unroll
-  for (int s = 0; s < S_; s++) {
-    float amax = 0.f;
-    for (int i = threadIdx.x * 4; i < I; i += Q4V_NT * 4) {
-      const float4 v = *(const float4*)(x + (int64_t)s * I + i);
-      amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-    }
-    amax = wave_max_f32(amax);
-    if (lane == 0) red[wv][s] = amax;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int s = 0; s < S_; s++) {
-    float amax = red[0][s];
-    for (int i = 1; i < Q4V_NT / MOTY_WAVE; i++) amax = fmaxf(amax, red[i][s]);
-    float sc = amax / 127.f;
-    if (sc < 1e-12f) sc = 1e-12f;
-    const float inv = 1.f / sc;
-    if (threadIdx.x == 0) sx_s[s] = sc;
-    for (int i = threadIdx.x * 4; i < I; i += Q4V_NT * 4) {
-      const float4 v = *(const float4*)(x + (int64_t)s * I + i);
-      const uint32_t p = (uint32_t)(rne_int(v.x * inv) & 0xff) | ((uint32_t)(rne_int(v.y * inv) & 0xff) << 8) |
-                         ((uint32_t)(rne_int(v.z * inv) & 0xff) << 16) |
-                         ((uint32_t)(rne_int(v.w * inv) & 0xff) << 24);
-      *(uint32_t*)(xq_s + s * I + i) = p;
-    }
-  }
-  __syncthreads();
-  float acc = 0.f;  // chain of lane j = r*S_ + s (j < Q4V_ROWS*S_)
-  const int cr = threadIdx.x / S_, cs = threadIdx.x % S_;
-  for (int c0 = 0; c0 < ng; c0 += 64) {
-    const int g = c0 + lane;
-    for (int r = wv; r < Q4V_ROWS; r += Q4V_NT / MOTY_WAVE) {
-      const int o = ob + r;
-      const bool ok = (o < O) && (g < ng);
-      const int4 wb = ok ? *(const int4*)(q4 + (int64_t)o * rb + g * 16) : int4{0, 0, 0, 0};
-      const float sc = ok ? scl[(int64_t)o * ng + g] : 0.f;
-      const int4 w0 = unpack_nib16(uint2{(uint32_t)wb.x, (uint32_t)wb.y});
-      const int4 w1 = unpack_nib16(uint2{(uint32_t)wb.z, (uint32_t)wb.w});
-#pragma unroll
-      for (int s = 0; s < S_; s++) {
-        int d = 0;
-        if (g < ng) {
-          const int4 x0 = *(const int4*)(xq_s + s * I + g * 32);
-          const int4 x1 = *(const int4*)(xq_s + s * I + g * 32 + 16);
-          d = dot16(w0, x0, 0);
-          d = dot16(w1, x1, d);
-        }
-        dv[r][s][lane] = d;
-      }
-      sv[r][lane] = sc;
-    }
-    __syncthreads();
-    if (threadIdx.x < Q4V_ROWS * S_) {
-      const int n = (ng - c0) < 64 ? (ng - c0) : 64;
-      for (int j = 0; j < n; j++) acc = __fmaf_rn(sv[cr][j], (float)dv[cr][cs][j], acc);
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x < Q4V_ROWS * S_) {
-    const int o = ob + cr;
-    if (o < O) y[(int64_t)cs * O + o] = sx_s[cs] * acc;
-  }
-}
-
 // v_cvt_off_f32_i4 of byte K of w: the signed nibble in bits [8K, 8K+4)
 // divided by 16 (exact), one SDWA-selected conversion
 template <int K>
@@ -1051,54 +964,41 @@ int launch_gemv_i4g_xf(const float* x, const uint8_t* q4, const float* scl, cons
 }
 
 int launch_gemv_i4g(const float* x, const uint8_t* q4, const float* scl, const uint8_t* q4b, const float* sclb,
-                    float* y, int S, int I, int O, hipStream_t st) {
-  if (S < 1 || S > 4 || (I % 64) || I > 16384) return MOTY_EUNSUP;
+                    float* y, int I, int O, hipStream_t st) {
+  if ((I % 64) || I > 16384) return MOTY_EUNSUP;
   if (O <= 0) return MOTY_OK;
-  if (S == 1) {
-    // widest instance whose LDS fits, else the next narrower one
-    const int ngc = (I / 32 + 63) / 64;
-    int rc = MOTY_EUNSUP;
-    if (q4b) {
-      // up to 2 chunks (I <= 4096): 2 gate + 2 up rows per wave (12288 x
-      // 4096 pair: 12.2 us against 12.5 with 4 + 4, 14.2 with 1 + 1, 13.6
-      // for 2 + 2 in 2-wave workgroups or with both chunks issued at once)
-      if (ngc <= 2) rc = go_gemv1_i4g<2, 2, true, 256, 1>(x, q4, scl, q4b, sclb, y, I, O, st);
-      else if (ngc <= 4) {
-        rc = go_gemv1_i4g<2, 4, true, 512>(x, q4, scl, q4b, sclb, y, I, O, st);
-        if (rc == MOTY_EUNSUP) rc = go_gemv1_i4g<2, 4, true, 256>(x, q4, scl, q4b, sclb, y, I, O, st);
-      } else if (ngc <= 8) {
-        rc = go_gemv1_i4g<1, 8, true, 512>(x, q4, scl, q4b, sclb, y, I, O, st);
-        if (rc == MOTY_EUNSUP) rc = go_gemv1_i4g<1, 8, true, 256>(x, q4, scl, q4b, sclb, y, I, O, st);
-      }
-      return rc;
-    }
-    if (ngc <= 2) rc = go_gemv1_i4g<8, 2, false, 256>(x, q4, scl, nullptr, nullptr, y, I, O, st);
+  // widest instance whose LDS fits, else the next narrower one
+  const int ngc = (I / 32 + 63) / 64;
+  int rc = MOTY_EUNSUP;
+  if (q4b) {
+    // up to 2 chunks (I <= 4096): 2 gate + 2 up rows per wave (12288 x
+    // 4096 pair: 12.2 us against 12.5 with 4 + 4, 14.2 with 1 + 1, 13.6
+    // for 2 + 2 in 2-wave workgroups or with both chunks issued at once)
+    if (ngc <= 2) rc = go_gemv1_i4g<2, 2, true, 256, 1>(x, q4, scl, q4b, sclb, y, I, O, st);
     else if (ngc <= 4) {
-      rc = go_gemv1_i4g<4, 4, false, 512>(x, q4, scl, nullptr, nullptr, y, I, O, st);
-      if (rc == MOTY_EUNSUP) rc = go_gemv1_i4g<4, 4, false, 256>(x, q4, scl, nullptr, nullptr, y, I, O, st);
-    } else if (ngc <= 6) {
-      // 4096 x 12288 (8B down) in a sweep of rows/wave x workgroup size x
-      // chunks in flight on MI355X, graph replays over rotating weights:
-      // 4 rows x 256 threads, one chunk ahead 8.0 us; two ahead 9.3, all six
-      // 10.9 (the whole row's chains then run after its last byte lands);
-      // 2 rows 9.6 / 10.9; 8 rows x 128 threads 10.1
-      rc = go_gemv1_i4g<4, 6, false, 256, 1>(x, q4, scl, nullptr, nullptr, y, I, O, st);
+      rc = go_gemv1_i4g<2, 4, true, 512>(x, q4, scl, q4b, sclb, y, I, O, st);
+      if (rc == MOTY_EUNSUP) rc = go_gemv1_i4g<2, 4, true, 256>(x, q4, scl, q4b, sclb, y, I, O, st);
     } else if (ngc <= 8) {
-      rc = go_gemv1_i4g<2, 8, false, 256>(x, q4, scl, nullptr, nullptr, y, I, O, st);
+      rc = go_gemv1_i4g<1, 8, true, 512>(x, q4, scl, q4b, sclb, y, I, O, st);
+      if (rc == MOTY_EUNSUP) rc = go_gemv1_i4g<1, 8, true, 256>(x, q4, scl, q4b, sclb, y, I, O, st);
     }
-    if (rc != MOTY_EUNSUP) return rc;
+    return rc;
   }
-  if (q4b) return MOTY_EUNSUP;
-  const unsigned nb = (unsigned)((O + Q4V_ROWS - 1) / Q4V_ROWS);
-  const size_t lds = (size_t)S * I;
-  switch (S) {
-    case 1: hipLaunchKernelGGL(k_gemv_i4g<1>, dim3(nb), dim3(Q4V_NT), lds, st, x, q4, scl, y, I, O); break;
-    case 2: hipLaunchKernelGGL(k_gemv_i4g<2>, dim3(nb), dim3(Q4V_NT), lds, st, x, q4, scl, y, I, O); break;
-    case 3: hipLaunchKernelGGL(k_gemv_i4g<3>, dim3(nb), dim3(Q4V_NT), lds, st, x, q4, scl, y, I, O); break;
-    default: hipLaunchKernelGGL(k_gemv_i4g<4>, dim3(nb), dim3(Q4V_NT), lds, st, x, q4, scl, y, I, O); break;
+  if (ngc <= 2) rc = go_gemv1_i4g<8, 2, false, 256>(x, q4, scl, nullptr, nullptr, y, I, O, st);
+  else if (ngc <= 4) {
+    rc = go_gemv1_i4g<4, 4, false, 512>(x, q4, scl, nullptr, nullptr, y, I, O, st);
+    if (rc == MOTY_EUNSUP) rc = go_gemv1_i4g<4, 4, false, 256>(x, q4, scl, nullptr, nullptr, y, I, O, st);
+  } else if (ngc <= 6) {
+    // 4096 x 12288 (8B down) in a sweep of rows/wave x workgroup size x
+    // chunks in flight on MI355X, graph replays over rotating weights:
+    // 4 rows x 256 threads, one chunk ahead 8.0 us; two ahead 9.3, all six
+    // 10.9 (the whole row's chains then run after its last byte lands);
+    // 2 rows 9.6 / 10.9; 8 rows x 128 threads 10.1
+    rc = go_gemv1_i4g<4, 6, false, 256, 1>(x, q4, scl, nullptr, nullptr, y, I, O, st);
+  } else if (ngc <= 8) {
+    rc = go_gemv1_i4g<2, 8, false, 256>(x, q4, scl, nullptr, nullptr, y, I, O, st);
   }
-  LAUNCH_TRY("k_gemv_i4g");
-  return MOTY_OK;
+  return rc;
 }
 
 int launch_gemm_i4g(const int8_t* xq, const float* sx, const uint8_t* q4, const float* scl, float* y, int M,
@@ -1341,6 +1241,234 @@ __global__ __launch_bounds__(64 * WM * WN * KS) void k_gemm_i4g_xf(const float* 
         }
       }
     }
+}
+
+// ---------------------------------------------------------------------------
+// IDOT4 for a few tokens: tiles of 16 TM tokens x 16 TN WN weight rows whose
+// K steps are split over KS waves by group, as the exact-f32 form above.  One
+// v_mfma_i32_16x16x32_i8 is a group's integer dots of 16 tokens and 16 rows;
+// the waves hand them over as floats through LDS and a wave per register (and
+// tile) continues the chains acc = fma(scale, d, acc), y = sx * acc.  A step
+// is KG = 8 or 16 groups long: its barrier, LDS and load latencies (0.5-0.7
+// us, whatever it holds) and not the weight stream were the time of the
+// kernels that take 4 groups a step (M = 6..40, 8B FFN: 97 us for 19 us of
+// bytes).  Lane l takes bytes [4 (l / 16), +4) of a row's 16 nibble bytes of
+// the group, low nibbles then high, and the same 8 elements of its token, the
+// even ones first (a k-permutation shared by both operands).
+template <int TM, int TN, int WN, int KS, int KG, bool PAIR>
+__global__ __launch_bounds__(64 * WN * KS, 2) void k_gemm_i4g_few(const int8_t* __restrict__ xq,
+                                                                  const float* __restrict__ sx,
+                                                                  const uint8_t* __restrict__ q4,
+                                                                  const float* __restrict__ scl,
+                                                                  const uint8_t* __restrict__ q4b,
+                                                                  const float* __restrict__ sclb,
+                                                                  float* __restrict__ y, int M, int I, int O) {
+  static_assert(!PAIR || TN == 2, "PAIR: one gate and one up tile per wave");
+  static_assert(KG % KS == 0 && KS == 8, "groups of a step over the K waves");
+  constexpr int NT = 64 * WN * KS;
+  constexpr int BM = 16 * TM, BW = 16 * TN * WN;  // tokens, weight rows of the tile
+  constexpr int OC = PAIR ? BW / 2 : BW;          // output columns
+  constexpr int XS = KG * 32 + 16, WS = KG * 16 + 16;  // LDS row strides of codes and nibbles (bytes)
+  constexpr int XC = BM * KG * 2, WC = BW * KG;        // a step's 16-byte pieces of x and of the nibbles
+  constexpr int NX = (XC + NT - 1) / NT, NW = (WC + NT - 1) / NT;
+  constexpr int NTL = TM * TN;                         // tiles of a wave
+  constexpr int NC = (NTL * 4 + KS - 1) / KS;          // (tile, register) chains per wave of the tile
+  __shared__ __align__(16) int8_t xs[2][BM * XS];
+  __shared__ __align__(16) uint8_t ws[2][BW * WS];
+  __shared__ float ss[2][KG * BW];  // [group][row]
+  __shared__ float rs[2][WN * KG * NTL * 256];
+  __shared__ uint64_t s_exp[PAIR ? 32 : 1];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int ks = wv % KS, wn = wv / KS;
+  const int r16 = lane & 15, b = lane >> 4;
+  const int tb = blockIdx.y * BM, ob = blockIdx.x * OC;
+  const int ng = I / 32, rb = I / 2, nstep = (ng + KG - 1) / KG;
+  if (PAIR) exp_tab_lds(s_exp);
+
+  // staging, two steps ahead: every load unconditional, from clamped piece
+  // numbers (the last piece stored more than once, the same bytes), rows past
+  // the end re-reading the last and groups past the end a row's first
+  struct Set {
+    v4i x[NX], w[NW];
+    float s[NW];
+  };
+  Set s0, s1;
+  auto piece = [&](int i, int n) { return n % NT == 0 || tid + i * NT < n ? tid + i * NT : n - 1; };
+  const int8_t* px[NX];
+  const uint8_t* pw[NW];
+  const float* ps[NW];
+#pragma unroll
+  for (int i = 0; i < NX; i++) {
+    const int c = piece(i, XC), row = c / (2 * KG), t = tb + row < M ? tb + row : M - 1;
+    px[i] = xq + (int64_t)t * I + c % (2 * KG) * 16;
+  }
+#pragma unroll
+  for (int i = 0; i < NW; i++) {
+    const int c = piece(i, WC), row = c / KG, k = c % KG;
+    const bool up = PAIR && row >= OC;
+    const int on = ob + (up ? row - OC : row);
+    const int64_t o = on < O ? on : O - 1;
+    pw[i] = (up ? q4b : q4) + o * rb + k * 16;
+    ps[i] = (up ? sclb : scl) + o * ng + k;
+  }
+  auto gload = [&](int st, Set& v) {
+    const int s = st < nstep ? st : nstep - 1, left = ng - s * KG;  // uniform
+#pragma unroll
+    for (int i = 0; i < NX; i++) {
+      const int k = piece(i, XC) % (2 * KG);
+      v.x[i] = *(const v4i*)(px[i] + (k / 2 < left ? s * (KG * 32) : -k * 16));
+    }
+#pragma unroll
+    for (int i = 0; i < NW; i++) {
+      const int k = piece(i, WC) % KG;
+      v.w[i] = *(const v4i*)(pw[i] + (k < left ? s * (KG * 16) : -k * 16));
+      v.s[i] = ps[i][k < left ? s * KG : -k];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto put = [&](int p, const Set& v) {
+#pragma unroll
+    for (int i = 0; i < NX; i++) {
+      const int c = piece(i, XC);
+      *(v4i*)(xs[p] + c / (2 * KG) * XS + c % (2 * KG) * 16) = v.x[i];
+    }
+#pragma unroll
+    for (int i = 0; i < NW; i++) {
+      const int c = piece(i, WC);
+      *(v4i*)(ws[p] + c / KG * WS + c % KG * 16) = v.w[i];
+      ss[p][c % KG * BW + c / KG] = v.s[i];
+    }
+  };
+
+  auto row_of = [&](int j) { return PAIR ? j * OC + wn * 16 + r16 : (wn * TN + j) * 16 + r16; };
+  float acc[NC], sc[NC][KG];
+#pragma unroll
+  for (int c = 0; c < NC; c++) acc[c] = 0.f;
+  // chain c of this wave: register and tile of index ks + KS c
+  auto chain = [&](int st) {
+    const int n = ng - st * KG < KG ? ng - st * KG : KG;
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      const int id = ks + KS * c;
+      if (id >= NTL * 4) break;  // wave-uniform
+      const float* rp = rs[st & 1] + wn * (KG * NTL * 256) + id * 64 + lane;
+      if (n == KG) {
+#pragma unroll
+        for (int k = 0; k < KG; k++) acc[c] = __fmaf_rn(sc[c][k], rp[k * NTL * 256], acc[c]);
+      } else {
+#pragma unroll
+        for (int k = 0; k < KG; k++)
+          if (k < n) acc[c] = __fmaf_rn(sc[c][k], rp[k * NTL * 256], acc[c]);
+      }
+    }
+  };
+  auto step = [&](int st, Set& v) {  // v: step st + 1's pieces; step st + 3's next
+    // step st is staged, the dots of step st - 1 are handed over, and every
+    // wave is done with the buffers of step st - 1
+    __syncthreads();
+    const int p = st & 1;
+    if (st > 0) chain(st - 1);
+    put(p ^ 1, v);
+    gload(st + 3, v);
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      const int id = ks + KS * c, row = row_of(id / 4 % NTL % TN);
+#pragma unroll
+      for (int k = 0; k < KG; k++) sc[c][k] = ss[p][k * BW + row];
+    }
+    // groups past the end are computed on the row's first and never chained
+    long fa[KG / KS][TM];
+    v4i d[KG / KS][TM][TN];
+#pragma unroll
+    for (int g = 0; g < KG / KS; g++) {
+      const int k = g * KS + ks;
+#pragma unroll
+      for (int i = 0; i < TM; i++) {
+        const uint2 c = *(const uint2*)(xs[p] + (i * 16 + r16) * XS + k * 32 + b * 8);
+        fa[g][i] = (long)((uint64_t)__builtin_amdgcn_perm(c.y, c.x, 0x06040200u) |
+                          ((uint64_t)__builtin_amdgcn_perm(c.y, c.x, 0x07050301u) << 32));
+      }
+#pragma unroll
+      for (int j = 0; j < TN; j++) {
+        const uint32_t w = *(const uint32_t*)(ws[p] + row_of(j) * WS + k * 16 + b * 4);
+        const long fb = (long)((uint64_t)nib_minus8(w & 0x0f0f0f0fu) | ((uint64_t)nib_minus8((w >> 4) & 0x0f0f0f0fu) << 32));
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+          d[g][i][j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(fa[g][i], fb, v4i{0, 0, 0, 0}, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < KG / KS; g++)
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            rs[p][((wn * KG + g * KS + ks) * NTL + i * TN + j) * 256 + r * 64 + lane] = (float)d[g][i][j][r];
+  };
+  gload(0, s0);
+  gload(1, s1);
+  put(0, s0);
+  gload(2, s0);
+  for (int st = 0; st < nstep; st += 2) {
+    step(st, s1);
+    if (st + 1 < nstep) step(st + 1, s0);
+  }
+  __syncthreads();
+  chain(nstep - 1);
+  __builtin_amdgcn_s_waitcnt(0);  // the clamped prefetches
+  if constexpr (PAIR) {
+    // gate and up chains of one output sit in different waves: through LDS
+    float* ex = rs[nstep & 1];  // the half the last chain did not read
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      const int id = ks + KS * c;
+      if (id < NTL * 4) ex[(wn * NTL * 4 + id) * 64 + lane] = acc[c];
+    }
+    __syncthreads();
+    for (int q = ks; q < TM * 4; q += KS) {  // (token tile, register)
+      const int i = q / 4, r = q % 4, t = tb + i * 16 + 4 * b + r, o = ob + wn * 16 + r16;
+      const float s = sx[t < M ? t : M - 1];
+      const float g = s * ex[(wn * NTL * 4 + (i * 2) * 4 + r) * 64 + lane];
+      const float u = s * ex[(wn * NTL * 4 + (i * 2 + 1) * 4 + r) * 64 + lane];
+      const float v = ref_silu_mul(g, u, s_exp);
+      if (t < M && o < O) y[(int64_t)t * O + o] = v;
+    }
+  } else {
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      const int id = ks + KS * c, tl = id / 4, r = id % 4;
+      if (id >= NTL * 4) break;
+      const int t = tb + tl / TN * 16 + 4 * b + r, o = ob + row_of(tl % TN);
+      if (t < M && o < O) y[(int64_t)t * O + o] = sx[t] * acc[c];
+    }
+  }
+}
+
+// M <= I4G_FEW_MAX tokens of activations from launch_qrow_i8.  Shapes from a
+// sweep on MI355X over (1, 2, 4) x 16 tokens, 16-32 columns and 8 or 16
+// groups a step, weights rotating past the Infinity Cache: gate + up of 4096
+// x 12288 25.7 us up to 16 tokens (16 groups a step 27.8, two column tiles
+// 33) and 42 up to 32; 12288 x 4096 16.5 (8 groups 29) and 22 (29).  The
+// GEMVs of 2-4 tokens took 72-96 us for the two, the f16-MFMA tiles 97.
+int launch_gemm_i4g_few(const int8_t* xq, const float* sx, const uint8_t* q4, const float* scl, const uint8_t* q4b,
+                        const float* sclb, float* y, int M, int I, int O, hipStream_t st) {
+  if (M > I4G_FEW_MAX || (I % 32)) return MOTY_EUNSUP;
+  if (M <= 0 || O <= 0) return MOTY_OK;
+  const dim3 grid((O + 15) / 16), blk(512);
+#define FEW(TM, TN, KG, P) \
+  hipLaunchKernelGGL((k_gemm_i4g_few<TM, TN, 1, 8, KG, P>), grid, blk, 0, st, xq, sx, q4, scl, q4b, sclb, y, M, I, O)
+  if (q4b) {
+    if (M <= 16) FEW(1, 2, 8, true);
+    else FEW(2, 2, 8, true);
+  } else {
+    if (M <= 16) FEW(1, 1, 16, false);
+    else FEW(2, 1, 16, false);
+  }
+#undef FEW
+  LAUNCH_TRY("k_gemm_i4g_few");
+  return MOTY_OK;
 }
 
 // The tile shapes, by the time one workgroup takes alone on a CU per 4096

@@ -284,6 +284,37 @@ def test_i4g_f32(ops, S, I, O):
 
 
 @pytest.mark.parametrize("S,I,O", [
+    # 2..32 tokens (one and two 16-token tiles), ragged rows, steps of 8 or 16
+    # groups that are short, full, and followed by a part
+    (2, 64, 33), (16, 512, 100), (16, 576, 47), (17, 64, 16), (32, 1088, 130), (31, 512, 1), (5, 4096, 70),
+    (3, 12288, 40), (33, 1088, 70)])
+def test_i4g_few_tokens(ops, S, I, O):
+    say("i4g few tokens", S, I, O)
+    q4, s = o_pack_int4_grouped(randn(O + I, (O, I), 0.02))
+    x = randn(S + 2 * I, (S, I))
+    x[S - 1] = 0.0
+    y = to_np(ops.matmul_i4_grouped_s(to_dev(x), to_dev(q4), to_dev(s), 32, True))
+    y2 = o_matmul_i4g(x, q4, s, True)
+    assert same_bits(y, y2), mismatch(y, y2)
+
+
+@pytest.mark.parametrize("S,D,I", [(2, 64, 192), (16, 512, 80 * 8), (17, 576, 64), (32, 1088, 448), (9, 4096, 128)])
+def test_dense_ffn_i4g_few_tokens(ops, S, D, I):
+    """The gate + up form, whose gate and up chains sit in different waves."""
+    say("dense_ffn_i4g few tokens", S, D, I)
+    gq, gs = o_pack_int4_grouped(randn(S + D, (I, D), 0.02))
+    uq, us = o_pack_int4_grouped(randn(S + D + 1, (I, D), 0.02))
+    dq, ds = o_pack_int4_grouped(randn(S + I, (D, I), 0.02))
+    x = randn(S + 3, (S, D))
+    y = to_np(ops.dense_ffn_i4g(to_dev(x), to_dev(gq), to_dev(gs), to_dev(uq), to_dev(us), to_dev(dq), to_dev(ds)))
+    g = o_matmul_i4g(x, gq, gs, True)
+    u = o_matmul_i4g(x, uq, us, True)
+    oracle().o_silu_mul(ptr(g), ptr(u), g.size)
+    y2 = o_matmul_i4g(g, dq, ds, True)
+    assert same_bits(y, y2), mismatch(y, y2)
+
+
+@pytest.mark.parametrize("S,I,O", [
     # every tile shape of the several-token GEMM (16 x 32, 16 x 64, 32 x 64,
     # 64 x 64 by the grid's size), ragged in tokens and rows; 1, 3 and 9
     # groups: less than a K step, one that is not full, several and a part
