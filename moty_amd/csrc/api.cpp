@@ -409,6 +409,29 @@ int moty_hip_matmul_q_s_dev(float* y, const float* x, const int8_t* q, const flo
   return launch_gemm_q8(xq, sx, q, scale, y, S, I, O, st);
 }
 
+// IDOT4 grouped int4, S > 1 tokens, K % 64 == 0, K <= 16384 (w2 non-null: gate
+// + up + SiLU in one pass): quantize the rows and run the kernel that is
+// faster here.  xq: S * K halves of scratch, sx: S floats.  MOTY_EUNSUP, with
+// nothing launched, where only the pair form is missing.
+static int i4g_idot_rows(const float* x, const uint8_t* w, const float* ws, const uint8_t* w2, const float* ws2,
+                         float* y, int S, int K, int N, void* xq, float* sx, hipStream_t st) {
+  const bool f16 = gemm_i4g_h_fits(S, K, N) &&
+                   !(((uintptr_t)x | (uintptr_t)w | (uintptr_t)ws | (uintptr_t)w2 | (uintptr_t)ws2) & 15);
+  int rc;
+  if (i4g_few_wins(S, K, N, w2 != nullptr, f16)) {
+    if ((rc = launch_qrow_i8(x, (int8_t*)xq, sx, nullptr, S, K, K, K, st))) return rc;
+    return launch_gemm_i4g_few((const int8_t*)xq, sx, w, ws, w2, ws2, y, S, K, N, st);
+  }
+  if (f16) {
+    // f16 codes + f16 MFMA: one FMA per output and group in the epilogue
+    if ((rc = launch_qrow_f16p(x, (uint16_t*)xq, sx, S, K, gemm_i4g_h_f8(S, N, w2 != nullptr), st))) return rc;
+    return launch_gemm_i4g_h((const uint16_t*)xq, sx, w, ws, w2, ws2, y, S, K, N, st);
+  }
+  if (w2) return MOTY_EUNSUP;
+  if ((rc = launch_qrow_i8(x, (int8_t*)xq, sx, nullptr, S, K, K, K, st))) return rc;
+  return launch_gemm_i4g((const int8_t*)xq, sx, w, ws, y, S, K, N, st);
+}
+
 int moty_hip_matmul_i4_grouped_s_dev(float* y, const float* x, const uint8_t* q4, const float* scale, int S,
                                      int I, int O, int gs, int idot4, void* stream) {
   CUR(d);
@@ -419,26 +442,11 @@ int moty_hip_matmul_i4_grouped_s_dev(float* y, const float* x, const uint8_t* q4
   if (idot4 && gs == 32 && (I % 64) == 0 && I <= 16384) {
     if (need_al16("matmul_i4_grouped_s", x, q4)) return MOTY_EUNSUP;
     if (S == 1) return launch_gemv_i4g(x, q4, scale, nullptr, nullptr, y, I, O, st);
+    const size_t bq = al256((size_t)S * I * 2);
     void* sp;
-    if (S > I4G_FEW_MAX && gemm_i4g_h_fits(S, I, O) && !(((uintptr_t)x | (uintptr_t)q4 | (uintptr_t)scale) & 15)) {
-      // f16 codes + f16 MFMA: one FMA per output and group in the epilogue
-      const size_t hb = al256((size_t)S * I * 2);
-      int rc = scratch_get(d, hb + al256((size_t)S * 4), st, &sp);
-      if (rc) return rc;
-      uint16_t* xh = (uint16_t*)sp;
-      float* sx = (float*)((char*)sp + hb);
-      if ((rc = launch_qrow_f16p(x, xh, sx, S, I, gemm_i4g_h_f8(S, O, false), st))) return rc;
-      return launch_gemm_i4g_h(xh, sx, q4, scale, nullptr, nullptr, y, S, I, O, st);
-    }
-    const size_t xb = al256((size_t)S * I);
-    int rc = scratch_get(d, xb + al256((size_t)S * 4), st, &sp);
+    int rc = scratch_get(d, bq + al256((size_t)S * 4), st, &sp);
     if (rc) return rc;
-    int8_t* xq = (int8_t*)sp;
-    float* sx = (float*)((char*)sp + xb);
-    rc = launch_qrow_i8(x, xq, sx, nullptr, S, I, I, I, st);
-    if (rc) return rc;
-    if (S <= I4G_FEW_MAX) return launch_gemm_i4g_few(xq, sx, q4, scale, nullptr, nullptr, y, S, I, O, st);
-    return launch_gemm_i4g(xq, sx, q4, scale, y, S, I, O, st);
+    return i4g_idot_rows(x, q4, scale, nullptr, nullptr, y, S, I, O, sp, (float*)((char*)sp + bq), st);
   }
   if (gs == 32 && xf_gemv_per_token(S, I, O, false)) {
     // a few tokens: the one-token GEMV per token (it refuses what it cannot
@@ -647,9 +655,6 @@ int moty_hip_dense_ffn_i4g_dev(float* out, const float* x, int S, const uint8_t*
   if (idot4 && need_al16("dense_ffn_i4g", x, gate, up, down)) return MOTY_EUNSUP;
   hipStream_t st = STREAM(stream);
   const bool vec = idot4 && (D % 64) == 0 && (I % 64) == 0 && D <= 16384 && I <= 16384;  // both matrices
-  const bool h16 = vec && S > I4G_FEW_MAX && gemm_i4g_h_fits(S, D, I) && gemm_i4g_h_fits(S, I, D) &&
-                   !(((uintptr_t)x | (uintptr_t)gate | (uintptr_t)gs | (uintptr_t)up | (uintptr_t)us |
-                      (uintptr_t)down | (uintptr_t)ds) & 15);
   const int W = D > I ? D : I;
   // scratch: h [S][I] f32 | u [S][I] f32 (paths without the fused pass) |
   // activation codes [S][W] (f16 or int8) | row scales [S]
@@ -661,32 +666,16 @@ int moty_hip_dense_ffn_i4g_dev(float* out, const float* x, int S, const uint8_t*
   float* u = (float*)((char*)sp + bh);
   void* xq = (char*)sp + 2 * bh;
   float* sx = (float*)((char*)sp + 2 * bh + bq);
-  if (h16) {
-    if ((rc = launch_qrow_f16p(x, (uint16_t*)xq, sx, S, D, gemm_i4g_h_f8(S, I, true), st))) return rc;
-    if ((rc = launch_gemm_i4g_h((const uint16_t*)xq, sx, gate, gs, up, us, h, S, D, I, st))) return rc;
-    if ((rc = launch_qrow_f16p(h, (uint16_t*)xq, sx, S, I, gemm_i4g_h_f8(S, D, false), st))) return rc;
-    return launch_gemm_i4g_h((const uint16_t*)xq, sx, down, ds, nullptr, nullptr, out, S, I, D, st);
-  }
   if (vec && S == 1) {
     if ((rc = launch_gemv_i4g(x, gate, gs, up, us, h, D, I, st))) return rc;
     return launch_gemv_i4g(h, down, ds, nullptr, nullptr, out, I, D, st);
-  }
-  if (vec && S <= I4G_FEW_MAX) {
-    int8_t* q = (int8_t*)xq;
-    if ((rc = launch_qrow_i8(x, q, sx, nullptr, S, D, D, D, st))) return rc;
-    if ((rc = launch_gemm_i4g_few(q, sx, gate, gs, up, us, h, S, D, I, st))) return rc;
-    if ((rc = launch_qrow_i8(h, q, sx, nullptr, S, I, I, I, st))) return rc;
-    return launch_gemm_i4g_few(q, sx, down, ds, nullptr, nullptr, out, S, I, D, st);
   }
   // one matmul_i4_grouped_s each, the path chosen per matrix as the
   // reference does (IDOT4 needs the row length a multiple of 64, <= 16384)
   auto mm = [&](const float* a, const uint8_t* w, const float* ws, float* o, int K, int N) -> int {
     if (idot4 && (K % 64) == 0 && K <= 16384) {
       if (S == 1) return launch_gemv_i4g(a, w, ws, nullptr, nullptr, o, K, N, st);
-      int r = launch_qrow_i8(a, (int8_t*)xq, sx, nullptr, S, K, K, K, st);
-      if (r) return r;
-      if (S <= I4G_FEW_MAX) return launch_gemm_i4g_few((const int8_t*)xq, sx, w, ws, nullptr, nullptr, o, S, K, N, st);
-      return launch_gemm_i4g((const int8_t*)xq, sx, w, ws, o, S, K, N, st);
+      return i4g_idot_rows(a, w, ws, nullptr, nullptr, o, S, K, N, xq, sx, st);
     }
     if (xf_gemv_per_token(S, K, N, false)) {
       // exact f32, a few tokens: the one-token GEMV per token (it refuses
@@ -712,6 +701,12 @@ int moty_hip_dense_ffn_i4g_dev(float* out, const float* x, int S, const uint8_t*
         rc = launch_gemv_i4g_xf(x + (int64_t)s * D, gate, gs, up, us, h + (int64_t)s * I, D, I, st);
     }
     if (rc == MOTY_EUNSUP && S > 1) rc = launch_gemm_i4g_xf(x, gate, gs, up, us, h, S, D, I, st);
+    if (rc == MOTY_OK) return mm(h, down, ds, out, I, D);
+    if (rc != MOTY_EUNSUP) return rc;
+  }
+  if (vec && S > 1) {
+    // gate + up + SiLU in one pass where a kernel has it, then down
+    rc = i4g_idot_rows(x, gate, gs, up, us, h, S, D, I, xq, sx, st);
     if (rc == MOTY_OK) return mm(h, down, ds, out, I, D);
     if (rc != MOTY_EUNSUP) return rc;
   }

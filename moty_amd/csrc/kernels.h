@@ -60,11 +60,13 @@ int launch_gemm_q8_pair(const int8_t* xq, const float* sx, const int8_t* W, cons
 // IDOT4, one token; q4b/sclb non-null: PAIR mode, y = silu(x.q4^T) * (x.q4b^T)
 int launch_gemv_i4g(const float* x, const uint8_t* q4, const float* scl, const uint8_t* q4b, const float* sclb,
                     float* y, int I, int O, hipStream_t st);
-// IDOT4, up to I4G_FEW_MAX tokens quantized by launch_qrow_i8 (PAIR alike);
-// I % 32 == 0, codes and nibbles 16-byte aligned
-constexpr int I4G_FEW_MAX = 32;
+// IDOT4, a few tokens quantized by launch_qrow_i8 (PAIR alike); I % 32 == 0,
+// codes and nibbles 16-byte aligned
 int launch_gemm_i4g_few(const int8_t* xq, const float* sx, const uint8_t* q4, const float* scl, const uint8_t* q4b,
                         const float* sclb, float* y, int M, int I, int O, hipStream_t st);
+// whether that kernel is the faster one, by measured times (f16: whether
+// launch_gemm_i4g_h would take the call otherwise)
+bool i4g_few_wins(int M, int I, int O, bool pair, bool f16);
 // the exact-f32 path (IDOT4 unset), several tokens; q4b/sclb non-null: PAIR
 int launch_gemm_i4g_xf(const float* x, const uint8_t* q4, const float* scl, const uint8_t* q4b, const float* sclb,
                        float* y, int M, int I, int O, hipStream_t st);

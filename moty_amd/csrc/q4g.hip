@@ -1446,25 +1446,51 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void k_gemm_i4g_few(const int8_t* 
   }
 }
 
-// M <= I4G_FEW_MAX tokens of activations from launch_qrow_i8.  Shapes from a
-// sweep on MI355X over (1, 2, 4) x 16 tokens, 16-32 columns and 8 or 16
-// groups a step, weights rotating past the Infinity Cache: gate + up of 4096
-// x 12288 25.7 us up to 16 tokens (16 groups a step 27.8, two column tiles
-// 33) and 42 up to 32; 12288 x 4096 16.5 (8 groups 29) and 22 (29).  The
-// GEMVs of 2-4 tokens took 72-96 us for the two, the f16-MFMA tiles 97.
+// Time of a launch, us, as u workgroups on the busiest CU (ceil(all / 256))
+// times a + b * groups, fitted on MI355X to sweeps over M = 2..100, six (I, O)
+// pairs, (1, 2, 4) x 16 tokens, 16-32 columns and 8 or 16 groups a step,
+// weights rotating past the Infinity Cache: gate + up of 4096 x 12288 25.7 us
+// up to 16 tokens (16 groups a step 27.8, two column tiles 33) and 42 up to
+// 32; 12288 x 4096 16.5 (8 groups 29) and 22 (29).
+static double few_us(int M, int I, int O, bool pair, bool* two) {
+  const double ng = I / 32;
+  const int64_t cols = (O + 15) / 16;
+  const double u1 = (double)((cols * ((M + 15) / 16) + 255) / 256), u2 = (double)((cols * ((M + 31) / 32) + 255) / 256);
+  const double t1 = pair ? u1 * (1.5 + 0.0405 * ng) : u1 * (0.5 + 0.029 * ng) + 1.7 + 0.008 * ng;
+  const double t2 = pair ? u2 * (1.5 + 0.100 * ng) : u2 * (0.7 + 0.050 * ng) + 1.5 + 0.006 * ng;
+  *two = t2 < t1;
+  return *two ? t2 : t1;
+}
+
+// The alternatives' times: the f16-MFMA tiles (64 tokens: a lone tile's K
+// loop, 42 us at 128 groups with SiLU, 57 at 384 without; at M = 128, two
+// tiles on a CU, 62), or, for other row lengths, one int8-MFMA GEMM each for
+// gate and up and silu_mul.
+bool i4g_few_wins(int M, int I, int O, bool pair, bool f16) {
+  if (M > 512) return false;
+  bool two;
+  const double ng = I / 32, few = few_us(M, I, O, pair, &two);
+  const double u = (double)(((int64_t)((M + 63) / 64) * ((O + 63) / 64) + 255) / 256);
+  const double other = f16 ? (pair ? 6.0 + 0.14 * ng + u * 0.14 * ng : 3.5 + 0.10 * ng + u * 0.04 * ng)
+                           : (pair ? 2 : 1) * (3.0 + 0.15 * ng + u * 0.09 * ng) + (pair ? 4 : 0);
+  return few < other;
+}
+
 int launch_gemm_i4g_few(const int8_t* xq, const float* sx, const uint8_t* q4, const float* scl, const uint8_t* q4b,
                         const float* sclb, float* y, int M, int I, int O, hipStream_t st) {
-  if (M > I4G_FEW_MAX || (I % 32)) return MOTY_EUNSUP;
+  if (I % 32) return MOTY_EUNSUP;
   if (M <= 0 || O <= 0) return MOTY_OK;
-  const dim3 grid((O + 15) / 16), blk(512);
+  bool two;
+  few_us(M, I, O, q4b != nullptr, &two);
+  const dim3 grid((O + 15) / 16, (M + (two ? 31 : 15)) / (two ? 32 : 16)), blk(512);
 #define FEW(TM, TN, KG, P) \
   hipLaunchKernelGGL((k_gemm_i4g_few<TM, TN, 1, 8, KG, P>), grid, blk, 0, st, xq, sx, q4, scl, q4b, sclb, y, M, I, O)
   if (q4b) {
-    if (M <= 16) FEW(1, 2, 8, true);
-    else FEW(2, 2, 8, true);
+    if (two) FEW(2, 2, 8, true);
+    else FEW(1, 2, 8, true);
   } else {
-    if (M <= 16) FEW(1, 1, 16, false);
-    else FEW(2, 1, 16, false);
+    if (two) FEW(2, 1, 16, false);
+    else FEW(1, 1, 16, false);
   }
 #undef FEW
   LAUNCH_TRY("k_gemm_i4g_few");

@@ -284,10 +284,10 @@ def test_i4g_f32(ops, S, I, O):
 
 
 @pytest.mark.parametrize("S,I,O", [
-    # 2..32 tokens (one and two 16-token tiles), ragged rows, steps of 8 or 16
-    # groups that are short, full, and followed by a part
+    # one and two 16-token tiles, several workgroups of tokens, ragged rows,
+    # steps of 8 or 16 groups that are short, full, and followed by a part
     (2, 64, 33), (16, 512, 100), (16, 576, 47), (17, 64, 16), (32, 1088, 130), (31, 512, 1), (5, 4096, 70),
-    (3, 12288, 40), (33, 1088, 70)])
+    (3, 12288, 40), (33, 1088, 70), (50, 3072, 1030), (97, 1024, 3075), (200, 576, 640)])
 def test_i4g_few_tokens(ops, S, I, O):
     say("i4g few tokens", S, I, O)
     q4, s = o_pack_int4_grouped(randn(O + I, (O, I), 0.02))
@@ -298,7 +298,8 @@ def test_i4g_few_tokens(ops, S, I, O):
     assert same_bits(y, y2), mismatch(y, y2)
 
 
-@pytest.mark.parametrize("S,D,I", [(2, 64, 192), (16, 512, 80 * 8), (17, 576, 64), (32, 1088, 448), (9, 4096, 128)])
+@pytest.mark.parametrize("S,D,I", [(2, 64, 192), (16, 512, 80 * 8), (17, 576, 64), (32, 1088, 448), (9, 4096, 128),
+                                   (70, 576, 3008), (130, 64, 128)])
 def test_dense_ffn_i4g_few_tokens(ops, S, D, I):
     """The gate + up form, whose gate and up chains sit in different waves."""
     say("dense_ffn_i4g few tokens", S, D, I)
