@@ -696,26 +696,268 @@ __global__ __launch_bounds__(64 * WR * WT, 2) void k_r4_gemm(const int8_t* __res
   }
 }
 
+// ---------------------------------------------------------------------------
+// The same for a few tokens: tiles of 16 TT tokens x 16 RT weight rows (PAIR:
+// RT = 2, gate and up rows of the same 16 columns) whose K steps of KG groups
+// are split over 8 waves by group.  Each wave forms its groups' integer dots
+// by one v_mfma_i32_16x16x32_i8 per tile and hands (float)(s + m8) over
+// through LDS, where a wave per register and tile continues the two-FMA
+// chains one step behind.  A step's barrier, LDS and load latencies (0.5-0.7
+// us, whatever it holds) bound k_r4_gemm's 4-group steps on grids this small.
+template <bool Q8, bool PAIR, int TT, int KG>
+__global__ __launch_bounds__(512, 2) void k_r4_few(const int8_t* __restrict__ xq, const float* __restrict__ xs,
+                                                   const int32_t* __restrict__ xm, const uint8_t* __restrict__ W,
+                                                   const uint16_t* __restrict__ d16, float* __restrict__ y, int S,
+                                                   int I, int O) {
+  constexpr int NT = 512, KS = 8, RT = PAIR ? 2 : 1;
+  constexpr int GB = Q8 ? 128 : 64, RB = Q8 ? 32 : 16;  // bytes of a block and group, of a row and group
+  constexpr int BT = 16 * TT, BR = 16 * RT;             // tokens, weight rows of the tile
+  constexpr int AS = KG * 32 + 16, BS = KG * RB + 16;   // LDS row strides of the codes (bytes)
+  constexpr int FS = KG + 4;                            // and of the per-group floats: 16 rows' float4s on 64 banks
+  constexpr int PB = KG * GB / 16;                      // a block's 16-byte pieces of a step
+  constexpr int AC = BT * KG * 2, BC = BR / 4 * PB, DC = BR / 4 * KG, TC = BT * KG;
+  constexpr int NA = (AC + NT - 1) / NT, NB = (BC + NT - 1) / NT, NTC = (TC + NT - 1) / NT;
+  constexpr int NTL = RT * TT;                // tiles
+  constexpr int NC = (NTL * 4 + KS - 1) / KS;  // (tile, register) chains per wave
+  static_assert(KG % KS == 0 && DC <= NT, "groups of a step over the K waves, one scale piece a thread");
+  __shared__ __align__(16) int8_t sA[2][BT * AS];
+  __shared__ __align__(16) uint8_t sB[2][BR * BS];
+  __shared__ __align__(16) float sD[2][BR * FS], sX[2][BT * FS], sC[2][Q8 ? 4 : BT * FS];  // [row or token][group]
+  __shared__ int sM[2][Q8 ? 4 : BT * FS];
+  __shared__ float rs[2][KG * NTL * 256];
+  __shared__ uint64_t s_exp[PAIR ? 32 : 1];
+  const int tid = threadIdx.x, lane = tid & 63, ks = tid >> 6;
+  const int rl = lane & 15, hk = lane >> 4;  // this lane's row / token of a tile, its K part
+  const int mb = blockIdx.y * BT, ob = blockIdx.x * 16;
+  const int nb = I / 32, S4 = S / 4 * 4, nstep = (nb + KG - 1) / KG;
+  const int O4 = ((PAIR ? 2 * O : O) + 3) / 4;
+  if (PAIR) exp_tab_lds(s_exp);
+
+  // staging, two steps ahead, every load unconditional as in k_r4_gemm: rows
+  // past the end re-read the last block or token, groups past the end group 0
+  auto blk = [&](int r4) {
+    const int row = 4 * r4, o = row >= 16 ? O + ob + row - 16 : ob + row;
+    return o / 4 < O4 ? o / 4 : O4 - 1;
+  };
+  struct Set {
+    v4i a[NA], b[NB];
+    u32x2_a2 d;
+    float x[NTC];
+    int m[NTC];
+  };
+  Set s0, s1;
+  auto piece = [&](int i, int n) { return n % NT == 0 || tid + i * NT < n ? tid + i * NT : n - 1; };
+  const int8_t* pa[NA];
+  const uint8_t* pb[NB];
+  uint32_t px[NTC];
+#pragma unroll
+  for (int i = 0; i < NA; i++) {
+    const int c = piece(i, AC), t = c / (2 * KG), m = mb + t < S ? mb + t : S - 1;
+    pa[i] = xq + (int64_t)m * I + c % (2 * KG) * 16;
+  }
+#pragma unroll
+  for (int i = 0; i < NB; i++) {
+    const int c = piece(i, BC);
+    pb[i] = W + (size_t)blk(c / PB) * nb * GB + c % PB * 16;
+  }
+  const uint16_t* pd = d16 + ((size_t)blk(piece(0, DC) / KG) * nb + piece(0, DC) % KG) * 4;
+#pragma unroll
+  for (int i = 0; i < NTC; i++) {
+    const int c = piece(i, TC), t = c / KG, m = mb + t < S ? mb + t : S - 1;
+    px[i] = (uint32_t)m * nb + c % KG;
+  }
+  auto gload = [&](int st, Set& v) {
+    const int s = st < nstep ? st : nstep - 1, left = nb - s * KG;  // uniform
+#pragma unroll
+    for (int i = 0; i < NA; i++) {
+      const int k = piece(i, AC) % (2 * KG);
+      v.a[i] = *(const v4i*)(pa[i] + (k / 2 < left ? s * (KG * 32) : -k * 16));
+    }
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+      const int q = piece(i, BC) % PB;
+      v.b[i] = *(const v4i*)(pb[i] + (q / (GB / 16) < left ? s * (KG * GB) : -q * 16));
+    }
+    {
+      const int k = piece(0, DC) % KG;
+      v.d = *(const u32x2_a2*)(pd + (k < left ? s * (KG * 4) : -k * 4));
+    }
+#pragma unroll
+    for (int i = 0; i < NTC; i++) {
+      const int k = piece(i, TC) % KG;
+      const uint32_t at = px[i] + (k < left ? s * KG : -k);
+      v.x[i] = xs[at];
+      if (!Q8) v.m[i] = xm[at];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto put = [&](int p, const Set& v) {
+#pragma unroll
+    for (int i = 0; i < NA; i++) {
+      const int c = piece(i, AC);
+      *(v4i*)(sA[p] + c / (2 * KG) * AS + c % (2 * KG) * 16) = v.a[i];
+    }
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+      constexpr int PR = RB / 16;
+      const int c = piece(i, BC), r4 = c / PB, q = c % PB, k = q / (GB / 16), h = q % (GB / 16);
+      *(v4i*)(sB[p] + (r4 * 4 + h / PR) * BS + k * RB + h % PR * 16) = v.b[i];
+    }
+    {
+      const int c = piece(0, DC), r4 = c / KG, k = c % KG;
+      const auto h = [](uint32_t u) { return (float)__builtin_bit_cast(_Float16, (uint16_t)u); };  // exact
+      float* o = sD[p] + r4 * 4 * FS + k;
+      o[0] = h(v.d.x & 0xffffu), o[FS] = h(v.d.x >> 16), o[2 * FS] = h(v.d.y & 0xffffu), o[3 * FS] = h(v.d.y >> 16);
+    }
+#pragma unroll
+    for (int i = 0; i < NTC; i++) {
+      const int c = piece(i, TC), t = c / KG, at = t * FS + c % KG;
+      sX[p][at] = v.x[i];
+      if (!Q8) {
+        const bool per_token = mb + t >= S4;
+        sC[p][at] = per_token ? 0.f : (8.f * (float)v.m[i]) * v.x[i];
+        sM[p][at] = per_token ? -8 * v.m[i] : 0;
+      }
+    }
+  };
+
+  // chain c of this wave: id = ks + 8 c, register id % 4 (row 4 hk + id % 4)
+  // of tile id / 4 (row tile id / 4 / TT, token tile id / 4 % TT)
+  float acc[NC], sc[NC][KG], nd[NC][KG], cv[NC][KG];
+#pragma unroll
+  for (int c = 0; c < NC; c++) acc[c] = 0.f;
+  auto chain = [&](int st) {
+    const int n = nb - st * KG < KG ? nb - st * KG : KG;
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      const int id = ks + KS * c;
+      if (id >= NTL * 4) break;  // wave-uniform
+      const float* rp = rs[st & 1] + id * 64 + lane;
+      auto link = [&](int k) {
+        acc[c] = __fmaf_rn(rp[k * NTL * 256], sc[c][k], acc[c]);
+        if (!Q8) acc[c] = __fmaf_rn(nd[c][k], cv[c][k], acc[c]);
+      };
+      if (n == KG) {
+#pragma unroll
+        for (int k = 0; k < KG; k++) link(k);
+      } else {
+#pragma unroll
+        for (int k = 0; k < KG; k++)
+          if (k < n) link(k);
+      }
+    }
+  };
+  auto step = [&](int st, Set& v) {  // v: step st + 1's pieces; step st + 3's next
+    // step st is staged, the dots of step st - 1 are handed over, and every
+    // wave is done with the buffers of step st - 1
+    __syncthreads();
+    const int p = st & 1;
+    if (st > 0) chain(st - 1);
+    put(p ^ 1, v);
+    gload(st + 3, v);
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      const int id = ks + KS * c, tl = id / 4 % NTL;
+      const float* dp = sD[p] + (tl / TT * 16 + 4 * hk + id % 4) * FS;
+      const int t = (tl % TT * 16 + rl) * FS;
+#pragma unroll
+      for (int k = 0; k < KG; k += 4) {
+        const float4 dv = *(const float4*)(dp + k), xv = *(const float4*)(sX[p] + t + k);
+        sc[c][k] = dv.x * xv.x, sc[c][k + 1] = dv.y * xv.y, sc[c][k + 2] = dv.z * xv.z, sc[c][k + 3] = dv.w * xv.w;
+        if (!Q8) {
+          const float4 cc = *(const float4*)(sC[p] + t + k);
+          nd[c][k] = -dv.x, nd[c][k + 1] = -dv.y, nd[c][k + 2] = -dv.z, nd[c][k + 3] = -dv.w;
+          cv[c][k] = cc.x, cv[c][k + 1] = cc.y, cv[c][k + 2] = cc.z, cv[c][k + 3] = cc.w;
+        }
+      }
+    }
+    // groups past the end are computed on the rows' first and never chained
+    v4i d[KG / KS][RT][TT];
+    int mv[KG / KS][TT];
+#pragma unroll
+    for (int g = 0; g < KG / KS; g++) {
+      const int k = g * KS + ks;
+      long fb[TT];
+#pragma unroll
+      for (int i = 0; i < TT; i++) {
+        fb[i] = *(const long*)(sA[p] + (i * 16 + rl) * AS + k * 32 + hk * 8);
+        mv[g][i] = Q8 ? 0 : sM[p][(i * 16 + rl) * FS + k];
+      }
+#pragma unroll
+      for (int j = 0; j < RT; j++) {
+        long fa;
+        const uint8_t* wp = sB[p] + (j * 16 + rl) * BS + k * RB;
+        if (Q8) {
+          fa = *(const long*)(wp + hk * 8);
+        } else {  // K part hk: codes 8 hk .. + 8, nibbles hk / 2 of bytes 8 (hk % 2) ..
+          const uint2 w = *(const uint2*)(wp + (hk & 1) * 8);
+          const int sh = (hk >> 1) * 4;
+          fa = (long)(((w.x >> sh) & 0x0f0f0f0fu) | ((uint64_t)((w.y >> sh) & 0x0f0f0f0fu) << 32));
+        }
+#pragma unroll
+        for (int i = 0; i < TT; i++)
+          d[g][j][i] = __builtin_amdgcn_mfma_i32_16x16x32_i8(fa, fb[i], v4i{0, 0, 0, 0}, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < KG / KS; g++)
+#pragma unroll
+      for (int j = 0; j < RT; j++)
+#pragma unroll
+        for (int i = 0; i < TT; i++)
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            rs[p][((g * KS + ks) * NTL + j * TT + i) * 256 + r * 64 + lane] = (float)(d[g][j][i][r] + mv[g][i]);
+  };
+  gload(0, s0);
+  gload(1, s1);
+  put(0, s0);
+  gload(2, s0);
+  for (int st = 0; st < nstep; st += 2) {
+    step(st, s1);
+    if (st + 1 < nstep) step(st + 1, s0);
+  }
+  __syncthreads();
+  chain(nstep - 1);
+  __builtin_amdgcn_s_waitcnt(0);  // the clamped prefetches
+  // the chains of a token's columns sit in different waves: through LDS, then
+  // a wave per token tile and register writes its outputs
+  float* ex = rs[nstep & 1];  // the half the last chain did not read
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+    const int id = ks + KS * c;
+    if (id < NTL * 4) ex[id * 64 + lane] = acc[c];
+  }
+  __syncthreads();
+  // 64 outputs at a time, 16 consecutive columns of 4 tokens
+  for (int q = ks; q < TT * 4; q += KS) {
+    const int t = q * 4 + hk, i = t / 16, o = rl;  // token and column of the tile
+    const int at = (i * 4 + o % 4) * 64 + o / 4 * 16 + t % 16;
+    float v = ex[at];
+    if constexpr (PAIR) v = ref_silu_mul(v, ex[TT * 256 + at], s_exp);
+    if (mb + t < S && ob + o < O) y[(int64_t)(mb + t) * O + ob + o] = v;
+  }
+}
+
 // Tile shapes of k_r4_gemm: tokens, output columns, and the time of a launch
 // as max(l0 + l1 * n, u * (e + f * n)) us for n steps of 4 groups and u =
 // ceil(tiles / 256) tiles on the busiest CU: a lone tile's step latency, and
 // the SIMDs' work.  Fitted on MI355X to M = 4..500 over (I, O) = (3072, 1024),
 // (9728, 2560), (12288, 4096) and, gate + up, (1024, 3072), (2560, 9728),
-// (4096, 12288).  Small tiles (16 x 16 MFMA) for few tokens: M = 4, 24576 x
-// 4096 36 us and 4096 x 12288 60 us; 64-token ones in 32 x 32 for many: M =
-// 301, 190 and 152 us against 246 and 195 in the former 64 x 64 tiles.
+// (4096, 12288).  Small tiles (16 x 16 MFMA) for tens of tokens; 64-token ones
+// in 32 x 32 for many: M = 301, 190 and 152 us against 246 and 195 in the
+// former 64 x 64 tiles.
 struct R4Tile {
   int bt, oc;
   double l0, l1, e, f;
 };
-static constexpr R4Tile R4_PAIR[2][3] = {{{16, 32, 3.0, 0.85, 1.2, 0.25}, {32, 64, 4.0, 2.0, 2.0, 0.69}, {64, 64, 4.0, 1.95, 4.0, 1.31}},
-                                         {{16, 32, 3.0, 0.75, 1.2, 0.25}, {32, 64, 4.0, 2.0, 2.0, 0.95}, {64, 64, 4.0, 1.75, 4.0, 1.10}}};
+static constexpr R4Tile R4_PAIR[2][3] = {{{16, 32, 1.5, 1.06, 1.2, 0.25}, {32, 64, 4.0, 2.0, 2.0, 0.69}, {64, 64, 4.0, 1.95, 4.0, 1.31}},
+                                         {{16, 32, 2.0, 0.92, 1.2, 0.25}, {32, 64, 4.0, 2.0, 2.0, 0.95}, {64, 64, 4.0, 1.75, 4.0, 1.10}}};
 static constexpr R4Tile R4_ONE[2][4] = {{{16, 32, 2.5, 0.60, 1.0, 0.16}, {32, 64, 4.0, 0.87, 2.0, 0.50}, {64, 64, 4.0, 1.22, 4.0, 0.80}, {64, 128, 4.0, 1.52, 6.0, 1.50}},
                                         {{16, 32, 2.5, 0.52, 1.0, 0.16}, {32, 64, 4.0, 0.72, 2.0, 0.46}, {64, 64, 4.0, 0.90, 4.0, 0.64}, {64, 128, 4.0, 1.15, 6.0, 1.28}}};
 template <int N>
-static int r4_pick(const R4Tile (&t)[N], int S, int I, int O) {
+static int r4_pick(const R4Tile (&t)[N], int S, int I, int O, double& bt) {
   int best = 0;
-  double bt = 0;
   for (int k = 0; k < N; k++) {
     const int64_t tiles = (int64_t)((S + t[k].bt - 1) / t[k].bt) * ((O + t[k].oc - 1) / t[k].oc);
     const double n = (I + 32 * R4M_KG - 1) / (32 * R4M_KG), u = (double)((tiles + 255) / 256);
@@ -723,6 +965,23 @@ static int r4_pick(const R4Tile (&t)[N], int S, int I, int O) {
     if (k == 0 || us < bt) best = k, bt = us;
   }
   return best;
+}
+
+// k_r4_few: the steps of its u workgroups on the busiest CU, fitted likewise
+// (S = 2..200, weights rotating past the Infinity Cache).  Q4R4, 12288 x 4096,
+// 16 / 64 tokens: 65 / 68 us by k_r4_gemm, 22.7 / 55 here; gate + up of 4096 x
+// 12288 36 -> 31.7 (8 groups a step 33.4; Q8R4 30.3, and 33.3 by 16), past 16
+// tokens 38 against 62.
+static double r4_few_us(bool q8, bool pair, int S, int I, int O, bool& two) {
+  const double ng = I / 32;
+  const int64_t cols = (O + 15) / 16;
+  const double u1 = (double)((cols * ((S + 15) / 16) + 255) / 256), u2 = (double)((cols * ((S + 31) / 32) + 255) / 256);
+  two = false;
+  if (pair) return 1.5 + u1 * (q8 ? 1.2 + 0.062 * ng : 1.3 + 0.068 * ng);
+  const double t1 = q8 ? 1.0 + 0.01 * ng + u1 * (1.0 + 0.040 * ng) : 0.9 + u1 * (1.0 + 0.0535 * ng);
+  const double t2 = 1.0 + u2 * (0.9 + (q8 ? 0.0625 : 0.0705) * ng);
+  two = t2 < t1;
+  return two ? t2 : t1;
 }
 
 // y [S][O] = R4 matmul of x [S][I]; xq/xs/xm: scratch for the activation
@@ -738,7 +997,24 @@ int launch_r4_matmul(bool q8, const float* x, const uint8_t* W, const uint16_t* 
   if (!xq || !xs || !xm) return MOTY_EINVAL;  // the GEMM path needs the activation scratch
   int rc = launch_quant_g32(x, xq, xs, xm, S, I, st);
   if (rc) return rc;
-  const int k = r4_pick(R4_ONE[q8], S, I, O);
+  double us;
+  bool two;
+  const int k = r4_pick(R4_ONE[q8], S, I, O, us);
+  if (r4_few_us(q8, false, S, I, O, two) < us) {
+    const dim3 grid((O + 15) / 16, two ? (S + 31) / 32 : (S + 15) / 16);
+#define R4F(Q, TT) \
+  hipLaunchKernelGGL((k_r4_few<Q, false, TT, 16>), grid, dim3(512), 0, st, xq, xs, xm, W, d16, y, S, I, O)
+    if (two) {
+      if (q8) R4F(true, 2);
+      else R4F(false, 2);
+    } else {
+      if (q8) R4F(true, 1);
+      else R4F(false, 1);
+    }
+#undef R4F
+    LAUNCH_TRY("k_r4_few");
+    return MOTY_OK;
+  }
   const R4Tile& t = R4_ONE[q8][k];
   const dim3 grid((O + t.oc - 1) / t.oc, (S + t.bt - 1) / t.bt);
 #define R4G(MT, TT, WR, WT)                                                                                      \
@@ -765,7 +1041,18 @@ int launch_r4_gate_up_gemm(bool q8, const float* x, const uint8_t* W, const uint
   if (S <= 0) return MOTY_OK;
   int rc = launch_quant_g32(x, xq, xs, xm, S, D, st);
   if (rc) return rc;
-  const int k = r4_pick(R4_PAIR[q8], S, D, I);
+  double us;
+  bool two;
+  const int k = r4_pick(R4_PAIR[q8], S, D, I, us);
+  if (r4_few_us(q8, true, S, D, I, two) < us) {
+    const dim3 grid((I + 15) / 16, (S + 15) / 16);
+    if (q8)
+      hipLaunchKernelGGL((k_r4_few<true, true, 1, 8>), grid, dim3(512), 0, st, xq, xs, xm, W, d16, h, S, D, I);
+    else
+      hipLaunchKernelGGL((k_r4_few<false, true, 1, 16>), grid, dim3(512), 0, st, xq, xs, xm, W, d16, h, S, D, I);
+    LAUNCH_TRY("k_r4_few<pair>");
+    return MOTY_OK;
+  }
   const R4Tile& t = R4_PAIR[q8][k];
   const dim3 grid((I + t.oc - 1) / t.oc, (S + t.bt - 1) / t.bt);
 #define R4P(MT, WR, WT)                                                                                          \

@@ -178,7 +178,10 @@ def test_dense_ffn_r4(ops, q8, S, D, I):
     # 128), ragged in rows and tokens (S % 4 != 0: both of the reference's
     # token forms, in one tile and in different ones), 1, 5 and 33 groups
     (31, 32, 5), (4099, 32, 130), (8201, 32, 70), (8201, 32, 301), (2050, 32, 503), (8201, 32, 701), (101, 1056, 70),
-    (4100, 160, 131), (36, 160, 64)])
+    (4100, 160, 131), (36, 160, 64), (4100, 288, 99),
+    # the few-token kernel's 16 and 32-token tiles: K steps of 16 groups that
+    # are full, short, and followed by a part
+    (100, 512, 5), (33, 544, 17), (40, 12288, 5), (36, 16640, 2), (1100, 3072, 50), (1093, 3104, 63)])
 def test_matmul_r4_tiles(ops, q8, O, I, S):
     say("matmul r4 tiles", q8, O, I, S)
     q, d = o_pack_r4(randn(O + I, (O, I), 0.02), q8)
@@ -189,7 +192,8 @@ def test_matmul_r4_tiles(ops, q8, O, I, S):
 
 
 @pytest.mark.parametrize("q8", [False, True])
-@pytest.mark.parametrize("S,D,I", [(5, 32, 96), (70, 32, 8224), (130, 32, 4128), (35, 32, 8224), (67, 288, 160)])
+@pytest.mark.parametrize("S,D,I", [(5, 32, 96), (70, 32, 8224), (130, 32, 4128), (35, 32, 8224), (67, 288, 160),
+                                   (40, 160, 8224), (16, 512, 96), (5, 544, 160), (33, 1056, 64)])
 def test_dense_ffn_r4_tiles(ops, q8, S, D, I):
     """The gate + up form of the same tiles against the plain matmul, SiLU
     and the plain matmul again."""
