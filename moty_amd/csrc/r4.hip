@@ -945,15 +945,16 @@ __global__ __launch_bounds__(512, 2) void k_r4_few(const int8_t* __restrict__ xq
 // the SIMDs' work.  Fitted on MI355X to M = 4..500 over (I, O) = (3072, 1024),
 // (9728, 2560), (12288, 4096) and, gate + up, (1024, 3072), (2560, 9728),
 // (4096, 12288).  Small tiles (16 x 16 MFMA) for tens of tokens; 64-token ones
-// in 32 x 32 for many: M = 301, 190 and 152 us against 246 and 195 in the
-// former 64 x 64 tiles.
+// in 32 x 32 for many; gate + up of 32 tokens in 16 x 16 too (M = 200, 2560 x
+// 9728: 95 us in 32 x 32, 90; M = 64, 4096 x 12288: 80 and 55).  M = 301: 190 and 152 us against 246
+// and 195 in the former 64 x 64 tiles.
 struct R4Tile {
   int bt, oc;
   double l0, l1, e, f;
 };
-static constexpr R4Tile R4_PAIR[2][3] = {{{16, 32, 1.5, 1.06, 1.2, 0.25}, {32, 64, 4.0, 2.0, 2.0, 0.69}, {64, 64, 4.0, 1.95, 4.0, 1.31}},
-                                         {{16, 32, 2.0, 0.92, 1.2, 0.25}, {32, 64, 4.0, 2.0, 2.0, 0.95}, {64, 64, 4.0, 1.75, 4.0, 1.10}}};
-static constexpr R4Tile R4_ONE[2][4] = {{{16, 32, 2.5, 0.60, 1.0, 0.16}, {32, 64, 4.0, 0.87, 2.0, 0.50}, {64, 64, 4.0, 1.22, 4.0, 0.80}, {64, 128, 4.0, 1.52, 6.0, 1.50}},
+static constexpr R4Tile R4_PAIR[2][3] = {{{16, 32, 1.5, 1.06, 1.2, 0.25}, {32, 64, 3.0, 1.25, 1.9, 0.80}, {64, 64, 4.0, 1.95, 4.0, 1.38}},
+                                         {{16, 32, 2.0, 0.92, 1.2, 0.25}, {32, 64, 3.0, 1.20, 1.9, 0.80}, {64, 64, 4.0, 1.75, 4.0, 1.15}}};
+static constexpr R4Tile R4_ONE[2][4] = {{{16, 32, 1.0, 0.70, 1.0, 0.178}, {32, 64, 4.0, 0.87, 2.0, 0.50}, {64, 64, 4.0, 1.12, 4.0, 0.72}, {64, 128, 4.0, 1.40, 6.0, 1.43}},
                                         {{16, 32, 2.5, 0.52, 1.0, 0.16}, {32, 64, 4.0, 0.72, 2.0, 0.46}, {64, 64, 4.0, 0.90, 4.0, 0.64}, {64, 128, 4.0, 1.15, 6.0, 1.28}}};
 template <int N>
 static int r4_pick(const R4Tile (&t)[N], int S, int I, int O, double& bt) {
@@ -1055,16 +1056,16 @@ int launch_r4_gate_up_gemm(bool q8, const float* x, const uint8_t* W, const uint
   }
   const R4Tile& t = R4_PAIR[q8][k];
   const dim3 grid((I + t.oc - 1) / t.oc, (S + t.bt - 1) / t.bt);
-#define R4P(MT, WR, WT)                                                                                          \
+#define R4P(MT, TT, WR, WT)                                                                                      \
   if (q8)                                                                                                        \
-    hipLaunchKernelGGL((k_r4_gemm<true, true, MT, 2, 1, WR, WT>), grid, dim3(64 * WR * WT), 0, st, xq, xs, xm,   \
+    hipLaunchKernelGGL((k_r4_gemm<true, true, MT, 2, TT, WR, WT>), grid, dim3(64 * WR * WT), 0, st, xq, xs, xm,  \
                        W, d16, h, S, D, I);                                                                      \
   else                                                                                                           \
-    hipLaunchKernelGGL((k_r4_gemm<false, true, MT, 2, 1, WR, WT>), grid, dim3(64 * WR * WT), 0, st, xq, xs, xm,  \
+    hipLaunchKernelGGL((k_r4_gemm<false, true, MT, 2, TT, WR, WT>), grid, dim3(64 * WR * WT), 0, st, xq, xs, xm, \
                        W, d16, h, S, D, I)
-  if (k == 0) { R4P(16, 2, 1); }
-  else if (k == 1) { R4P(32, 2, 1); }
-  else { R4P(32, 2, 2); }
+  if (k == 0) { R4P(16, 1, 2, 1); }
+  else if (k == 1) { R4P(16, 2, 4, 1); }
+  else { R4P(32, 1, 2, 2); }
 #undef R4P
   LAUNCH_TRY("k_r4_gemm<pair>");
   return MOTY_OK;

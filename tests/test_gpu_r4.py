@@ -193,7 +193,7 @@ def test_matmul_r4_tiles(ops, q8, O, I, S):
 
 @pytest.mark.parametrize("q8", [False, True])
 @pytest.mark.parametrize("S,D,I", [(5, 32, 96), (70, 32, 8224), (130, 32, 4128), (35, 32, 8224), (67, 288, 160),
-                                   (40, 160, 8224), (16, 512, 96), (5, 544, 160), (33, 1056, 64)])
+                                   (40, 160, 8224), (399, 160, 4128), (150, 544, 4128), (16, 512, 96), (5, 544, 160), (33, 1056, 64)])
 def test_dense_ffn_r4_tiles(ops, q8, S, D, I):
     """The gate + up form of the same tiles against the plain matmul, SiLU
     and the plain matmul again."""
