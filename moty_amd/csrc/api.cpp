@@ -441,7 +441,13 @@ int moty_hip_matmul_i4_grouped_s_dev(float* y, const float* x, const uint8_t* q4
   hipStream_t st = STREAM(stream);
   if (idot4 && gs == 32 && (I % 64) == 0 && I <= 16384) {
     if (need_al16("matmul_i4_grouped_s", x, q4)) return MOTY_EUNSUP;
-    if (S == 1) return launch_gemv_i4g(x, q4, scale, nullptr, nullptr, y, I, O, st);
+    // A captured call of 2..4 tokens runs the one-token GEMV, which quantizes
+    // in its workgroups: the graph then holds no address in the shared
+    // scratch, and its replays may overlap other calls.  (4 tokens, replayed,
+    // 3072 x 1024 then 1024 x 3072: 10.7 us, quantized into scratch 15.3;
+    // 12288 x 4096 and back 41.8 and 40.4.)
+    if (S == 1 || (S <= 4 && capturing(st)))
+      return launch_gemv_i4g(x, q4, scale, nullptr, nullptr, y, I, O, st, S);
     const size_t bq = al256((size_t)S * I * 2);
     void* sp;
     int rc = scratch_get(d, bq + al256((size_t)S * 4), st, &sp);

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from cpu_libs import o_dense_ffn_q8, o_moe, o_quantize_rows, o_route, randn
+from cpu_libs import o_dense_ffn_q8, o_matmul_i4g, o_moe, o_pack_int4_grouped, o_quantize_rows, o_route, randn
 from gpu_util import mismatch, same_bits, say, to_dev, to_np
 
 pytestmark = pytest.mark.gpu
@@ -267,3 +267,41 @@ def test_scratch_handed_between_streams_from_the_first_call(dev):
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     r = subprocess.run([sys.executable, "-c", _TWO_STREAMS.format(root=root)], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and "two streams ok" in r.stdout, r.stdout[-1000:] + r.stderr[-2000:]
+
+
+@pytest.mark.parametrize("S", [2, 3, 4])
+def test_captured_few_tokens_share_nothing(ops, S):
+    """IDOT4 grouped int4 of 2..4 tokens, captured: the graph holds no address
+    in the library's scratch, so its replays stay right after a larger call
+    has moved the scratch, and beside eager calls on another stream."""
+    import moty_amd
+    say("captured few tokens", S)
+    I, O = 1088, 1040
+    q4, s = o_pack_int4_grouped(randn(60, (O, I), 0.02))
+    qd, sd = to_dev(q4), to_dev(s)
+    xs = [randn(61 + k, (S, I)) for k in range(2)]
+    ref = [o_matmul_i4g(x, q4, s, True) for x in xs]
+    xd = [to_dev(x) for x in xs]
+    torch.cuda.synchronize()
+    assert moty_amd.lib().moty_hip_shutdown() == 0  # back to the scratch of a new process
+    y = ops.matmul_i4_grouped_s(xd[0], qd, sd, 32, True)
+    assert same_bits(to_np(y), ref[0])
+    g, side, other = torch.cuda.CUDAGraph(), torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.graph(g, stream=side):
+        ops.matmul_i4_grouped_s(xd[0], qd, sd, 32, True, out=y)
+    big = torch.randn((2048, I), device="cuda:0")
+    want = to_np(ops.matmul_i4_grouped_s(big, qd, sd, 32, True))  # a larger scratch
+    for rep in range(4):
+        y.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(other):
+            e = [ops.matmul_i4_grouped_s(xd[1], qd, sd, 32, True) for _ in range(8)]
+        for _ in range(8):
+            g.replay()
+        with torch.cuda.stream(other):
+            e += [ops.matmul_i4_grouped_s(xd[1], qd, sd, 32, True) for _ in range(8)]
+        torch.cuda.synchronize()
+        assert same_bits(to_np(y), ref[0]), "replay %d" % rep
+        for k, v in enumerate(e):
+            assert same_bits(to_np(v), ref[1]), "eager %d beside replay %d" % (k, rep)
+        assert same_bits(to_np(ops.matmul_i4_grouped_s(big, qd, sd, 32, True)), want)
