@@ -19,9 +19,10 @@
  * re-entrant from several host threads at once, like the reference's
  * process-static activation buffers (nn/matmul.c:55-58).  Sequential _dev
  * calls may use different streams: a call whose stream differs from the
- * previous scratch user's is ordered behind that stream's queued work.
- * Under HIP graph capture that ordering is not added: capture the calls of
- * one device on one stream.
+ * previous scratch user's is ordered behind that stream's queued work, on
+ * the device (a stream is told by its handle: let its calls finish before it
+ * is destroyed).  Under HIP graph capture that ordering is not added: capture
+ * the calls of one device on one stream.
  *
  * Numerics match the reference's x86-64 AVX512-VNNI build: int8 activations
  * and int32 accumulators bit-exact, float steps in the reference's order

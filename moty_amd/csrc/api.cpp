@@ -63,6 +63,7 @@ static int dev_init(int d) {
     HIP_TRY(hipGetSymbolAddress(&fp, HIP_SYMBOL(scratch)));
     g_dev[d].fixed_scratch = fp;
     HIP_TRY(hipEventCreateWithFlags(&g_dev[d].fx_ev, hipEventDisableTiming));
+    HIP_TRY(hipEventCreateWithFlags(&g_dev[d].scr_ev, hipEventDisableTiming));
     {
       // the one-launch FFN's exchange words (9 copies of I <= 4096 words),
       // per-workgroup call counters and wait-error flag, zeroed once
@@ -79,8 +80,8 @@ static int dev_init(int d) {
     }
     HIP_TRY(hipStreamCreateWithFlags(&g_dev[d].stream, hipStreamNonBlocking));
     {
-      // a first megabyte of scratch: calls of a few tokens (grouped int4 takes
-      // S * I bytes of codes) can then be captured without ever having run
+      // a first megabyte of scratch: small calls can then be captured without
+      // ever having run
       void* p = nullptr;
       const int rc = arena_get(g_dev[d].scratch, (size_t)1 << 20, &p);
       if (rc) return rc;
@@ -129,54 +130,63 @@ int arena_get(Arena& a, size_t bytes, void** p) {
 
 static bool capturing(hipStream_t st) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cs) != hipSuccess) {
+    (void)hipGetLastError();  // leave no error for a launch check to find
+    return false;
+  }
+  return cs != hipStreamCaptureStatusNone;
 }
 
-// The first time a second stream uses the arena: everything queued so far is
-// waited for once, and from then on each use records an event (scratch_mark).
-// In the relaxed capture mode, so that a capture the caller has open on some
-// other stream neither forbids the wait nor is broken by it.
-static int scratch_second_stream(Dev* d, hipStream_t st) {
+// Orders `st` behind the work of the scratch's previous stream where no event
+// marks that work yet (one stream used the arena until now): the event is
+// recorded there now, and the host waits for nothing.  Only where that stream
+// cannot take it (destroyed since, or under capture itself) the host waits for
+// the device, in the relaxed capture mode: an open capture neither forbids
+// that nor is broken by it.
+static int scratch_hand_over(Dev* d, hipStream_t st) {
+  if (!capturing(d->scr_stream) && hipEventRecord(d->scr_ev, d->scr_stream) == hipSuccess) {
+    HIP_TRY(hipStreamWaitEvent(st, d->scr_ev, 0));
+  } else {
+    (void)hipGetLastError();
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    const hipError_t e = hipDeviceSynchronize();
+    if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) return check_hip(e, "scratch hand-over between streams");
+  }
   d->scr_multi = true;
-  if (capturing(st) || d->scr_cap) return MOTY_OK;  // captured work is ordered by the caller
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-  const hipError_t e = hipDeviceSynchronize();
-  if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
-  return e == hipSuccess ? MOTY_OK : check_hip(e, "scratch hand-over between streams");
+  return MOTY_OK;
 }
 
 int scratch_get(Dev* d, size_t bytes, hipStream_t st, void** p) {
-  if (d->scr_used && d->scr_stream != st) {
-    if (!d->scr_multi) {
-      const int rc = scratch_second_stream(d, st);
-      if (rc) return rc;
-    } else if (d->scr_ev_ok && !capturing(st)) {
+  const bool cap = capturing(st);
+  if (!cap && d->scr_used && d->scr_stream != st) {
+    if (d->scr_ev_ok) {
       HIP_TRY(hipStreamWaitEvent(st, d->scr_ev, 0));
+      d->scr_multi = true;
+    } else {
+      const int rc = scratch_hand_over(d, st);
+      if (rc) return rc;
     }
   }
   int rc = arena_get(d->scratch, bytes, p);
-  if (rc) return rc;
+  if (rc || cap) return rc;
   d->scr_stream = st;
   d->scr_used = true;
   d->scr_pend = true;
+  d->scr_ev_ok = false;
   return MOTY_OK;
 }
 
 void scratch_mark(Dev* d) {
   d->scr_pend = false;
-  d->scr_ev_ok = false;
   // One stream so far: no event.  A program that keeps to one stream then
   // pays neither the record (about 3 us of a 14 us decode call) nor its
-  // barrier between the kernels of successive calls.
-  d->scr_cap = capturing(d->scr_stream);
-  if (d->scr_cap || !d->scr_multi) return;
-  if (!d->scr_ev && hipEventCreateWithFlags(&d->scr_ev, hipEventDisableTiming) != hipSuccess) {
-    d->scr_ev = nullptr;
-    return;
-  }
-  // a failed record leaves scr_ev_ok false: the next call on another stream
-  // then runs unordered, so synchronise here instead
+  // barrier between the kernels of successive calls.  (hipStreamPerThread
+  // names another stream in every thread: its work is marked here and now.)
+  if (!d->scr_multi && d->scr_stream != hipStreamPerThread) return;
+  // a failed record leaves nothing to order a call on another stream by, so
+  // synchronise here instead
   if (hipEventRecord(d->scr_ev, d->scr_stream) == hipSuccess)
     d->scr_ev_ok = true;
   else
@@ -284,7 +294,7 @@ int moty_hip_shutdown(void) {
     d.stream = nullptr;
     if (d.scr_ev) hipEventDestroy(d.scr_ev);
     d.scr_ev = nullptr;
-    d.scr_used = d.scr_pend = d.scr_ev_ok = d.scr_multi = d.scr_cap = false;
+    d.scr_used = d.scr_pend = d.scr_ev_ok = d.scr_multi = false;
     if (d.fx_ev) hipEventDestroy(d.fx_ev);
     d.fx_ev = nullptr;
     d.fx_used = d.fx_ev_ok = false;

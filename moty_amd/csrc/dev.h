@@ -25,15 +25,14 @@ struct Dev {
   int cus = 0;  // compute units
   hipStream_t stream = nullptr;
   Arena scratch, io;
-  // the stream whose queued work last used `scratch`; scr_multi: more than
-  // one stream has used it, and from then on an event recorded on the stream
-  // when a call returns (after its work was queued) orders a later call on
-  // another stream behind that work; scr_pend: a call took the arena and has
-  // not returned yet; scr_ev_ok: scr_ev marks the last use; scr_cap: the last
-  // use was under graph capture (and left no event)
+  // the stream whose queued work last used `scratch` (a use under graph
+  // capture is none: its replays are the caller's to order); scr_multi: more
+  // than one stream has used it, and from then on scr_ev is recorded on the
+  // stream when a call returns (after its work was queued); scr_pend: a call
+  // took the arena and has not returned yet; scr_ev_ok: scr_ev marks the last use
   hipStream_t scr_stream = nullptr;
-  bool scr_used = false, scr_pend = false, scr_ev_ok = false, scr_multi = false, scr_cap = false;
-  hipEvent_t scr_ev = nullptr;
+  bool scr_used = false, scr_pend = false, scr_ev_ok = false, scr_multi = false;
+  hipEvent_t scr_ev = nullptr;  // created at set-up
   // device address of this device's copy of the fixed no-allocation
   // scratch array (api.cpp), taken once at set-up, and the same ordering
   // state for it (event created at set-up)

@@ -269,6 +269,108 @@ def test_scratch_handed_between_streams_from_the_first_call(dev):
     assert r.returncode == 0 and "two streams ok" in r.stdout, r.stdout[-1000:] + r.stderr[-2000:]
 
 
+_HAND_OVER = r"""
+import ctypes
+import sys
+sys.path.insert(0, {root!r})
+import torch
+import moty_amd
+from moty_amd import ops
+lib = moty_amd.lib()
+def q8(O, K, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return (torch.randint(-128, 128, (O, K), generator=g, device="cuda", dtype=torch.int8),
+            torch.rand(O, generator=g, device="cuda") * 1e-4 + 1e-5)
+w = q8(3072, 1024, 1) + q8(3072, 1024, 2) + q8(1024, 3072, 3)
+xs = [torch.randn(7, 1024, device="cuda", generator=torch.Generator(device="cuda").manual_seed(k)) for k in range(3)]
+ys = [torch.empty(7, 1024, device="cuda") for _ in xs]
+a, b, c = (torch.cuda.Stream() for _ in range(3))
+def fresh():  # the library as in a new process, its kernels loaded
+    torch.cuda.synchronize()
+    assert lib.moty_hip_shutdown() == 0
+    assert lib.moty_hip_init(0) == 0
+    for y in ys:
+        y.zero_()
+    torch.cuda.synchronize()
+def call(st, k):
+    with torch.cuda.stream(st):
+        ops.dense_ffn_q8(xs[k], *w, out=ys[k])
+refs = [ops.dense_ffn_q8(x, *w) for x in xs]
+t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+for _ in range(2):  # clocks of a busy wait of 0.4 s
+    t0.record(); torch.cuda._sleep(10000000); t1.record(); t1.synchronize()
+clocks = int(10000000 * 400.0 / t0.elapsed_time(t1))
+def slow_then_call(st, k):
+    with torch.cuda.stream(st):
+        torch.cuda._sleep(clocks)
+    call(st, k)
+    e = torch.cuda.Event()
+    e.record(st)
+    return e
+def check(what, ks):
+    torch.cuda.synchronize()
+    for k in ks:
+        assert torch.equal(ys[k], refs[k]), (what, k)
+    print(what, "ok", flush=True)
+
+if {case!r} == "queued":
+    # the first call on a second stream waits on the device, not on the host
+    fresh()
+    e = slow_then_call(a, 0)
+    call(b, 1)
+    assert not e.query(), "the call waited for the device"
+    b.synchronize()
+    assert e.query(), "the second stream ran ahead of the first"
+    check("queued", (0, 1))
+elif {case!r} == "captured":
+    # a captured call in between does not hide the first stream's work
+    fresh()
+    e = slow_then_call(a, 0)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(c):
+        g.capture_begin(capture_error_mode="thread_local")
+        ops.dense_ffn_q8(xs[2], *w, out=ys[2])
+        g.capture_end()
+    call(b, 1)
+    assert not e.query(), "the call waited for the device"
+    b.synchronize()
+    assert e.query(), "the second stream ran ahead of the first"
+    for _ in range(3):
+        ys[2].zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(ys[2], refs[2])
+        call(b, 1)
+    check("captured", (0, 1, 2))
+else:
+    # the previous stream is gone when another one comes in
+    fresh()
+    path = [l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l][0]
+    hip = ctypes.CDLL(path)
+    h = ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(h)) == 0
+    s = torch.cuda.ExternalStream(h.value)
+    call(s, 0)
+    s.synchronize()
+    assert hip.hipStreamDestroy(h) == 0
+    call(b, 1)
+    check("destroyed", (0, 1))
+"""
+
+
+@pytest.mark.parametrize("case", ["queued", "captured", "destroyed"])
+def test_scratch_hand_over(dev, case):
+    """What the first call on a second stream waits for, and where."""
+    import os
+    import subprocess
+    import sys
+    say("scratch hand-over", case)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", _HAND_OVER.format(root=root, case=case)], capture_output=True, text=True,
+                       timeout=100)
+    assert r.returncode == 0 and case + " ok" in r.stdout, r.stdout[-1000:] + r.stderr[-2000:]
+
+
 @pytest.mark.parametrize("S", [2, 3, 4])
 def test_captured_few_tokens_share_nothing(ops, S):
     """IDOT4 grouped int4 of 2..4 tokens, captured: the graph holds no address
