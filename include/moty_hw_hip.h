@@ -22,7 +22,10 @@
  * previous scratch user's is ordered behind that stream's queued work, on
  * the device (a stream is told by its handle: let its calls finish before it
  * is destroyed).  Under HIP graph capture that ordering is not added: capture
- * the calls of one device on one stream.
+ * the calls of one device on one stream, and let no replay overlap other calls
+ * that use scratch.  Scratch that a captured call has used stays allocated
+ * until moty_hip_shutdown, so replays after later, larger calls are sound; no
+ * graph may be replayed after a shutdown.
  *
  * Numerics match the reference's x86-64 AVX512-VNNI build: int8 activations
  * and int32 accumulators bit-exact, float steps in the reference's order

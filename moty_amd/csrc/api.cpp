@@ -105,11 +105,13 @@ int cur(Dev** out) {
 }
 
 // Grow an arena to at least `bytes`.  Waits for queued work that may still
-// read the old buffer before releasing it.
+// read the old buffer before releasing it.  A buffer that a captured graph
+// holds addresses in is kept instead: each growth is by a quarter at least, so
+// all kept ones together are under four times the present one.
 int arena_get(Arena& a, size_t bytes, void** p) {
   if (bytes == 0) bytes = 256;
   if (a.cap < bytes) {
-    if (a.p) {
+    if (a.p && !a.captured) {
       HIP_TRY(hipDeviceSynchronize());
       HIP_TRY(hipFree(a.p));
       a.p = nullptr;
@@ -117,15 +119,22 @@ int arena_get(Arena& a, size_t bytes, void** p) {
     }
     size_t nb = bytes + bytes / 4;
     nb = (nb + (1 << 20) - 1) & ~(size_t)((1 << 20) - 1);
-    hipError_t e = hipMalloc(&a.p, nb);
-    if (e != hipSuccess) {
-      a.p = nullptr;
-      return check_hip(e, "scratch hipMalloc");
-    }
+    void* np = nullptr;
+    const hipError_t e = hipMalloc(&np, nb);
+    if (e != hipSuccess) return check_hip(e, "scratch hipMalloc");
+    if (a.p) a.kept.push_back(a.p);
+    a.p = np;
     a.cap = nb;
+    a.captured = false;
   }
   *p = a.p;
   return MOTY_OK;
+}
+
+static void arena_free(Arena& a) {
+  if (a.p) hipFree(a.p);
+  for (void* q : a.kept) hipFree(q);
+  a = Arena();
 }
 
 static bool capturing(hipStream_t st) {
@@ -170,6 +179,7 @@ int scratch_get(Dev* d, size_t bytes, hipStream_t st, void** p) {
     }
   }
   int rc = arena_get(d->scratch, bytes, p);
+  if (rc == MOTY_OK && cap) d->scratch.captured = true;
   if (rc || cap) return rc;
   d->scr_stream = st;
   d->scr_used = true;
@@ -286,10 +296,8 @@ int moty_hip_shutdown(void) {
     HIP_TRY(hipDeviceSynchronize());
     for (auto& kv : d.wcache) hipFree(kv.second.dev);
     d.wcache.clear();
-    if (d.scratch.p) hipFree(d.scratch.p);
-    if (d.io.p) hipFree(d.io.p);
-    d.scratch = Arena();
-    d.io = Arena();
+    arena_free(d.scratch);
+    arena_free(d.io);
     hipStreamDestroy(d.stream);
     d.stream = nullptr;
     if (d.scr_ev) hipEventDestroy(d.scr_ev);

@@ -6,6 +6,7 @@
 #include <stddef.h>
 
 #include <unordered_map>
+#include <vector>
 
 namespace moty {
 
@@ -18,6 +19,8 @@ struct WEntry {
 struct Arena {
   void* p = nullptr;
   size_t cap = 0;
+  bool captured = false;    // a graph holds addresses in p
+  std::vector<void*> kept;  // outgrown blocks that graphs hold addresses in, until shutdown
 };
 
 struct Dev {
@@ -52,7 +55,8 @@ struct Dev {
 
 // The calling thread's device (device 0 on first use), made current.
 int cur(Dev** out);
-// Grow an arena to at least `bytes`; waits for queued work before freeing.
+// Grow an arena to at least `bytes`; waits for queued work before freeing, and
+// frees no block that work under graph capture has used.
 int arena_get(Arena& a, size_t bytes, void** p);
 // The device's scratch arena for work about to be queued on `st`: when the
 // previous user queued on another stream, `st` first waits for that work

@@ -407,3 +407,38 @@ def test_captured_few_tokens_share_nothing(ops, S):
         for k, v in enumerate(e):
             assert same_bits(to_np(v), ref[1]), "eager %d beside replay %d" % (k, rep)
         assert same_bits(to_np(ops.matmul_i4_grouped_s(big, qd, sd, 32, True)), want)
+
+
+def test_captured_scratch_outlives_growth(ops):
+    """Replays after larger calls have moved the scratch, twice: its block is
+    kept for the graph that holds it."""
+    import moty_amd
+    say("captured scratch, growth")
+    D, I = 512, 640
+    w = [to_dev(a) for a in (*q8(1, (I, D)), *q8(2, (I, D)), *q8(3, (D, I)))]
+    xs = [to_dev(randn(70 + S, (S, D))) for S in (40, 200, 3000, 9000)]  # 9000: past the first megabyte many times
+    refs = [to_np(ops.dense_ffn_q8(x, *w)) for x in xs]
+    torch.cuda.synchronize()
+    assert moty_amd.lib().moty_hip_shutdown() == 0  # back to the scratch of a new process
+    ys = [torch.zeros_like(x) for x in xs]
+    side, graphs = torch.cuda.Stream(), []
+    for k in (0, 1):
+        ops.dense_ffn_q8(xs[k], *w, out=ys[k])
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=side):
+            ops.dense_ffn_q8(xs[k], *w, out=ys[k])
+        graphs.append((k, g))
+        ops.dense_ffn_q8(xs[k + 2], *w, out=ys[k + 2])  # the scratch grows
+        assert same_bits(to_np(ys[k + 2]), refs[k + 2])
+    for rep in range(3):
+        fill = [torch.full((1 << 20,), float("nan"), device="cuda:0") for _ in range(64)]  # takes freed memory
+        for k, g in graphs:
+            ys[k].zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert same_bits(to_np(ys[k]), refs[k]), (rep, k)
+        assert all(bool(f.isnan().all()) for f in fill)
+        ops.dense_ffn_q8(xs[2], *w, out=ys[2])
+        assert same_bits(to_np(ys[2]), refs[2])
+        del fill
