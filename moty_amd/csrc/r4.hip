@@ -431,7 +431,6 @@ __global__ __launch_bounds__(64 * WR * WT, 2) void k_r4_gemm(const int8_t* __res
   constexpr int BT = MT * TT * WT, BR = MT * RT * WR;   // tokens, weight rows of the tile
   constexpr int OC = PAIR ? BR / 2 : BR;                // output columns
   constexpr int BS = R4M_KG * RB + 16;                  // LDS row stride of the weight codes (bytes)
-  constexpr int NQ = MT / 8;                            // float4s of rows per lane: 4 (MT 32) or 2
   constexpr int ND = MT == 32 ? 16 : 4;                 // registers of a tile
   constexpr int AC = BT * R4M_KG * 2, BC = BR * R4M_KG * (RB / 16), DC = BR / 4 * R4M_KG, TC = BT * R4M_KG;
   constexpr int NA = (AC + NT - 1) / NT, NB = (BC + NT - 1) / NT, NDC = (DC + NT - 1) / NT, NTC = (TC + NT - 1) / NT;
@@ -451,7 +450,8 @@ __global__ __launch_bounds__(64 * WR * WT, 2) void k_r4_gemm(const int8_t* __res
   if (PAIR) exp_tab_lds(s_exp);
 
   // staging.  Rows past the end re-read the last block or token; groups past
-  // the end group 0 (their scales and codes are zeroed when staged).
+  // the end hold the row's first group and are never chained (compute takes a
+  // short step's groups one by one).
   auto blk = [&](int r4) {  // global 4-row block of tile row 4 * r4
     const int row = 4 * r4, o = PAIR && row >= OC ? O + ob + row - OC : ob + row;
     return o / 4 < O4 ? o / 4 : O4 - 1;
@@ -939,51 +939,298 @@ __global__ __launch_bounds__(512, 2) void k_r4_few(const int8_t* __restrict__ xq
   }
 }
 
-// Tile shapes of k_r4_gemm: tokens, output columns, and the time of a launch
-// as max(l0 + l1 * n, u * (e + f * n)) us for n steps of 4 groups and u =
-// ceil(tiles / 256) tiles on the busiest CU: a lone tile's step latency, and
-// the SIMDs' work.  Fitted on MI355X to M = 4..500 over (I, O) = (3072, 1024),
-// (9728, 2560), (12288, 4096) and, gate + up, (1024, 3072), (2560, 9728),
-// (4096, 12288).  Small tiles (16 x 16 MFMA) for tens of tokens; 64-token ones
-// in 32 x 32 for many; gate + up of 32 tokens in 16 x 16 too (M = 200, 2560 x
-// 9728: 95 us in 32 x 32, 90; M = 64, 4096 x 12288: 80 and 55).  M = 301: 190 and 152 us against 246
-// and 195 in the former 64 x 64 tiles.
+// Q4R4 with the operands the other way round: the tokens are the MFMA's rows
+// and the weights its columns, a lane holding one weight row's dd and reading
+// the xs, xct and m8 of its 16 (4) tokens per group.  Block tile 64 tokens x 64
+// weight rows, K steps of 4 groups single-buffered in LDS with two more in
+// registers.  Slower per output than k_r4_gemm on full grids, but its small LDS
+// and register shares hold more waves on a CU, so it is the faster one where
+// k_r4_gemm's tiles leave CUs idle or a last round nearly empty (4096 x 12288,
+// 256 tokens: 94.8 us against 99.9 in any of k_r4_gemm's tiles; 10240 x 1024,
+// 400 tokens: 34.2 and 39.0).
+// WV = 4: waves of 32 x 32.  WV = 16, for at most one workgroup per CU: waves
+// of 16 x 16, the first four stage (4096 x 12288, 256 tokens: 92.7 us against
+// 132 with four).  PAIR (WV = 4): 32 gate rows and the same up rows, y [S][O] =
+// silu(gate) * up, the up waves handing their sums over through LDS.
+constexpr int R4T_NT = 256;  // staging threads
+
+template <int WV, bool PAIR>
+__global__ __launch_bounds__(64 * WV, WV <= 8 ? 8 / WV : 1) void k_r4_gemm_tok(const int8_t* __restrict__ xq,
+                                                                               const float* __restrict__ xs,
+                                                                               const int32_t* __restrict__ xm,
+                                                                               const uint8_t* __restrict__ W,
+                                                                               const uint16_t* __restrict__ d16,
+                                                                               float* __restrict__ y, int S, int I,
+                                                                               int O) {
+  static_assert(WV == 16 ? !PAIR : WV == 4, "waves");
+  constexpr int GB = 64, RB = 16;       // bytes of a block and group, of a row and group
+  constexpr int BS = R4M_KG * RB + 16;  // LDS row stride of the weight codes
+  __shared__ __align__(16) int8_t sA[64 * R4M_AS];
+  __shared__ __align__(16) uint8_t sB[64 * BS];
+  __shared__ float sD[64 * R4M_KG];                                 // [row][group]
+  __shared__ __align__(16) float sX[R4M_KG * 64], sC[R4M_KG * 64];  // [group][token]
+  __shared__ __align__(16) int sM[R4M_KG * 64];
+  const int tid = threadIdx.x, lane = tid % MOTY_WAVE, wv = tid / MOTY_WAVE;
+  const int mb = blockIdx.y * 64, nb0 = blockIdx.x * (PAIR ? 32 : 64);
+  const int nb = I / 32, S4 = S / 4 * 4;
+  const bool tile = mb + 64 <= S4 || S == S4;  // no per-token tokens here: m8 is 0 throughout
+  const int O4 = ((PAIR ? 2 * O : O) + 3) / 4;
+
+  // staging: thread -> two 16-byte chunks of the tokens' codes, 16 bytes and
+  // one scale of weight row tid / 4, group tid % 4, the scales of token
+  // tid % 64, group tid / 64.  Rows past the end re-read the last; groups past
+  // the end re-read others and are never chained.
+  const int8_t* srcA[2];
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const int q = tid + i * R4T_NT, m = mb + (q >> 3) < S ? mb + (q >> 3) : S - 1;
+    srcA[i] = xq + (int64_t)m * I + (q & 7) * 16;
+  }
+  const int trow = tid >> 2;
+  const int orow = !PAIR ? nb0 + trow : trow < 32 ? nb0 + trow : O + nb0 + trow - 32;
+  const int ob = orow / 4 < O4 ? orow / 4 : O4 - 1;
+  const uint8_t* srcB = W + (size_t)ob * nb * GB + (size_t)(orow & 3) * RB;
+  const uint16_t* srcD = d16 + (size_t)ob * nb * 4 + (orow & 3);
+  const int st_g = (tid >> 6) & 3, st_t = mb + (tid & 63) < S ? mb + (tid & 63) : S - 1;
+  struct Set {
+    v4i a[2], b;
+    uint32_t d;
+    float x;
+    int m;
+  };
+  Set s0, s1;
+  const bool stager = WV == 4 || tid < R4T_NT;  // wave-uniform
+  const int glast = (nb - 1) / R4M_KG * R4M_KG;
+  auto gload = [&](int g0, Set& v) {
+    if (!stager) return;
+    const int gc = g0 < nb ? g0 : glast;
+    const int kb = gc * 32;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const int k = ((tid + i * R4T_NT) & 7) * 16;
+      v.a[i] = *(const v4i*)(srcA[i] + (kb + k < I ? kb : -k));
+    }
+    const int g = gc + (tid & 3) < nb ? gc + (tid & 3) : 0;
+    v.b = *(const v4i*)(srcB + (size_t)g * GB);
+    v.d = srcD[(size_t)g * 4];
+    const int gt = gc + st_g < nb ? gc + st_g : 0;
+    v.x = xs[(size_t)st_t * nb + gt];
+    v.m = xm[(size_t)st_t * nb + gt];
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  float acc[WV == 16 ? 4 : 16];
+#pragma unroll
+  for (float& v : acc) v = 0.f;
+  auto compute = [&](int ngk, auto tl) {
+    constexpr bool TILE = decltype(tl)::value;
+#pragma unroll
+    for (int gg = 0; gg < R4M_KG; gg++) {
+      if (gg >= ngk) break;  // wave-uniform
+      if constexpr (WV == 16) {
+        // tokens wm * 16 + [0, 16) x rows wn * 16 + [0, 16)
+        const int wm = wv / 4, row = wv % 4 * 16 + (lane & 15), q4 = lane >> 4;
+        const long a = *(const long*)(sA + (wm * 16 + (lane & 15)) * R4M_AS + gg * 32 + q4 * 8);
+        const int t = gg * 64 + wm * 16 + 4 * q4;  // this lane's 4 tokens
+        const float4 xv = *(const float4*)(sX + t), cv = *(const float4*)(sC + t);
+        const int4 mv = TILE ? int4{0, 0, 0, 0} : *(const int4*)(sM + t);
+        // codes 8 q4 .. + 8: nibbles q4 / 2 of bytes 8 (q4 % 2) ..
+        const uint2 w = *(const uint2*)(sB + row * BS + gg * RB + (q4 & 1) * 8);
+        const int sh = (q4 >> 1) * 4;
+        const long b = (long)(((w.x >> sh) & 0x0f0f0f0fu) | ((uint64_t)((w.y >> sh) & 0x0f0f0f0fu) << 32));
+        const v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, v4i{0, 0, 0, 0}, 0, 0, 0);
+        const float dd = sD[row * R4M_KG + gg];
+        acc[0] = __fmaf_rn(-dd, cv.x, __fmaf_rn((float)(d[0] + mv.x), dd * xv.x, acc[0]));
+        acc[1] = __fmaf_rn(-dd, cv.y, __fmaf_rn((float)(d[1] + mv.y), dd * xv.y, acc[1]));
+        acc[2] = __fmaf_rn(-dd, cv.z, __fmaf_rn((float)(d[2] + mv.z), dd * xv.z, acc[2]));
+        acc[3] = __fmaf_rn(-dd, cv.w, __fmaf_rn((float)(d[3] + mv.w), dd * xv.w, acc[3]));
+      } else {
+        const int wm = wv >> 1, row = (wv & 1) * 32 + (lane & 31), hk = lane >> 5;
+        const v4i a = *(const v4i*)(sA + (wm * 32 + (lane & 31)) * R4M_AS + gg * 32 + hk * 16);
+        v4i w = *(const v4i*)(sB + row * BS + gg * RB);
+#pragma unroll
+        for (int q = 0; q < 4; q++) w[q] = (w[q] >> (4 * hk)) & 0x0f0f0f0f;  // low nibbles for hk = 0, high for 1
+        const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, w, v16i{}, 0, 0, 0);
+        const float dd = sD[row * R4M_KG + gg];
+        // register r: token 8 (r / 4) + 4 hk + r % 4
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const int t = gg * 64 + wm * 32 + 8 * q + 4 * hk;
+          const float4 xv = *(const float4*)(sX + t), cv = *(const float4*)(sC + t);
+          const int4 mv = TILE ? int4{0, 0, 0, 0} : *(const int4*)(sM + t);
+          acc[4 * q] = __fmaf_rn(-dd, cv.x, __fmaf_rn((float)(d[4 * q] + mv.x), dd * xv.x, acc[4 * q]));
+          acc[4 * q + 1] = __fmaf_rn(-dd, cv.y, __fmaf_rn((float)(d[4 * q + 1] + mv.y), dd * xv.y, acc[4 * q + 1]));
+          acc[4 * q + 2] = __fmaf_rn(-dd, cv.z, __fmaf_rn((float)(d[4 * q + 2] + mv.z), dd * xv.z, acc[4 * q + 2]));
+          acc[4 * q + 3] = __fmaf_rn(-dd, cv.w, __fmaf_rn((float)(d[4 * q + 3] + mv.w), dd * xv.w, acc[4 * q + 3]));
+        }
+      }
+    }
+  };
+  auto stage = [&](int g0, Set& v) {
+    if (stager) {
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        const int q = tid + i * R4T_NT;
+        *(v4i*)(sA + (q >> 3) * R4M_AS + (q & 7) * 16) = v.a[i];
+      }
+      *(v4i*)(sB + trow * BS + (tid & 3) * RB) = v.b;
+      sD[trow * R4M_KG + (tid & 3)] = f16_to_f32(v.d);
+      sX[st_g * 64 + (tid & 63)] = v.x;
+      const bool per_token = mb + (tid & 63) >= S4;
+      sC[st_g * 64 + (tid & 63)] = per_token ? 0.f : (8.f * (float)v.m) * v.x;
+      sM[st_g * 64 + (tid & 63)] = per_token ? -8 * v.m : 0;
+    }
+    __syncthreads();
+    gload(g0 + 2 * R4M_KG, v);
+    const int ngk = nb - g0 < R4M_KG ? nb - g0 : R4M_KG;
+    if (tile) compute(ngk, std::true_type{});  // workgroup-uniform
+    else compute(ngk, std::false_type{});
+    __syncthreads();
+  };
+  gload(0, s0);
+  gload(R4M_KG, s1);
+  for (int g0 = 0; g0 < nb; g0 += 2 * R4M_KG) {
+    stage(g0, s0);
+    stage(g0 + R4M_KG, s1);
+  }
+  // retire the clamped prefetches once before the conditional stores
+  __builtin_amdgcn_s_waitcnt(0);
+  if constexpr (WV == 16) {
+    const int col = nb0 + wv % 4 * 16 + (lane & 15);
+    if (col >= O) return;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int t = mb + wv / 4 * 16 + 4 * (lane >> 4) + r;
+      if (t < S) y[(int64_t)t * O + col] = acc[r];
+    }
+  } else {
+    const int wm = wv >> 1, wn = wv & 1, hk = lane >> 5;
+    float* xch = (float*)sA;  // up sums, [r][wm][lane]
+    if constexpr (PAIR) {
+      if (wn == 1) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) xch[r * 128 + wm * 64 + lane] = acc[r];
+      }
+      __syncthreads();
+    }
+    const int col = nb0 + (PAIR ? 0 : wn * 32) + (lane & 31);
+    if ((PAIR && wn == 1) || col >= O) return;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const int t = mb + wm * 32 + 8 * (r >> 2) + 4 * hk + (r & 3);
+      float v = acc[r];
+      if constexpr (PAIR) v = ref_silu_mul(v, xch[r * 128 + wm * 64 + lane]);
+      if (t < S) y[(int64_t)t * O + col] = v;
+    }
+  }
+}
+
+// The kernels' tile shapes and times: a launch of j tiles on the busiest CU
+// (ceil(tiles / 256)) and n steps of 4 groups takes a + b * j + n * g[j] us,
+// past eight tiles n * g[8] * j / 8.  The tiles on a CU share its SIMDs, so g
+// is no multiple of j: two small tiles cost hardly more than one, and odd
+// numbers of 64 x 64 tiles waste a slot.  Fitted on MI355X to 240 to 304
+// points each: S = 4..4096 over the FFNs' gate + up (1024 x 3072 to 4096 x
+// 14336) and down, 1024 x 10240 and 4096 x 4096, weights rotating past the
+// Infinity Cache; off by 2 to 4 % (root mean square).  Where each wins: the
+// few-token kernel to about 64 tokens, 16 x 32 tiles (MFMA 16 x 16) to a few
+// hundred on narrow matrices, large tiles where several rounds of them fill
+// the chip, and for Q4R4 k_r4_gemm_tok between.
+enum R4Kern { R4_FEW16, R4_FEW32, R4_16x32, R4_32x64, R4_64x64, R4_64x128, R4_TOK, R4_NONE };
 struct R4Tile {
-  int bt, oc;
-  double l0, l1, e, f;
+  R4Kern kern;
+  int bt, oc;  // tokens, output columns
+  double a, b, g[8];
 };
-static constexpr R4Tile R4_PAIR[2][3] = {{{16, 32, 1.5, 1.06, 1.2, 0.25}, {32, 64, 3.0, 1.25, 1.9, 0.80}, {64, 64, 4.0, 1.95, 4.0, 1.38}},
-                                         {{16, 32, 2.0, 0.92, 1.2, 0.25}, {32, 64, 3.0, 1.20, 1.9, 0.80}, {64, 64, 4.0, 1.75, 4.0, 1.15}}};
-static constexpr R4Tile R4_ONE[2][4] = {{{16, 32, 1.0, 0.70, 1.0, 0.178}, {32, 64, 4.0, 0.87, 2.0, 0.50}, {64, 64, 4.0, 1.12, 4.0, 0.72}, {64, 128, 4.0, 1.40, 6.0, 1.43}},
-                                        {{16, 32, 2.5, 0.52, 1.0, 0.16}, {32, 64, 4.0, 0.72, 2.0, 0.46}, {64, 64, 4.0, 0.90, 4.0, 0.64}, {64, 128, 4.0, 1.15, 6.0, 1.28}}};
+static constexpr R4Tile R4_ONE_Q4[] = {
+    {R4_FEW16, 16, 16, 3.18, 1.17, {0.196, 0.404, 0.609, 0.815, 0.994, 1.137, 1.327, 1.516}},
+    {R4_FEW32, 32, 16, 2.93, 1.52, {0.269, 0.549, 0.791, 1.035, 1.288, 1.542, 1.799, 2.056}},
+    {R4_16x32, 16, 32, 4.65, 0.04, {0.570, 0.643, 0.685, 0.767, 0.920, 0.984, 1.148, 1.312}},
+    {R4_32x64, 32, 64, 3.42, 0.95, {0.802, 0.990, 1.360, 1.903, 2.191, 2.457, 2.866, 3.276}},
+    {R4_TOK, 64, 64, 2.50, 1.15, {0.938, 1.502, 2.022, 2.475, 3.176, 3.287, 3.835, 4.383}},
+    {R4_64x128, 64, 128, 2.22, 3.64, {1.355, 2.758, 4.078, 5.439, 6.767, 8.121, 9.475, 10.828}},
+};
+static constexpr R4Tile R4_PAIR_Q4[] = {
+    {R4_FEW16, 16, 16, 2.70, 2.01, {0.250, 0.489, 0.737, 0.990, 1.169, 1.472, 1.653, 1.813}},
+    {R4_16x32, 16, 32, 5.03, 0.43, {0.766, 0.960, 1.015, 1.117, 1.405, 1.534, 1.793, 2.053}},
+    {R4_32x64, 32, 64, 4.70, 1.69, {1.196, 1.488, 2.577, 2.984, 3.828, 4.423, 5.301, 5.815}},
+    {R4_TOK, 64, 32, 6.36, 0.88, {1.169, 1.499, 1.966, 2.536, 3.352, 3.909, 4.705, 5.084}},
+    {R4_64x64, 64, 64, 3.71, 2.16, {1.868, 2.270, 3.933, 4.603, 5.963, 6.761, 7.864, 8.966}},
+};
+static constexpr R4Tile R4_ONE_Q8[] = {
+    {R4_FEW16, 16, 16, 3.69, 0.50, {0.167, 0.302, 0.450, 0.591, 0.720, 0.805, 0.939, 1.073}},
+    {R4_FEW32, 32, 16, 2.81, 1.52, {0.235, 0.480, 0.697, 0.903, 1.111, 1.323, 1.543, 1.764}},
+    {R4_16x32, 16, 32, 4.46, 0.00, {0.469, 0.529, 0.604, 0.697, 0.812, 0.930, 1.085, 1.240}},
+    {R4_32x64, 32, 64, 4.02, 0.82, {0.672, 0.920, 1.231, 1.685, 2.011, 2.269, 2.647, 3.025}},
+    {R4_64x64, 64, 64, 3.15, 1.97, {0.862, 1.112, 1.856, 2.160, 2.826, 3.081, 3.595, 4.108}},
+    {R4_64x128, 64, 128, 1.15, 4.50, {1.083, 2.115, 3.048, 3.978, 4.968, 5.961, 6.955, 7.948}},
+};
+static constexpr R4Tile R4_PAIR_Q8[] = {
+    {R4_FEW16, 16, 16, 4.00, 0.79, {0.250, 0.454, 0.732, 0.968, 1.139, 1.239, 1.446, 1.652}},
+    {R4_16x32, 16, 32, 5.57, 0.03, {0.607, 0.809, 0.970, 1.146, 1.442, 1.595, 1.861, 2.127}},
+    {R4_32x64, 32, 64, 3.80, 1.08, {1.110, 1.624, 2.480, 3.036, 3.823, 4.515, 5.267, 6.020}},
+    {R4_64x64, 64, 64, 3.76, 2.13, {1.638, 2.033, 3.450, 4.130, 5.306, 5.920, 6.907, 7.893}},
+};
+
+// the fastest shape; its grid's extents in `grid`
 template <int N>
-static int r4_pick(const R4Tile (&t)[N], int S, int I, int O, double& bt) {
-  int best = 0;
+static R4Kern r4_pick(const R4Tile (&t)[N], int S, int I, int O, dim3& grid) {
+  R4Kern best = R4_NONE;
+  double bt = 0;
   for (int k = 0; k < N; k++) {
-    const int64_t tiles = (int64_t)((S + t[k].bt - 1) / t[k].bt) * ((O + t[k].oc - 1) / t[k].oc);
-    const double n = (I + 32 * R4M_KG - 1) / (32 * R4M_KG), u = (double)((tiles + 255) / 256);
-    const double lone = t[k].l0 + t[k].l1 * n, full = u * (t[k].e + t[k].f * n), us = lone > full ? lone : full;
-    if (k == 0 || us < bt) best = k, bt = us;
+    if (t[k].bt < 64 && S > t[k].bt * 65535) continue;  // a grid's rows
+    const int64_t gx = (O + t[k].oc - 1) / t[k].oc, gy = (S + t[k].bt - 1) / t[k].bt, j = (gx * gy + 255) / 256;
+    const double n = (I + 32 * R4M_KG - 1) / (32 * R4M_KG), g = j <= 8 ? t[k].g[j - 1] : t[k].g[7] * j / 8;
+    double us = t[k].a + t[k].b * j + n * g;
+    // its workgroups with per-token tokens read and add m8, and are waited for
+    if (t[k].kern == R4_TOK && S % 4) us *= 1.08;
+    if (best != R4_NONE && us >= bt) continue;
+    best = t[k].kern;
+    bt = us;
+    grid = dim3((unsigned)gx, (unsigned)gy);
   }
   return best;
 }
 
-// k_r4_few: the steps of its u workgroups on the busiest CU, fitted likewise
-// (S = 2..200, weights rotating past the Infinity Cache).  Q4R4, 12288 x 4096,
-// 16 / 64 tokens: 65 / 68 us by k_r4_gemm, 22.7 / 55 here; gate + up of 4096 x
-// 12288 36 -> 31.7 (8 groups a step 33.4; Q8R4 30.3, and 33.3 by 16), past 16
-// tokens 38 against 62.
-static double r4_few_us(bool q8, bool pair, int S, int I, int O, bool& two) {
-  const double ng = I / 32;
-  const int64_t cols = (O + 15) / 16;
-  const double u1 = (double)((cols * ((S + 15) / 16) + 255) / 256), u2 = (double)((cols * ((S + 31) / 32) + 255) / 256);
-  two = false;
-  if (pair) return 1.5 + u1 * (q8 ? 1.2 + 0.062 * ng : 1.3 + 0.068 * ng);
-  const double t1 = q8 ? 1.0 + 0.01 * ng + u1 * (1.0 + 0.040 * ng) : 0.9 + u1 * (1.0 + 0.0535 * ng);
-  const double t2 = 1.0 + u2 * (0.9 + (q8 ? 0.0625 : 0.0705) * ng);
-  two = t2 < t1;
-  return two ? t2 : t1;
+#define R4_LAUNCH(KERN, THREADS) \
+  hipLaunchKernelGGL((KERN), grid, dim3(THREADS), 0, st, xq, xs, xm, W, d16, y, S, I, O)
+
+// y [S][O] from quantized activations
+template <bool Q8>
+static int r4_one(const int8_t* xq, const float* xs, const int32_t* xm, const uint8_t* W, const uint16_t* d16, float* y,
+                  int S, int I, int O, hipStream_t st) {
+  dim3 grid;
+  R4Kern k;
+  if constexpr (Q8) k = r4_pick(R4_ONE_Q8, S, I, O, grid);
+  else k = r4_pick(R4_ONE_Q4, S, I, O, grid);
+  if (k == R4_FEW16) R4_LAUNCH((k_r4_few<Q8, false, 1, 16>), 512);
+  else if (k == R4_FEW32) R4_LAUNCH((k_r4_few<Q8, false, 2, 16>), 512);
+  else if (k == R4_16x32) R4_LAUNCH((k_r4_gemm<Q8, false, 16, 1, 1, 2, 1>), 128);
+  else if (k == R4_32x64) R4_LAUNCH((k_r4_gemm<Q8, false, 16, 1, 2, 4, 1>), 256);
+  else if (k == R4_64x128) R4_LAUNCH((k_r4_gemm<Q8, false, 32, 1, 1, 4, 2>), 512);
+  else if constexpr (Q8) R4_LAUNCH((k_r4_gemm<true, false, 32, 1, 1, 2, 2>), 256);
+  else if ((int64_t)grid.x * grid.y <= 256) R4_LAUNCH((k_r4_gemm_tok<16, false>), 1024);
+  else R4_LAUNCH((k_r4_gemm_tok<4, false>), 256);
+  LAUNCH_TRY("R4 matmul");
+  return MOTY_OK;
 }
+
+// y [S][O] = silu(gate) * up, W the row-fused [gate; up] of 2 O rows
+template <bool Q8>
+static int r4_pair(const int8_t* xq, const float* xs, const int32_t* xm, const uint8_t* W, const uint16_t* d16,
+                   float* y, int S, int I, int O, hipStream_t st) {
+  dim3 grid;
+  R4Kern k;
+  if constexpr (Q8) k = r4_pick(R4_PAIR_Q8, S, I, O, grid);
+  else k = r4_pick(R4_PAIR_Q4, S, I, O, grid);
+  if (k == R4_FEW16) R4_LAUNCH((k_r4_few<Q8, true, 1, Q8 ? 8 : 16>), 512);
+  else if (k == R4_16x32) R4_LAUNCH((k_r4_gemm<Q8, true, 16, 2, 1, 2, 1>), 128);
+  else if (k == R4_32x64) R4_LAUNCH((k_r4_gemm<Q8, true, 16, 2, 2, 4, 1>), 256);
+  else if (Q8 || k == R4_64x64) R4_LAUNCH((k_r4_gemm<Q8, true, 32, 2, 1, 2, 2>), 256);
+  else R4_LAUNCH((k_r4_gemm_tok<4, true>), 256);
+  LAUNCH_TRY("R4 gate + up");
+  return MOTY_OK;
+}
+#undef R4_LAUNCH
 
 // y [S][O] = R4 matmul of x [S][I]; xq/xs/xm: scratch for the activation
 // codes (S*I bytes, S*(I/32) floats and ints)
@@ -998,40 +1245,7 @@ int launch_r4_matmul(bool q8, const float* x, const uint8_t* W, const uint16_t* 
   if (!xq || !xs || !xm) return MOTY_EINVAL;  // the GEMM path needs the activation scratch
   int rc = launch_quant_g32(x, xq, xs, xm, S, I, st);
   if (rc) return rc;
-  double us;
-  bool two;
-  const int k = r4_pick(R4_ONE[q8], S, I, O, us);
-  if (r4_few_us(q8, false, S, I, O, two) < us) {
-    const dim3 grid((O + 15) / 16, two ? (S + 31) / 32 : (S + 15) / 16);
-#define R4F(Q, TT) \
-  hipLaunchKernelGGL((k_r4_few<Q, false, TT, 16>), grid, dim3(512), 0, st, xq, xs, xm, W, d16, y, S, I, O)
-    if (two) {
-      if (q8) R4F(true, 2);
-      else R4F(false, 2);
-    } else {
-      if (q8) R4F(true, 1);
-      else R4F(false, 1);
-    }
-#undef R4F
-    LAUNCH_TRY("k_r4_few");
-    return MOTY_OK;
-  }
-  const R4Tile& t = R4_ONE[q8][k];
-  const dim3 grid((O + t.oc - 1) / t.oc, (S + t.bt - 1) / t.bt);
-#define R4G(MT, TT, WR, WT)                                                                                      \
-  if (q8)                                                                                                        \
-    hipLaunchKernelGGL((k_r4_gemm<true, false, MT, 1, TT, WR, WT>), grid, dim3(64 * WR * WT), 0, st, xq, xs, xm, \
-                       W, d16, y, S, I, O);                                                                      \
-  else                                                                                                           \
-    hipLaunchKernelGGL((k_r4_gemm<false, false, MT, 1, TT, WR, WT>), grid, dim3(64 * WR * WT), 0, st, xq, xs, xm, \
-                       W, d16, y, S, I, O)
-  if (k == 0) { R4G(16, 1, 2, 1); }
-  else if (k == 1) { R4G(16, 2, 4, 1); }
-  else if (k == 2) { R4G(32, 1, 2, 2); }
-  else { R4G(32, 1, 4, 2); }
-#undef R4G
-  LAUNCH_TRY("k_r4_gemm");
-  return MOTY_OK;
+  return q8 ? r4_one<true>(xq, xs, xm, W, d16, y, S, I, O, st) : r4_one<false>(xq, xs, xm, W, d16, y, S, I, O, st);
 }
 
 // gate/up + SiLU over a row-fused [gate; up] R4 matrix (2*I rows) for S > 3
@@ -1042,33 +1256,7 @@ int launch_r4_gate_up_gemm(bool q8, const float* x, const uint8_t* W, const uint
   if (S <= 0) return MOTY_OK;
   int rc = launch_quant_g32(x, xq, xs, xm, S, D, st);
   if (rc) return rc;
-  double us;
-  bool two;
-  const int k = r4_pick(R4_PAIR[q8], S, D, I, us);
-  if (r4_few_us(q8, true, S, D, I, two) < us) {
-    const dim3 grid((I + 15) / 16, (S + 15) / 16);
-    if (q8)
-      hipLaunchKernelGGL((k_r4_few<true, true, 1, 8>), grid, dim3(512), 0, st, xq, xs, xm, W, d16, h, S, D, I);
-    else
-      hipLaunchKernelGGL((k_r4_few<false, true, 1, 16>), grid, dim3(512), 0, st, xq, xs, xm, W, d16, h, S, D, I);
-    LAUNCH_TRY("k_r4_few<pair>");
-    return MOTY_OK;
-  }
-  const R4Tile& t = R4_PAIR[q8][k];
-  const dim3 grid((I + t.oc - 1) / t.oc, (S + t.bt - 1) / t.bt);
-#define R4P(MT, TT, WR, WT)                                                                                      \
-  if (q8)                                                                                                        \
-    hipLaunchKernelGGL((k_r4_gemm<true, true, MT, 2, TT, WR, WT>), grid, dim3(64 * WR * WT), 0, st, xq, xs, xm,  \
-                       W, d16, h, S, D, I);                                                                      \
-  else                                                                                                           \
-    hipLaunchKernelGGL((k_r4_gemm<false, true, MT, 2, TT, WR, WT>), grid, dim3(64 * WR * WT), 0, st, xq, xs, xm, \
-                       W, d16, h, S, D, I)
-  if (k == 0) { R4P(16, 1, 2, 1); }
-  else if (k == 1) { R4P(16, 2, 4, 1); }
-  else { R4P(32, 1, 2, 2); }
-#undef R4P
-  LAUNCH_TRY("k_r4_gemm<pair>");
-  return MOTY_OK;
+  return q8 ? r4_pair<true>(xq, xs, xm, W, d16, h, S, D, I, st) : r4_pair<false>(xq, xs, xm, W, d16, h, S, D, I, st);
 }
 
 // Decode gate/up + SiLU over a row-fused [gate; up] R4 matrix (2*I rows,

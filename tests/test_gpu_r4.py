@@ -174,9 +174,16 @@ def test_dense_ffn_r4(ops, q8, S, D, I):
 
 @pytest.mark.parametrize("q8", [False, True])
 @pytest.mark.parametrize("O,I,S", [
-    # every tile of the several-token GEMM (16 x 32, 32 x 64, 64 x 64, 64 x
-    # 128), ragged in rows and tokens (S % 4 != 0: both of the reference's
-    # token forms, in one tile and in different ones), 1, 5 and 33 groups
+    # ragged in rows and tokens (S % 4 != 0: both of the reference's token
+    # forms, in one tile and in different ones), 1, 5, 9, 17, 33 and 65 groups.
+    # By the present times Q4R4 takes, of the several-token kernels, 16 x 32
+    # tiles at (4099, 288, 5) and (545, 544, 260), 32 x 64 at (8201, 288, 19),
+    # 64 x 128 at (8201, 288, 131) and the tokens-as-rows form in 16 waves at
+    # (545, 288, 260) and (8201, 288, 33), in 4 at (4099, 288, 260), (4099, 288,
+    # 503) and (2050, 32, 702); Q8R4 16 x 32 at (8201, 288, 5), 32 x 64 at (545,
+    # 2080, 702), 64 x 64 at (1093, 288, 702), 64 x 128 at (8201, 288, 131)
+    (4099, 288, 5), (545, 544, 260), (8201, 288, 19), (8201, 288, 131), (545, 288, 260), (8201, 288, 33),
+    (4099, 288, 260), (4099, 288, 503), (2050, 32, 702), (8201, 288, 5), (545, 2080, 702), (1093, 288, 702),
     (31, 32, 5), (4099, 32, 130), (8201, 32, 70), (8201, 32, 301), (2050, 32, 503), (8201, 32, 701), (101, 1056, 70),
     (4100, 160, 131), (36, 160, 64), (4100, 288, 99),
     # the few-token kernel's 16 and 32-token tiles: K steps of 16 groups that
@@ -193,7 +200,10 @@ def test_matmul_r4_tiles(ops, q8, O, I, S):
 
 @pytest.mark.parametrize("q8", [False, True])
 @pytest.mark.parametrize("S,D,I", [(5, 32, 96), (70, 32, 8224), (130, 32, 4128), (35, 32, 8224), (67, 288, 160),
-                                   (40, 160, 8224), (399, 160, 4128), (150, 544, 4128), (16, 512, 96), (5, 544, 160), (33, 1056, 64)])
+                                   (40, 160, 8224), (399, 160, 4128), (150, 544, 4128), (16, 512, 96), (5, 544, 160), (33, 1056, 64),
+                                   # Q4R4 tokens-as-rows; 32 x 64, 64 x 64, 16 x 32; Q8R4 32 x 64, 64 x 64
+                                   (260, 544, 4128), (503, 544, 4128), (131, 288, 3008), (702, 288, 1088),
+                                   (5, 288, 4128), (19, 288, 8224), (259, 288, 3008)])
 def test_dense_ffn_r4_tiles(ops, q8, S, D, I):
     """The gate + up form of the same tiles against the plain matmul, SiLU
     and the plain matmul again."""
