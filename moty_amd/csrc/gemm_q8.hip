@@ -187,10 +187,12 @@ __global__ __launch_bounds__(64 * WGM * WGN * KS) void k_gemm_q8_dma(const int8_
     // XCD takes a contiguous run of tiles, walked column by column in groups
     // of GM tile rows, so the 32 tiles its CUs hold at a time share 4 blocks
     // of activation rows and 8 of weight rows in its L2 (256 x 256 tiles, M =
-    // 2000, 24576 x 4096: 273 -> 265 us).  GM = 0, for grids of short K loops:
-    // XCD x takes a (gy/2) x (gx/4) block, half the activation rows and a
-    // quarter of the weight rows (64 x 128 tiles, M = 512, 10240 x 1024: 13.5
-    // us against 17.6 in runs, 15.0 in plain order)
+    // 2000, 24576 x 4096: 273 -> 265 us).  GM = 0, by rows of tiles: XCD x
+    // takes a (gy/2) x (gx/4) block, half the activation rows and a quarter of
+    // the weight rows (64 x 128 tiles, M = 512, 10240 x 1024: 13.5 us against
+    // 17.6 in runs, 15.0 in plain order), or, where the grid does not divide
+    // so, every eighth column of every row in plain order; where that is the
+    // better walk: q8_form
     const int gx = gridDim.x, gy = gridDim.y, lin = by * gx + bx, xcd = lin & 7, j = lin >> 3;
     if constexpr (GM > 0) {
       const int n = gx * gy, q = n / 8, r = n % 8;
@@ -386,6 +388,45 @@ int launch_gemm_q8_pair(const int8_t* xq, const float* sx, const int8_t* W, cons
   return MOTY_OK;
 }
 
+// The forms of one matrix's tiles.  DEEP: four stages instead of three.  ROWS:
+// the former walk of the tiles (GM = 0: blocks of the grid per XCD, or plain
+// order, by rows of tiles) instead of runs in groups of 4 tile rows.
+enum Q8Form { Q8_32x32, Q8_32x64, Q8_64x64, Q8_64x128, Q8_128x128, Q8_256x256,  // as Q8_ONE
+              Q8_64x32, Q8_64x32_ROWS, Q8_64x64_ROWS, Q8_64x64_DEEP, Q8_64x64_DEEP_ROWS };
+
+// Which form of the tile q8_pick chose.  Each line was measured against the
+// form that it replaces over the FFN and projection shapes at M = 5..4000:
+static Q8Form q8_form(int pick, int M, int K, int O) {
+  const int gx = (O + 63) / 64, gy = (M + 63) / 64;
+  const int64_t t = (int64_t)gx * gy;
+  if (pick == Q8_32x64) {
+    // short rows, few tokens: nothing for the K split to hide (M = 24, 10240 x
+    // 1024: 7.3 -> 6.7 us)
+    if (M <= 32 && K <= 2048) return Q8_64x64;
+    // 64 x 32 where that is no more rounds: half the waves' weight reads (M =
+    // 80, 4096 x 12288: 24.1 -> 20.9 us; M = 512, 1024 x 3072: 9.5 -> 9.1)
+    const int gx2 = (O + 31) / 32;
+    if (M > 32 && ((int64_t)gx2 * gy + 255) / 256 <= ((int64_t)gx * ((M + 31) / 32) + 255) / 256) {
+      if (gx2 % 4 == 0 && gy >= 5) return Q8_64x32_ROWS;
+      if (K > 8192 || (gy >= 3 && K > 4096)) return Q8_64x32;
+    }
+  } else if (pick == Q8_64x64) {
+    // a lone tile per CU is its K loop's latency: a stage more (M = 200, 4096 x
+    // 12288: 37.3 -> 31.8 us); with more tiles the third workgroup that fits a
+    // CU with three stages hides more (M = 512, 4864 x 896: 15 % slower in four)
+    if (t <= 256) return K >= 2048 && (gy > 1 || K > 2048) ? Q8_64x64_DEEP : Q8_64x64;
+    // few tiles more than CUs, long rows: four stages, and by rows, since groups
+    // of 4 tile rows leave the last XCDs a short group and with it all the
+    // weights (M = 300, 4096 x 12288: 51.5 -> 37.8 us, three stages 42; from
+    // 449 tiles on no gain)
+    if (gx % 4 == 0 && gy >= 5 && K >= 4096 && t <= (K >= 5120 ? 448 : 384)) return Q8_64x64_DEEP_ROWS;
+    // an odd number of tile rows: by rows for the same reason (M = 192, 12288 x
+    // 4096: 31.3 -> 27.4 us)
+    if (gx % 4 == 0 && gy % 2 && gy > 1 && gy < 16 && t < 768) return Q8_64x64_ROWS;
+  }
+  return (Q8Form)pick;
+}
+
 int launch_gemm_q8(const int8_t* xq, const float* sx, const int8_t* W, const float* scale, float* y, int M,
                    int K, int O, hipStream_t st) {
   if (K % 16) return MOTY_EUNSUP;
@@ -394,16 +435,20 @@ int launch_gemm_q8(const int8_t* xq, const float* sx, const int8_t* W, const flo
     // Every form writes y with nontemporal stores: the output then does not
     // sit dirty in L2 to be evicted under the next kernels' reads (at M =
     // 512 a layer's seven projections 42.7 -> 40.8 us).
-    const int k = q8_pick(Q8_ONE, M, K, O);
-    const dim3 grid((O + Q8_ONE[k].oc - 1) / Q8_ONE[k].oc, (M + Q8_ONE[k].bm - 1) / Q8_ONE[k].bm);
-#define QD(BM, BN, S, WM, WN, KS, GM)                                                                         \
-  hipLaunchKernelGGL((k_gemm_q8_dma<BM, BN, S, WM, WN, KS, false, GM>), grid, dim3(64 * WM * WN * KS), 0, st, \
-                     xq, sx, W, scale, nullptr, nullptr, y, M, K, O)
-    if (k == 0) QD(32, 32, 4, 1, 1, 4, 4);
-    else if (k == 1) QD(32, 64, 3, 1, 2, 4, 4);
-    else if (k == 2) QD(64, 64, 3, 2, 2, 1, 4);
-    else if (k == 3) QD(64, 128, 2, 2, 4, 1, 0);
-    else if (k == 4) QD(128, 128, 2, 4, 2, 1, 4);
+    const Q8Form k = q8_form(q8_pick(Q8_ONE, M, K, O), M, K, O);
+#define QD(BM, BN, S, WM, WN, KS, GM)                                                                     \
+  hipLaunchKernelGGL((k_gemm_q8_dma<BM, BN, S, WM, WN, KS, false, GM>), dim3((O + BN - 1) / BN, (M + BM - 1) / BM), \
+                     dim3(64 * WM * WN * KS), 0, st, xq, sx, W, scale, nullptr, nullptr, y, M, K, O)
+    if (k == Q8_32x32) QD(32, 32, 4, 1, 1, 4, 4);
+    else if (k == Q8_32x64) QD(32, 64, 3, 1, 2, 4, 4);
+    else if (k == Q8_64x32) QD(64, 32, 3, 2, 1, 4, 4);
+    else if (k == Q8_64x32_ROWS) QD(64, 32, 3, 2, 1, 4, 0);
+    else if (k == Q8_64x64) QD(64, 64, 3, 2, 2, 1, 4);
+    else if (k == Q8_64x64_ROWS) QD(64, 64, 3, 2, 2, 1, 0);
+    else if (k == Q8_64x64_DEEP) QD(64, 64, 4, 2, 2, 1, 4);
+    else if (k == Q8_64x64_DEEP_ROWS) QD(64, 64, 4, 2, 2, 1, 0);
+    else if (k == Q8_64x128) QD(64, 128, 2, 2, 4, 1, 0);
+    else if (k == Q8_128x128) QD(128, 128, 2, 4, 2, 1, 4);
     else QD(256, 256, 2, 2, 4, 1, 4);
 #undef QD
     LAUNCH_TRY("k_gemm_q8_dma");

@@ -184,9 +184,15 @@ def test_matmul_q_s(ops, S, I, O):
 
 
 @pytest.mark.parametrize("S,I,O", [
-    # each tile shape of the int8 GEMM (32 x 32 and 32 x 64 with K split four
-    # ways, 64 x 64, 64 x 128, 128 x 128, 256 x 256), ragged in tokens and
-    # rows, with one K block, fewer than the wave groups, and many
+    # each tile shape of the int8 GEMM, ragged in tokens and rows, with one K
+    # block, fewer than the wave groups, and many.  By the present times 32 x 32
+    # at (600, 4096, 100) and (5, 512, 33), 32 x 64 at (100, 3072, 2081), 64 x
+    # 32 at (257, 5120, 901), by rows at (257, 1024, 1000), 64 x 64 at (300,
+    # 256, 3001), by rows at (257, 128, 4095), in four stages at (515, 2048,
+    # 1000), those by rows at (321, 4096, 3071), 64 x 128 at (250, 128, 20001)
+    # and (1001, 1024, 10239), 128 x 128 at (2001, 1024, 10241), 256 x 256 at
+    # (4095, 12288, 4095)
+    (5, 512, 33), (257, 5120, 901), (257, 1024, 1000), (257, 128, 4095), (515, 2048, 1000), (321, 4096, 3071),
     (600, 4096, 100), (3, 128, 31), (100, 3072, 2081), (300, 256, 3001), (70, 128, 33), (250, 128, 20001),
     (1001, 1024, 10239), (2001, 1024, 10241), (4095, 12288, 4095)])
 def test_gemm_q8_tiles(ops, S, I, O):
@@ -203,8 +209,12 @@ def test_gemm_q8_tiles(ops, S, I, O):
 
 
 @pytest.mark.parametrize("S,D,I", [
-    # each gate + up tile (32 x 32, 64 x 32, 128 x 64, 256 x 128 columns),
-    # ragged; D % 128 != 0 runs the two GEMMs and silu_mul
+    # each gate + up tile, ragged in tokens and columns: by the present times 32
+    # x 32 (tokens x columns) at (24, 1024, 3088), 64 x 32 at (33, 512, 5008),
+    # 128 x 64 at (5, 128, 48), (130, 256, 2000) and (2001, 4096, 12304), 256 x
+    # 128 at (515, 2048, 10256) and (2001, 4096, 12272); D % 128 != 0 runs the
+    # two GEMMs and silu_mul
+    (33, 512, 5008), (515, 2048, 10256), (2001, 4096, 12272),
     (5, 128, 48), (24, 1024, 3088), (70, 1024, 3072), (130, 256, 2000), (2001, 4096, 12304), (37, 1088, 3008)])
 def test_dense_ffn_q8_prefill_tiles(ops, S, D, I):
     """The fused gate + up GEMM against one GEMM each and silu_mul."""
