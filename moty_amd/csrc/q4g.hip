@@ -794,6 +794,9 @@ __global__ __launch_bounds__(NW * 64, NW <= 8 ? 8 / NW : 1) void k_gemm_i4g_h(co
 static bool gemm_i4g_h_big(int M, int O) { return (int64_t)((M + 127) / 128) * ((O + 127) / 128) >= 160; }
 // 128 x 128 tiles give every CU a workgroup
 static bool gemm_i4g_h_full(int M, int O) { return (int64_t)((M + 127) / 128) * ((O + 127) / 128) >= 256; }
+static bool gemm_i4g_h_pair192(int M, int O) {
+  return !gemm_i4g_h_full(M, O) && (int64_t)((M + 63) / 64) * ((O + 191) / 192) >= 192;
+}
 int gemm_i4g_h_f8(int M, int O, bool pair) { return !pair && !gemm_i4g_h_big(M, O); }
 
 // the f16 GEMM's 32-bit buffer offsets: activations and nibbles under 4 GiB
@@ -811,9 +814,8 @@ int launch_gemm_i4g_h(const uint16_t* xh, const float* sx, const uint8_t* q4, co
 #define Q4H(BM, BN, S, WGM, NW, P, T16)                                                                         \
   hipLaunchKernelGGL((k_gemm_i4g_h<BM, BN, S, WGM, NW, P, T16>), dim3((O + BN - 1) / BN, (M + BM - 1) / BM),   \
                      dim3(NW * 64), 0, st, xh, sx, q4, scl, q4b, sclb, y, M, I, O)
-  const bool pair192 = !gemm_i4g_h_full(M, O) && (int64_t)((M + 63) / 64) * ((O + 191) / 192) >= 192;
   if (q4b) {
-    if (pair192) Q4H(64, 192, 2, 1, 6, true, false);
+    if (gemm_i4g_h_pair192(M, O)) Q4H(64, 192, 2, 1, 6, true, false);
     else if (big) Q4H(128, 128, 3, 2, 8, true, false);
     else Q4H(64, 64, 3, 2, 4, true, false);
   } else {
@@ -1450,34 +1452,51 @@ __global__ __launch_bounds__(64 * WN * KS, 2) void k_gemm_i4g_few(const int8_t* 
   }
 }
 
-// Time of a launch, us, as u workgroups on the busiest CU (ceil(all / 256))
-// times a + b * groups, fitted on MI355X to sweeps over M = 2..100, six (I, O)
-// pairs, (1, 2, 4) x 16 tokens, 16-32 columns and 8 or 16 groups a step,
-// weights rotating past the Infinity Cache: gate + up of 4096 x 12288 25.7 us
-// up to 16 tokens (16 groups a step 27.8, two column tiles 33) and 42 up to
-// 32; 12288 x 4096 16.5 (8 groups 29) and 22 (29).
+// The IDOT4 kernels' tiles (tokens, columns) and times: a launch with j tiles on
+// the busiest CU (ceil(tiles / 256)) takes a + b * j + g[j] * groups us, past
+// eight tiles g[8] * j / 8.  Fitted on MI355X to M = 5..512 over 25 (I, O) pairs
+// from 576 x 1536 to 12352 x 4096, weights rotating past the Infinity Cache, to
+// 2 to 6 % (root mean square).  Gate + up of 4096 x 12288: few-token kernel 25.7
+// us up to 16 tokens (16 groups a step 27.8, two column tiles 33) and 42 up to
+// 32, f16-MFMA tiles 42 to 64; 12288 x 4096 16.5 (8 groups 29), 22 (29) and 57.
+struct I4Tile {
+  int bm, oc;
+  double a, b, g[8];
+};
+static constexpr I4Tile I4_FEW_ONE[] = {{16, 16, 3.80, 0.59, {0.0336, 0.0577, 0.0868, 0.1127, 0.1396, 0.1649, 0.1904, 0.2053}},
+                                        {32, 16, 3.04, 1.62, {0.0481, 0.0963, 0.1414, 0.1863, 0.2325, 0.2758, 0.3237, 0.3641}}};
+static constexpr I4Tile I4_FEW_PAIR[] = {{16, 16, 3.76, 0.59, {0.0642, 0.1029, 0.1445, 0.1905, 0.2309, 0.2731, 0.3146, 0.3380}},
+                                         {32, 16, 2.60, 1.83, {0.0895, 0.1737, 0.2592, 0.3435, 0.4265, 0.5089, 0.5972, 0.6635}}};
+static constexpr I4Tile I4_INT8 = {64, 64, 2.79, 2.00, {0.1816, 0.2434, 0.3393, 0.4399, 0.4933, 0.5706, 0.6657, 0.7608}};
+static constexpr I4Tile I4_H_ONE = {64, 64, 2.90, 2.71, {0.1335, 0.2746, 0.4106, 0.5474, 0.6843, 0.8212, 0.9580, 1.0949}};
+static constexpr I4Tile I4_H_ONE_BIG = {128, 128, 4.03, 4.08, {0.3722, 0.7232, 1.0848, 1.4465, 1.8081, 2.1697, 2.5313, 2.8929}};
+static constexpr I4Tile I4_H_PAIR = {64, 64, 6.80, 1.85, {0.2382, 0.3787, 0.6003, 0.8004, 1.0005, 1.2006, 1.4007, 1.6008}};
+static constexpr I4Tile I4_H_PAIR_BIG = {128, 128, 6.87, 9.34, {0.5647, 1.0630, 1.5946, 2.1261, 2.6576, 3.1891, 3.7206, 4.2521}};
+static constexpr I4Tile I4_H_PAIR_192 = {64, 192, 3.69, 10.11, {0.5399, 1.0007, 1.5011, 2.0014, 2.5018, 3.0022, 3.5025, 4.0029}};
+
+static double i4_us(const I4Tile& t, int M, int I, int O) {
+  const int64_t j = ((int64_t)((M + t.bm - 1) / t.bm) * ((O + t.oc - 1) / t.oc) + 255) / 256;
+  return t.a + t.b * j + (I / 32) * (j <= 8 ? t.g[j - 1] : t.g[7] * j / 8);
+}
+
 static double few_us(int M, int I, int O, bool pair, bool* two) {
-  const double ng = I / 32;
-  const int64_t cols = (O + 15) / 16;
-  const double u1 = (double)((cols * ((M + 15) / 16) + 255) / 256), u2 = (double)((cols * ((M + 31) / 32) + 255) / 256);
-  const double t1 = pair ? u1 * (1.5 + 0.0405 * ng) : u1 * (0.5 + 0.029 * ng) + 1.7 + 0.008 * ng;
-  const double t2 = pair ? u2 * (1.5 + 0.100 * ng) : u2 * (0.7 + 0.050 * ng) + 1.5 + 0.006 * ng;
+  const I4Tile* t = pair ? I4_FEW_PAIR : I4_FEW_ONE;
+  const double t1 = i4_us(t[0], M, I, O), t2 = i4_us(t[1], M, I, O);
   *two = t2 < t1;
   return *two ? t2 : t1;
 }
 
-// The alternatives' times: the f16-MFMA tiles (64 tokens: a lone tile's K
-// loop, 42 us at 128 groups with SiLU, 57 at 384 without; at M = 128, two
-// tiles on a CU, 62), or, for other row lengths, one int8-MFMA GEMM each for
-// gate and up and silu_mul.
+// against the f16-MFMA tiles or, for other row lengths, the int8-MFMA GEMM (one
+// each for gate and up, and silu_mul)
 bool i4g_few_wins(int M, int I, int O, bool pair, bool f16) {
   if (M > 512) return false;
   bool two;
-  const double ng = I / 32, few = few_us(M, I, O, pair, &two);
-  const double u = (double)(((int64_t)((M + 63) / 64) * ((O + 63) / 64) + 255) / 256);
-  const double other = f16 ? (pair ? 6.0 + 0.14 * ng + u * 0.14 * ng : 3.5 + 0.10 * ng + u * 0.04 * ng)
-                           : (pair ? 2 : 1) * (3.0 + 0.15 * ng + u * 0.09 * ng) + (pair ? 4 : 0);
-  return few < other;
+  const double few = few_us(M, I, O, pair, &two);
+  if (!f16) return few < (pair ? 2 * i4_us(I4_INT8, M, I, O) + 4 : i4_us(I4_INT8, M, I, O));
+  const bool big = gemm_i4g_h_big(M, O);
+  const I4Tile& h = !pair ? (big ? I4_H_ONE_BIG : I4_H_ONE)
+                          : gemm_i4g_h_pair192(M, O) ? I4_H_PAIR_192 : big ? I4_H_PAIR_BIG : I4_H_PAIR;
+  return few < i4_us(h, M, I, O);
 }
 
 int launch_gemm_i4g_few(const int8_t* xq, const float* sx, const uint8_t* q4, const float* scl, const uint8_t* q4b,

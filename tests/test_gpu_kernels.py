@@ -246,7 +246,11 @@ def test_matmul_q8_extremes(ops):
                                    (256, 4096, 192), (37, 1024, 100), (5, 128, 64), (1, 12288, 100),
                                    (9, 192, 40), (70, 64, 33), (65, 12288, 70),
                                    (1, 8192, 77), (1, 16384, 40), (1, 2048, 1000), (130, 1088, 200), (64, 12288, 64),
-                                   (250, 1024, 4100)])
+                                   # past the few-token kernel by the present times: the f16-MFMA
+                                   # GEMM in 64 x 64 and 128 x 128 tiles, the int8-MFMA GEMM with
+                                   # two and (I >= 4096) three K blocks in flight
+                                   (250, 1024, 4100), (513, 1024, 100), (390, 256, 8223), (130, 256, 12401),
+                                   (600, 576, 200), (513, 1088, 100), (200, 576, 1540), (513, 4160, 200)])
 def test_i4g_idot4(ops, S, I, O):
     say("i4g idot4", S, I, O)
     w = randn(O + I, (O, I), 0.02)
@@ -279,8 +283,8 @@ def test_gate_up_silu_i4g(ops, D, I):
                                    (1, 12288, 100), (1, 8192, 77), (1, 96, 40), (1, 2080, 300), (1, 16384, 20),
                                    (1, 14336, 300), (2, 16384, 64), (1, 16416, 10),
                                    (1, 64, 1000),
-                                   # 2..24 tokens: the GEMV per token; more: the tiled GEMM (64 x 64
-                                   # tiles, ragged in tokens and rows; I % 64 != 0 falls back)
+                                   # several tokens: the GEMV per token or the f32-MFMA GEMM, by
+                                   # measured time, ragged in tokens and rows
                                    (4, 2048, 100), (65, 4096, 130), (256, 1088, 70), (7, 128, 33),
                                    (24, 1024, 96), (25, 1024, 96), (40, 128, 33), (5, 96, 40)])
 def test_i4g_f32(ops, S, I, O):
@@ -294,8 +298,9 @@ def test_i4g_f32(ops, S, I, O):
 
 
 @pytest.mark.parametrize("S,I,O", [
-    # one and two 16-token tiles, several workgroups of tokens, ragged rows,
-    # steps of 8 or 16 groups that are short, full, and followed by a part
+    # one and two 16-token tiles a workgroup (the two at (50, 3072, 1030)),
+    # several workgroups of tokens, ragged rows, steps of 8 or 16 groups that
+    # are short, full, and followed by a part
     (2, 64, 33), (16, 512, 100), (16, 576, 47), (17, 64, 16), (32, 1088, 130), (31, 512, 1), (5, 4096, 70),
     (3, 12288, 40), (33, 1088, 70), (50, 3072, 1030), (97, 1024, 3075), (200, 576, 640)])
 def test_i4g_few_tokens(ops, S, I, O):
@@ -309,7 +314,9 @@ def test_i4g_few_tokens(ops, S, I, O):
 
 
 @pytest.mark.parametrize("S,D,I", [(2, 64, 192), (16, 512, 80 * 8), (17, 576, 64), (32, 1088, 448), (9, 4096, 128),
-                                   (70, 576, 3008), (130, 64, 128)])
+                                   (70, 576, 3008), (130, 64, 128),
+                                   # two 16-token tiles a workgroup
+                                   (32, 1088, 3008), (30, 1024, 3136)])
 def test_dense_ffn_i4g_few_tokens(ops, S, D, I):
     """The gate + up form, whose gate and up chains sit in different waves."""
     say("dense_ffn_i4g few tokens", S, D, I)
@@ -397,15 +404,18 @@ def test_silu_and_softmax(ops):
                                    (70, 192, 320), (3, 4096, 96), (300, 512, 1280),
                                    # 64 x 192 gate/up tiles, ragged in tokens and rows
                                    (130, 256, 12416),
+                                   # 64 x 64 and 128 x 128 ones; two int8 GEMMs and silu_mul
+                                   (513, 256, 544), (390, 256, 8224), (300, 1088, 3008),
                                    # one token through the exact-f32 fused gate/up GEMV
                                    (1, 4096, 1056), (1, 96, 8192), (1, 12288, 2080),
                                    # rows past 12288 (more than 64 KiB of x in LDS), and 2-4
                                    # tokens through the per-token GEMV
                                    (1, 1024, 14336), (1, 16384, 96), (3, 1024, 2048), (4, 14336, 64)])
 def test_dense_ffn_i4g(ops, idot4, S, D, I):
-    # nn/ffn.c:26-55 over grouped-int4 Mats: the fused gate/up f16 pass
-    # (S > 4, D and I multiples of 128), the int8 GEMM fallback (other
-    # multiples of 64), the GEMVs (S <= 4) and the exact f32 path
+    # nn/ffn.c:26-55 over grouped-int4 Mats.  IDOT4: the one-token GEMVs, the
+    # few-token kernel, the fused gate/up f16 pass (D a multiple of 128), the
+    # int8 GEMM (other multiples of 64), each matrix by its measured time; the
+    # exact f32 path: the GEMV per token or the f32-MFMA GEMM
     say("dense_ffn_i4g", idot4, S, D, I)
     gq, gs = o_pack_int4_grouped(randn(S + D, (I, D), 0.02))
     uq, us = o_pack_int4_grouped(randn(S + D + 1, (I, D), 0.02))
