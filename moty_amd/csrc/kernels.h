@@ -57,8 +57,8 @@ int launch_gemm_q8(const int8_t* xq, const float* sx, const int8_t* W, const flo
 int launch_gemm_q8_pair(const int8_t* xq, const float* sx, const int8_t* W, const float* scale, const int8_t* W2,
                         const float* scale2, float* y, int M, int K, int O, hipStream_t st);
 
-// IDOT4, one token (S > 1: each on its own in one launch, no scratch); q4b/sclb
-// non-null: PAIR mode, y = silu(x.q4^T) * (x.q4b^T)
+// IDOT4, one token; q4b/sclb non-null: PAIR mode, y = silu(x.q4^T) * (x.q4b^T),
+// else S > 1 takes each token on its own in one launch (no scratch)
 int launch_gemv_i4g(const float* x, const uint8_t* q4, const float* scl, const uint8_t* q4b, const float* sclb,
                     float* y, int I, int O, hipStream_t st, int S = 1);
 // IDOT4, a few tokens quantized by launch_qrow_i8 (PAIR alike); I % 32 == 0,

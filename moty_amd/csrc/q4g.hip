@@ -47,9 +47,9 @@ __device__ __forceinline__ float cvt_off_b(uint32_t w) {
 //      and parks it, with the group scale, in the wave's LDS slice;
 //   4. one lane per row extends the reference's FMA chain over the chunk's
 //      groups in order; y = sx * acc (PAIR: h = silu(g) * u).
-// blockIdx.y: the token (one for decode; 2..4 where a call must not keep its
-// activation codes in memory, the weights then coming from the caches).
-template <int RW, int NGC, bool PAIR, int NT, int PD = NGC, bool XF = false>
+// MT: several tokens, blockIdx.y, where a call must not keep its activation
+// codes in memory (the weights of all but the first come from the caches).
+template <int RW, int NGC, bool PAIR, int NT, int PD = NGC, bool XF = false, bool MT = false>
 __global__ __launch_bounds__(NT) void k_gemv1_i4g(const float* __restrict__ x, const uint8_t* __restrict__ q4,
                                                       const float* __restrict__ scl,
                                                       const uint8_t* __restrict__ q4b,
@@ -63,8 +63,10 @@ __global__ __launch_bounds__(NT) void k_gemv1_i4g(const float* __restrict__ x, c
   __shared__ float sx_s;
   const int lane = threadIdx.x % MOTY_WAVE, wv = threadIdx.x / MOTY_WAVE;
   const int ng = I / 32, rb = I / 2;
-  x += (int64_t)blockIdx.y * I;
-  y += (int64_t)blockIdx.y * O;
+  if constexpr (MT) {
+    x += (int64_t)blockIdx.y * I;
+    y += (int64_t)blockIdx.y * O;
+  }
   constexpr int ldv = 66;  // one chunk's 64 groups, padded (even: float4 reads stay aligned)
   int8_t* xq_s = lds;                                                          // [I]
   int* xg8 = (int*)(lds + I);                                                  // [ng] -8 * group sums
@@ -914,7 +916,7 @@ int launch_i4row_f32(const float* x, const uint8_t* q4, const float* scale, floa
 
 // NT = 256 or 512 threads: wider workgroups amortize the activation row
 // (read once per workgroup) over more weight rows when I is large
-template <int RW, int NGC, bool PAIR, int NT, int PD = NGC, bool XF = false>
+template <int RW, int NGC, bool PAIR, int NT, int PD = NGC, bool XF = false, bool MT = false>
 static int go_gemv1_i4g(const float* x, const uint8_t* q4, const float* scl, const uint8_t* q4b, const float* sclb,
                         float* y, int I, int O, hipStream_t st, int S = 1) {
   constexpr int NM = PAIR ? 2 : 1;
@@ -931,7 +933,7 @@ static int go_gemv1_i4g(const float* x, const uint8_t* q4, const float* scl, con
       return MOTY_EUNSUP;
     }
     if (lds > allowed[dev]) {
-      if (hipFuncSetAttribute((const void*)&k_gemv1_i4g<RW, NGC, PAIR, NT, PD, XF>,
+      if (hipFuncSetAttribute((const void*)&k_gemv1_i4g<RW, NGC, PAIR, NT, PD, XF, MT>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
         (void)hipGetLastError();  // leave no error for a later call to find
         return MOTY_EUNSUP;
@@ -940,7 +942,7 @@ static int go_gemv1_i4g(const float* x, const uint8_t* q4, const float* scl, con
     }
   }
   const unsigned nb = (unsigned)((O + RW * (NT / MOTY_WAVE) - 1) / (RW * (NT / MOTY_WAVE)));
-  hipLaunchKernelGGL((k_gemv1_i4g<RW, NGC, PAIR, NT, PD, XF>), dim3(nb, S), dim3(NT), lds, st, x, q4, scl, q4b, sclb, y, I, O);
+  hipLaunchKernelGGL((k_gemv1_i4g<RW, NGC, PAIR, NT, PD, XF, MT>), dim3(nb, S), dim3(NT), lds, st, x, q4, scl, q4b, sclb, y, I, O);
   LAUNCH_TRY("k_gemv1_i4g");
   return MOTY_OK;
 }
@@ -969,42 +971,49 @@ int launch_gemv_i4g_xf(const float* x, const uint8_t* q4, const float* scl, cons
   return go_gemv1_i4g<2, 8, false, 256, 1, true>(x, q4, scl, nullptr, nullptr, y, I, O, st);
 }
 
-int launch_gemv_i4g(const float* x, const uint8_t* q4, const float* scl, const uint8_t* q4b, const float* sclb,
-                    float* y, int I, int O, hipStream_t st, int S) {
-  if ((I % 64) || I > 16384) return MOTY_EUNSUP;
-  if (O <= 0 || S <= 0) return MOTY_OK;
-  // widest instance whose LDS fits, else the next narrower one
+// one matrix: the widest instance whose LDS fits, else the next narrower one
+template <bool MT>
+static int go_gemv_i4g(const float* x, const uint8_t* q4, const float* scl, float* y, int I, int O, hipStream_t st, int S) {
   const int ngc = (I / 32 + 63) / 64;
   int rc = MOTY_EUNSUP;
-  if (q4b) {
-    // up to 2 chunks (I <= 4096): 2 gate + 2 up rows per wave (12288 x
-    // 4096 pair: 12.2 us against 12.5 with 4 + 4, 14.2 with 1 + 1, 13.6
-    // for 2 + 2 in 2-wave workgroups or with both chunks issued at once)
-    if (ngc <= 2) rc = go_gemv1_i4g<2, 2, true, 256, 1>(x, q4, scl, q4b, sclb, y, I, O, st, S);
-    else if (ngc <= 4) {
-      rc = go_gemv1_i4g<2, 4, true, 512>(x, q4, scl, q4b, sclb, y, I, O, st, S);
-      if (rc == MOTY_EUNSUP) rc = go_gemv1_i4g<2, 4, true, 256>(x, q4, scl, q4b, sclb, y, I, O, st, S);
-    } else if (ngc <= 8) {
-      rc = go_gemv1_i4g<1, 8, true, 512>(x, q4, scl, q4b, sclb, y, I, O, st, S);
-      if (rc == MOTY_EUNSUP) rc = go_gemv1_i4g<1, 8, true, 256>(x, q4, scl, q4b, sclb, y, I, O, st, S);
-    }
-    return rc;
-  }
-  if (ngc <= 2) rc = go_gemv1_i4g<8, 2, false, 256>(x, q4, scl, nullptr, nullptr, y, I, O, st, S);
+  if (ngc <= 2) rc = go_gemv1_i4g<8, 2, false, 256, 2, false, MT>(x, q4, scl, nullptr, nullptr, y, I, O, st, S);
   else if (ngc <= 4) {
-    rc = go_gemv1_i4g<4, 4, false, 512>(x, q4, scl, nullptr, nullptr, y, I, O, st, S);
-    if (rc == MOTY_EUNSUP) rc = go_gemv1_i4g<4, 4, false, 256>(x, q4, scl, nullptr, nullptr, y, I, O, st, S);
+    rc = go_gemv1_i4g<4, 4, false, 512, 4, false, MT>(x, q4, scl, nullptr, nullptr, y, I, O, st, S);
+    if (rc == MOTY_EUNSUP) rc = go_gemv1_i4g<4, 4, false, 256, 4, false, MT>(x, q4, scl, nullptr, nullptr, y, I, O, st, S);
   } else if (ngc <= 6) {
     // 4096 x 12288 (8B down) in a sweep of rows/wave x workgroup size x
     // chunks in flight on MI355X, graph replays over rotating weights:
     // 4 rows x 256 threads, one chunk ahead 8.0 us; two ahead 9.3, all six
     // 10.9 (the whole row's chains then run after its last byte lands);
     // 2 rows 9.6 / 10.9; 8 rows x 128 threads 10.1
-    rc = go_gemv1_i4g<4, 6, false, 256, 1>(x, q4, scl, nullptr, nullptr, y, I, O, st, S);
+    rc = go_gemv1_i4g<4, 6, false, 256, 1, false, MT>(x, q4, scl, nullptr, nullptr, y, I, O, st, S);
   } else if (ngc <= 8) {
-    rc = go_gemv1_i4g<2, 8, false, 256>(x, q4, scl, nullptr, nullptr, y, I, O, st, S);
+    rc = go_gemv1_i4g<2, 8, false, 256, 8, false, MT>(x, q4, scl, nullptr, nullptr, y, I, O, st, S);
   }
   return rc;
+}
+
+int launch_gemv_i4g(const float* x, const uint8_t* q4, const float* scl, const uint8_t* q4b, const float* sclb,
+                    float* y, int I, int O, hipStream_t st, int S) {
+  if ((I % 64) || I > 16384 || (q4b && S > 1)) return MOTY_EUNSUP;
+  if (O <= 0 || S <= 0) return MOTY_OK;
+  if (q4b) {
+    const int ngc = (I / 32 + 63) / 64;
+    int rc = MOTY_EUNSUP;
+    // up to 2 chunks (I <= 4096): 2 gate + 2 up rows per wave (12288 x
+    // 4096 pair: 12.2 us against 12.5 with 4 + 4, 14.2 with 1 + 1, 13.6
+    // for 2 + 2 in 2-wave workgroups or with both chunks issued at once)
+    if (ngc <= 2) rc = go_gemv1_i4g<2, 2, true, 256, 1>(x, q4, scl, q4b, sclb, y, I, O, st);
+    else if (ngc <= 4) {
+      rc = go_gemv1_i4g<2, 4, true, 512>(x, q4, scl, q4b, sclb, y, I, O, st);
+      if (rc == MOTY_EUNSUP) rc = go_gemv1_i4g<2, 4, true, 256>(x, q4, scl, q4b, sclb, y, I, O, st);
+    } else if (ngc <= 8) {
+      rc = go_gemv1_i4g<1, 8, true, 512>(x, q4, scl, q4b, sclb, y, I, O, st);
+      if (rc == MOTY_EUNSUP) rc = go_gemv1_i4g<1, 8, true, 256>(x, q4, scl, q4b, sclb, y, I, O, st);
+    }
+    return rc;
+  }
+  return S == 1 ? go_gemv_i4g<false>(x, q4, scl, y, I, O, st, 1) : go_gemv_i4g<true>(x, q4, scl, y, I, O, st, S);
 }
 
 int launch_gemm_i4g(const int8_t* xq, const float* sx, const uint8_t* q4, const float* scl, float* y, int M,
