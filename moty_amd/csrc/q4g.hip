@@ -1560,17 +1560,19 @@ static int xf_pick(int M, int I, int O, bool pair, double* us) {
   return best;
 }
 
-// S tokens: the one-token GEMV once per token (about 4 us plus the matrix
-// bytes at 5 TB/s each: 5.0 us at 1024 x 3072 gate + up, 14.2 at 4096 x
-// 12288), or the GEMM above?  The GEMM wins from 3 tokens at the smaller
-// shapes and from 6 at the larger one (82 us for up to 16 tokens).
+// S tokens: the one-token GEMV once per token, its row's latency or, from the
+// second token out of the Infinity Cache, the matrix bytes at 5.6 TB/s each
+// (1024 x 3072 gate + up 4.4 us a token, 4096 x 12288 13.4, 14336 x 4096 11.5),
+// or the GEMM above?  Measured at 2 to 10 tokens over 23 shapes: the GEMM wins
+// from 2 to 4 tokens at the smaller shapes, at the larger ones from 6 (gate + up
+// of 4096 x 12288, 5 / 6 tokens: 71 / 85 us against 84) or 8.
 bool xf_gemv_per_token(int S, int I, int O, bool pair) {
   if (S <= 1) return true;
   if (S > 64) return false;
   double gemm_us;
   xf_pick(S, I, O, pair, &gemm_us);
-  const double gemv_us = 4.0 + ((double)O * I * (pair ? 1.25 : 0.625)) / 5.0e6;
-  return S * gemv_us < gemm_us + 3.0;
+  const double row_us = 3.8 + 0.54e-3 * I, bytes_us = 3.9 + 0.178e-6 * ((double)O * I * (pair ? 1.25 : 0.625));
+  return S * (row_us > bytes_us ? row_us : bytes_us) < gemm_us + 1.6;
 }
 
 // I % 32 == 0, 16-byte aligned x and 8-byte aligned nibbles; PAIR (q4b):
