@@ -237,10 +237,11 @@ __global__ __launch_bounds__(NW * MOTY_WAVE) void k_gemv1_q8(const float* __rest
     }
   }
   // the RPW row sums at once: lane l ends with row rl's; the first lane of
-  // each group holding a row finishes it (computed on every lane, so the
-  // scale loads above stay where they were issued)
+  // each group holding a row finishes it
   const int a = wave_sum_multi_i32<RPW>(acc);
   const int a2 = PAIR ? wave_sum_multi_i32<RPW>(acc2) : 0;
+  keep_loaded(sc, a);
+  if (PAIR) keep_loaded(sc2, a2);
   float v = (sc * sx) * (float)a;
   if (PAIR) v = ref_silu_mul(v, (sc2 * sx) * (float)a2);
   const int o = o0 + rl;
@@ -350,10 +351,11 @@ __global__ __launch_bounds__(NW * MOTY_WAVE) void k_gemv1_q8_lds(const float* __
     }
   }
   // the RPW row sums at once: lane l ends with row rl's; the first lane of
-  // each group holding a row finishes it (computed on every lane, so the
-  // scale loads above stay where they were issued)
+  // each group holding a row finishes it
   const int a = wave_sum_multi_i32<RPW>(acc);
   const int a2 = PAIR ? wave_sum_multi_i32<RPW>(acc2) : 0;
+  keep_loaded(sc, a);
+  if (PAIR) keep_loaded(sc2, a2);
   float v = (sc * sx) * (float)a;
   if (PAIR) v = ref_silu_mul(v, (sc2 * sx) * (float)a2);
   const int o = o0 + rl;

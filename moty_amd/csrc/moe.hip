@@ -842,7 +842,7 @@ __global__ __launch_bounds__(D1_NW * MOTY_WAVE) void k_moe_d1_gateup(
   }
   const int rl = wave_sum_row<4>(lane);
   const int ir = i0 + rl < I ? i0 + rl : I - 1;
-  const float sg = GS[(int64_t)e * I + ir], su = US[(int64_t)e * I + ir];
+  float sg = GS[(int64_t)e * I + ir], su = US[(int64_t)e * I + ir];
   __builtin_amdgcn_sched_barrier(0);
   // qrow_i8 of x while the weights fly
   float amax = 0.f;
@@ -880,6 +880,8 @@ __global__ __launch_bounds__(D1_NW * MOTY_WAVE) void k_moe_d1_gateup(
   }
   const int a = wave_sum_multi_i32<4>(ag);
   const int a2 = wave_sum_multi_i32<4>(au);
+  keep_loaded(sg, a);
+  keep_loaded(su, a2);
   const float v = ref_silu_mul((sg * sx) * (float)a, (su * sx) * (float)a2);
   if ((lane & 15) == 0 && i0 + rl < I) h[(int64_t)k * I + i0 + rl] = v;
 }
