@@ -187,7 +187,7 @@ __global__ __launch_bounds__(64 * WGM * WGN * KS) void k_gemm_q8_dma(const int8_
     // XCD takes a contiguous run of tiles, walked column by column in groups
     // of GM tile rows, so the 32 tiles its CUs hold at a time share 4 blocks
     // of activation rows and 8 of weight rows in its L2 (256 x 256 tiles, M =
-    // 2000, 24576 x 4096: 273 -> 265 us).  GM = 0, by rows of tiles: XCD x
+    // 2000, 24576 x 4096: 235 us, 237 by rows).  GM = 0, by rows of tiles: XCD x
     // takes a (gy/2) x (gx/4) block, half the activation rows and a quarter of
     // the weight rows (64 x 128 tiles, M = 512, 10240 x 1024: 13.5 us against
     // 17.6 in runs, 15.0 in plain order), or, where the grid does not divide
@@ -342,7 +342,7 @@ __global__ __launch_bounds__(64 * WGM * WGN * KS) void k_gemm_q8_dma(const int8_
 // tiles with the K blocks split over wave groups (M = 24: 22 us for 2 x
 // 12288 x 4096, 17 us for 4096 x 12288; 64-row tiles took 38 and 22); many
 // tokens by the bytes every CU pulls from L2 (about 20 a clock), which fall
-// with the tile's width (M = 2000: 24576 x 4096 with SiLU 258 us in 256 x
+// with the tile's width (M = 2000: 24576 x 4096 with SiLU 235 us in 256 x
 // 256 tiles against 484 + 82 for two GEMMs in 64 x 64 and silu_mul; 4096 x
 // 12288 120 us in 128 x 128 against 205).
 struct Q8Tile {

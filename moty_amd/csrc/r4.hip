@@ -400,12 +400,13 @@ static int launch_r4_gemv(const float* x, const uint8_t* W, const uint16_t* d16,
 // The weight rows are the MFMA's rows and the tokens its columns: a lane then
 // holds one token (of each token tile), whose xs and xct it reads once per
 // group, and reads the scales dd of its 16 rows as four float4s, shared by
-// all its token tiles.  With the operands the other way round the per-token
-// xs, xct and m8 were 8-12 ds_read_b128 per group and 32 x 32 outputs, and
-// the CU's LDS pipe, 14 reads x 4 waves x 8 clocks = 448, was the whole time
-// (424 clocks measured for 275 of MFMA and vector work).  What is left is
-// that work: 34 clocks of MFMA and 64 vector operations (convert, dd*xs, two
-// FMAs) of 2.6 per 16 registers, which do not overlap on a SIMD.
+// all its token tiles.  With the operands the other way round
+// (k_r4_gemm_tok) the per-token xs, xct and m8 are 8-12 ds_read_b128 per group
+// and 32 x 32 outputs, three times the LDS instructions per output.  What bounds
+// this one on full grids is the vector work of the chains, 64 operations
+// (convert, dd*xs, two FMAs) per 16 registers and MFMA: 24576 x 4096, 256
+// tokens, counters: vector pipes busy 73 % of the kernel's time, MFMA 7 %, LDS
+// bank conflicts 5 %.
 //
 // Tiles of MT x MT outputs (32: v_mfma_i32_32x32x32_i8; 16: 16x16x32, for
 // grids that leave SIMDs idle), RT row tiles x TT token tiles per wave, WR x
