@@ -1,4 +1,4 @@
-"""bench.py -- one-GPU benchmark of libmoty-hw-hip on BASELINE.json's configs.
+"""bench.py -- one-GPU benchmark of libmoty-hw-hip on the library's workloads C1 to C5.
 
 Headline (`value`): C1, the Qwen3-0.6B-shaped decode FFN through the Q8_0
 path (fused gate/up GEMV with the SiLU epilogue, then the down GEMV), as
@@ -91,7 +91,7 @@ class Ctx:
         while the GPU is still busy, and A and B do the same work on cold
         copies, so the difference is the time the K steps add, with the fixed
         cost of an event pair around a graph launch (about 9 us on MI355X,
-        0.45 us per C1 step at the driver's K = 20) cancelled.  The result is
+        0.45 us per C1 step at K = 20) cancelled.  The result is
         the median round's seconds per step (self.last holds the round count,
         the spread and the raw B + timed figure).  Returns (seconds per step,
         steps timed)."""

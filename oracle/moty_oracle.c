@@ -1,6 +1,6 @@
 /* moty_oracle.c -- CPU restatement of moty's quantized-matmul + MoE path.
  *
- * TEST INFRASTRUCTURE ONLY.  This file is the checker for the HIP library in
+ * TEST INFRASTRUCTURE ONLY.  This file is the oracle for the HIP library in
  * moty_amd/: only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline
  * leg may load it.  The product path never calls into it.
  *

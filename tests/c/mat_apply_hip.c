@@ -4,7 +4,7 @@
  *
  * Built by oracle/Makefile (target `harness`) against the reference headers
  * and objects under oracle/_ref (compiled from /root/reference/c) and
- * libmoty_hw_hip.so; run by tests/test_gpu_harness.py on the GPU box.
+ * libmoty_hw_hip.so; run by tests/test_gpu_harness.py.
  *
  * What it binds, each with the reference's CPU function as the fallback:
  *   hip_mat_apply        moty_mat_apply (nn/mat.c:70-83): WF_I8, WF_I4G,

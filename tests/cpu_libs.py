@@ -1,4 +1,4 @@
-"""ctypes loaders for the CPU checkers: the oracle restatement
+"""ctypes loaders for the CPU libraries: the oracle restatement
 (oracle/liboracle.so) and the compiled reference (oracle/_ref/*.so).
 
 Test infrastructure only; the product library is loaded by moty_amd."""
